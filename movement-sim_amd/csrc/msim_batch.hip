@@ -41,35 +41,44 @@ SortedBufs bsorted_bufs(const msim_batch* b, int k) {
 
 constexpr uint32_t kBScanThreads = 1024;
 
+// mv.cur.seg null: scan, move and route choice, each in a launch of its own.
+// Otherwise the move alone (the route choice joins the neighbour pass).
 template <uint32_t U, bool UN, bool W>
-void blaunch_sorted(msim_batch* b, const SortedMove& mv, const BatchBin& bb) {
+void blaunch_sorted(msim_batch* b, const SortedMove& mv, const BatchBin& bb, bool finish) {
+    if (!mv.cur.seg) {
+        bprobe_pre(b);
+        hipLaunchKernelGGL(k_seg_scan<kBScanThreads>, dim3(1), dim3(kBScanThreads), 0, b->stream,
+                           b->seg_cnt[b->cur], b->seg_group[b->cur], b->seg_start, b->n_seg, b->n, b->faults);
+        bprobe_post(b);
+    }
+    constexpr uint32_t waves = kBSortedThreads / 64;
+    const uint32_t extra = finish ? ((b->n_scen + waves - 1) / waves + kXcds - 1) / kXcds * kXcds : 0u;
     bprobe_pre(b);
-    hipLaunchKernelGGL(k_seg_scan<kBScanThreads>, dim3(1), dim3(kBScanThreads), 0, b->stream, b->seg_cnt[b->cur],
-                       b->seg_start, b->n_seg, b->n, b->faults);
+    hipLaunchKernelGGL((k_bmove_sorted<U, kBSortedThreads, UN, W>), dim3(b->n_seg + extra), dim3(kBSortedThreads),
+                       bsorted_lds_bytes(b->max_seg_log), b->stream, mv, bb, bfinish_args(b));
     bprobe_post(b);
-    bprobe_pre(b);
-    hipLaunchKernelGGL((k_bmove_sorted<U, kBSortedThreads, UN, W>), dim3(b->n_seg), dim3(kBSortedThreads),
-                       bsorted_lds_bytes(b->max_seg_log), b->stream, mv, bb);
-    bprobe_post(b);
-    bprobe_pre(b);
-    hipLaunchKernelGGL((k_broute_sorted<UN, W>), dim3(b->n_seg), dim3(kBlock), 0, b->stream, mv, bb);
-    bprobe_post(b);
+    if (!mv.cur.seg) {
+        bprobe_pre(b);
+        hipLaunchKernelGGL((k_broute_sorted<UN, W>), dim3(b->n_seg), dim3(kBlock), 0, b->stream, mv, bb);
+        bprobe_post(b);
+    }
 }
 
 template <uint32_t U>
-void blaunch_sorted_u(msim_batch* b, const SortedMove& mv, const BatchBin& bb, bool write_dir) {
+void blaunch_sorted_u(msim_batch* b, const SortedMove& mv, const BatchBin& bb, bool write_dir, bool finish) {
     if (b->uniform) {
-        if (write_dir) blaunch_sorted<U, true, true>(b, mv, bb);
-        else blaunch_sorted<U, true, false>(b, mv, bb);
+        if (write_dir) blaunch_sorted<U, true, true>(b, mv, bb, finish);
+        else blaunch_sorted<U, true, false>(b, mv, bb, finish);
     } else {
-        if (write_dir) blaunch_sorted<U, false, true>(b, mv, bb);
-        else blaunch_sorted<U, false, false>(b, mv, bb);
+        if (write_dir) blaunch_sorted<U, false, true>(b, mv, bb, finish);
+        else blaunch_sorted<U, false, false>(b, mv, bb, finish);
     }
 }
 
 // Sorted move of every scenario: buf[cur] / binning bcur -> buf[1-cur] /
-// binning 1-bcur in one launch.
-int benqueue_move_sorted(msim_batch* b, bool write_dir) {
+// binning 1-bcur.  fused: the tick's two-launch form, whose route choice runs
+// in the neighbour pass's launch and whose pair totals the next move folds.
+int benqueue_tick_sorted(msim_batch* b, bool write_dir, bool fused) {
     b->launch_no = 0;
     const int nb = 1 - b->cur;
     SortedMove mv{};
@@ -84,7 +93,8 @@ int benqueue_move_sorted(msim_batch* b, bool write_dir) {
     mv.arr_rec = b->arr_rec;
     mv.arr_spd = b->arr_spd;
     mv.seg_start = b->seg_start;
-    mv.seg_next = b->seg_cnt[nb];
+    if (fused) mv.cur = bseg_counts(b, b->cur);
+    mv.next = bseg_counts(b, nb);
     mv.seg_arr = b->seg_arr;
     mv.n = b->n;
     BatchBin bb{};
@@ -97,16 +107,40 @@ int benqueue_move_sorted(msim_batch* b, bool write_dir) {
     bb.faults = b->faults;
     bb.inv_cell = b->inv_cell;
     bb.n_seg = b->n_seg;
-    if (b->bin_unroll == 2) blaunch_sorted_u<2>(b, mv, bb, write_dir);
-    else if (b->bin_unroll == 8) blaunch_sorted_u<8>(b, mv, bb, write_dir);
-    else blaunch_sorted_u<4>(b, mv, bb, write_dir);
+    const bool finish = b->finish_pending;
+    b->finish_pending = false;
+    if (b->bin_unroll == 2) blaunch_sorted_u<2>(b, mv, bb, write_dir, finish);
+    else if (b->bin_unroll == 8) blaunch_sorted_u<8>(b, mv, bb, write_dir, finish);
+    else blaunch_sorted_u<4>(b, mv, bb, write_dir, finish);
     b->cur = nb;
     b->bcur = 1 - b->bcur;
-    return bcheck(b, "batched sorted move dispatch");
+    if (!fused) {
+        int rc = bcheck(b, "batched sorted move dispatch");
+        return rc == MSIM_OK ? benqueue_collide(b) : rc;
+    }
+    const uint32_t per = kBlock * 2u;
+    const RouteMix mix{b->n_seg, std::max(1u, (b->n + per - 1) / per)};
+    const BatchCollide c = bcollide_args(b);
+    if (b->uniform) {
+        hipLaunchKernelGGL((k_broute_collide<true, 2>), dim3(mix.blocks()), dim3(kBlock), 0, b->stream, mv, bb, c,
+                           mix);
+    } else {
+        hipLaunchKernelGGL((k_broute_collide<false, 2>), dim3(mix.blocks()), dim3(kBlock), 0, b->stream, mv, bb, c,
+                           mix);
+    }
+    b->finish_pending = true;
+    return bcheck(b, "batched sorted tick");
+}
+
+// Folds the pair totals a fused tick left to its successor.
+void bflush_finish(msim_batch* b) {
+    if (b->finish_pending) {
+        hipLaunchKernelGGL(k_bfinish, dim3(b->n_scen), dim3(64), 0, b->stream, bfinish_args(b));
+        b->finish_pending = false;
+    }
 }
 
 int benqueue_move(msim_batch* b, bool write_dir) {
-    if (b->sorted) return benqueue_move_sorted(b, write_dir);
     b->launch_no = 0;
     bprobe_pre(b);
     if (b->uniform) {
@@ -150,9 +184,17 @@ int breorder(msim_batch* b) {
     return MSIM_OK;
 }
 
-int btick(msim_batch* b, bool write_dir) {
-    int rc = benqueue_move(b, write_dir);
-    if (rc == MSIM_OK) rc = benqueue_collide(b);
+// One tick.  Inside a run (last = false) the sorted state with the two-slot
+// staged neighbour pass takes its two-launch form; a run's last tick writes
+// the headings and folds its own totals, in one launch per kernel.
+int btick(msim_batch* b, bool last, bool allow_fused = true) {
+    int rc;
+    if (b->sorted) {
+        rc = benqueue_tick_sorted(b, last, allow_fused && !last && b->collide_mode == 0);
+    } else {
+        rc = benqueue_move(b, last);
+        if (rc == MSIM_OK) rc = benqueue_collide(b);
+    }
     b->tick += 2;
     b->since_reorder++;
     if (rc == MSIM_OK && !b->sorted && b->reorder_interval && b->since_reorder >= b->reorder_interval) {
@@ -174,13 +216,14 @@ int benter_sorted(msim_batch* b) {
     const dim3 gs((b->n_seg + kBlock - 1) / kBlock);
     for (int k = 0; k < 2; k++) {
         hipLaunchKernelGGL(k_fill_u32, gs, dim3(kBlock), 0, b->stream, b->seg_cnt[k], 0u, b->n_seg);
+        hipLaunchKernelGGL(k_fill_u32, gs, dim3(kBlock), 0, b->stream, b->seg_group[k], 0u, seg_groups(b->n_seg));
     }
     if (b->uniform) {
         hipLaunchKernelGGL(k_bsorted_next<true>, g, dim3(kBlock), 0, b->stream, bsorted_bufs(b, b->cur), b->blk_scen,
-                           b->scen, b->agent_off, b->n, kShaderSpeed, b->inv_cell, b->seg_cnt[b->cur]);
+                           b->scen, b->agent_off, b->n, kShaderSpeed, b->inv_cell, bseg_counts(b, b->cur));
     } else {
         hipLaunchKernelGGL(k_bsorted_next<false>, g, dim3(kBlock), 0, b->stream, bsorted_bufs(b, b->cur), b->blk_scen,
-                           b->scen, b->agent_off, b->n, kShaderSpeed, b->inv_cell, b->seg_cnt[b->cur]);
+                           b->scen, b->agent_off, b->n, kShaderSpeed, b->inv_cell, bseg_counts(b, b->cur));
     }
     b->sorted = true;
     return bcheck(b, "sorted state set-up");
@@ -206,6 +249,7 @@ int bbuild_graph(msim_batch* b) {
     for (uint32_t t = 0; t < b->seg_ticks && rc == MSIM_OK; t++) {
         rc = btick(b, false);
     }
+    bflush_finish(b);
     b->capturing = false;
     e = hipStreamEndCapture(b->stream, &graph);
     msim_batch::Segment& g = b->gexec[cur0][bcur0];
@@ -483,6 +527,8 @@ extern "C" int msim_batch_create(uint32_t n_scen, const uint32_t* road_off, cons
         BALLOC(b->seg_start, b->n_seg + 1);
         BALLOC(b->seg_cnt[0], b->n_seg);
         BALLOC(b->seg_cnt[1], b->n_seg);
+        BALLOC(b->seg_group[0], seg_groups(b->n_seg));
+        BALLOC(b->seg_group[1], seg_groups(b->n_seg));
         BALLOC(b->seg_arr, b->n_seg);
     }
     BALLOC(b->part, static_cast<size_t>(n_scen) * kScenSlots * kScenSlotStride);
@@ -608,6 +654,7 @@ extern "C" int msim_batch_run_ticks(msim_batch* b, uint32_t n_ticks) {
     while (done < n_ticks && rc == MSIM_OK) {
         const uint32_t left = n_ticks - done;
         if (left - 1 >= b->seg_ticks && (b->reorder_interval == 0 || b->since_reorder == 0)) {
+            bflush_finish(b);  // the segment's first move folds nothing
             msim_batch::Segment& g = b->gexec[b->cur][b->bcur];
             if (!g.exec) {
                 rc = bbuild_graph(b);
@@ -760,7 +807,7 @@ extern "C" int msim_batch_time_ticks(msim_batch* b, uint32_t n_ticks, float* ms_
             b->probe_kernel = k;
             b->probe_ev[0] = ev[0];
             b->probe_ev[1] = ev[1];
-            rc = btick(b, t + 1 == n_ticks);
+            rc = btick(b, t + 1 == n_ticks, false);
             b->probe_kernel = -1;
             if (rc == MSIM_OK) rc = bwait(b);
             float ms = 0.f;

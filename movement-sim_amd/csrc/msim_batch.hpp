@@ -112,20 +112,54 @@ static __global__ __launch_bounds__(T, 8) void k_bbin_fused(const float2* __rest
     }
 }
 
-// Sorted move of every scenario's table (see msim_sorted.hpp): segments are
-// handed out by ticket, each scenario's look-back chain starts at its first
-// segment (prefix = the scenario's first slot).  Dynamic LDS: counters for
-// the largest segment.
+// One wave: fold scenario sidx's slots into its pair totals.
+struct BatchFinish {
+    unsigned long long* part;    // [n_scen][kScenSlots * kScenSlotStride]
+    unsigned long long* totals;  // [n_scen]
+    uint32_t* last;              // [n_scen]
+    uint32_t n_scen;
+};
+
+__device__ __forceinline__ void bfinish_scenario(const BatchFinish& f, uint32_t sidx) {
+    unsigned long long v = 0;
+    const uint32_t lane = __lane_id();
+    if (lane < kScenSlots) {
+        unsigned long long* p = &f.part[(static_cast<size_t>(sidx) * kScenSlots + lane) * kScenSlotStride];
+        v = *p;
+        *p = 0ull;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        v += __shfl_xor(v, o, 64);
+    }
+    if (lane == 0) {
+        const unsigned long long pairs = v / 2;
+        f.totals[sidx] += pairs;
+        f.last[sidx] = static_cast<uint32_t>(pairs);
+    }
+}
+
+// Sorted move of every scenario's table (see msim_sorted.hpp; the segments of
+// all scenarios are numbered in order, so a scenario's first segment starts at
+// its first agent).  Dynamic LDS: counters for the largest segment.  Grid:
+// n_seg workgroups, after a multiple of kXcds for the previous tick's totals
+// when pending.
 template <uint32_t U, uint32_t T, bool UNIFORM, bool WRITE_DIR>
-static __global__ __launch_bounds__(T) void k_bmove_sorted(SortedMove mv, BatchBin b) {
+static __global__ __launch_bounds__(T) void k_bmove_sorted(SortedMove mv, BatchBin b, BatchFinish fin) {
     extern __shared__ uint32_t hist[];
     __shared__ uint32_t lds[T / 64];
     __shared__ uint32_t nh[2 * kNextReach + 1];
-    __shared__ uint32_t sh[1];
-    const uint32_t g = xcd_block(blockIdx.x, gridDim.x);
+    __shared__ uint32_t sh[1 + T / 64];
+    const uint32_t extra = gridDim.x - b.n_seg;
+    if (blockIdx.x < extra) {  // the previous tick's pair totals, beside the move: a wave per scenario
+        const uint32_t sidx = blockIdx.x * (T / 64) + (threadIdx.x >> 6);
+        if (sidx < fin.n_scen) bfinish_scenario(fin, sidx);
+        return;
+    }
+    const uint32_t g = xcd_block(blockIdx.x - extra, b.n_seg);
     const ScenDev sc = b.scen[b.seg_scen[g]];
     const uint32_t gl = g - sc.seg_first;
-    const NextCount nc{nh, mv.seg_next, gl, sc.n_seg, sc.seg_first, sc.seg_log};
+    const NextCount nc{nh, mv.next, gl, sc.n_seg, sc.seg_first, sc.seg_log};
     uint32_t base, total;
     sorted_segment<U, T, UNIFORM, WRITE_DIR>(mv, scen_view(sc, b), nc, gl << sc.seg_log, g, hist, lds, sh,
                                              b.new_start + sc.start_base, &base, &total);
@@ -165,19 +199,19 @@ static __global__ __launch_bounds__(kBlock) void k_broute_sorted(SortedMove mv, 
     __shared__ uint32_t nh[2 * kNextReach + 1];
     const uint32_t g = xcd_block(blockIdx.x, gridDim.x);
     const ScenDev sc = b.scen[b.seg_scen[g]];
-    const NextCount nc{nh, mv.seg_next, g - sc.seg_first, sc.n_seg, sc.seg_first, sc.seg_log};
+    const NextCount nc{nh, mv.next, g - sc.seg_first, sc.n_seg, sc.seg_first, sc.seg_log};
     route_segment_list<UNIFORM, WRITE_DIR>(mv, scen_view(sc, b), nc, g);
 }
 
 // nxt for every slot of every scenario: the bucket of the agent's next
-// position in its own scenario's table; seg_next (cleared before) counts them
+// position in its own scenario's table; next (cleared before) counts them
 // per (global) segment.
 template <bool UNIFORM>
 static __global__ __launch_bounds__(kBlock) void k_bsorted_next(SortedBufs st, const BlockScen* __restrict__ blk,
                                                                 const ScenDev* __restrict__ scen,
                                                                 const uint32_t* __restrict__ agent_off, uint32_t n,
                                                                 float spd_const, float inv_cell,
-                                                                uint32_t* __restrict__ seg_next) {
+                                                                SegCounts next) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     uint32_t gseg = 0;
     if (i < n) {
@@ -196,7 +230,7 @@ static __global__ __launch_bounds__(kBlock) void k_bsorted_next(SortedBufs st, c
         st.nxt[i] = b;
         gseg = sc.seg_first + (b >> sc.seg_log);
     }
-    count_next_segment(seg_next, gseg, i < n);
+    count_next_segment(next, gseg, i < n);
 }
 
 // Per-scenario partial sums of a wave's counts: one atomic per wave when
@@ -267,11 +301,10 @@ __device__ __forceinline__ uint32_t bcount_slot(const BatchCollide& c, uint32_t 
 // Staged neighbour pass: each wave takes 64 P consecutive slots, P per
 // lane; a wave whose slots all lie in one scenario runs wave_count_in_cells
 // on that scenario's table, a wave across a scenario boundary walks per slot
-// (grid: ceil(n / (kBlock P)) workgroups).
+// (workgroup blk of ceil(n / (kBlock P)); stage_all: kStage positions per
+// wave).
 template <int P>
-static __global__ __launch_bounds__(kBlock, P == 1 ? 8 : 6) void k_bcollide_staged(BatchCollide c) {
-    __shared__ float2 stage_all[kBlock / 64 * kStage];
-    const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+__device__ __forceinline__ void bcollide_block(const BatchCollide& c, uint32_t blk, float2* stage_all) {
     const uint32_t wave = blk * (kBlock / 64) + (threadIdx.x >> 6);
     const uint32_t w0 = wave * (64u * P);
     if (w0 >= c.n) {
@@ -319,27 +352,35 @@ static __global__ __launch_bounds__(kBlock, P == 1 ? 8 : 6) void k_bcollide_stag
     }
 }
 
-// One wave per scenario: fold the slots into the scenario's pair totals.
-static __global__ __launch_bounds__(64) void k_bfinish(unsigned long long* __restrict__ part,
-                                                unsigned long long* __restrict__ totals,
-                                                uint32_t* __restrict__ last) {
-    const uint32_t sidx = blockIdx.x;
-    unsigned long long v = 0;
-    if (threadIdx.x < kScenSlots) {
-        unsigned long long* p = &part[(static_cast<size_t>(sidx) * kScenSlots + threadIdx.x) * kScenSlotStride];
-        v = *p;
-        *p = 0ull;
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        v += __shfl_xor(v, o, 64);
-    }
-    if (threadIdx.x == 0) {
-        const unsigned long long pairs = v / 2;
-        totals[sidx] += pairs;
-        last[sidx] = static_cast<uint32_t>(pairs);
+template <int P>
+static __global__ __launch_bounds__(kBlock, P == 1 ? 8 : 6) void k_bcollide_staged(BatchCollide c) {
+    __shared__ float2 stage_all[kBlock / 64 * kStage];
+    bcollide_block<P>(c, xcd_block(blockIdx.x, gridDim.x), stage_all);
+}
+
+// k_route_collide for every scenario.
+template <bool UNIFORM, int P>
+static __global__ __launch_bounds__(kBlock, 6) void k_broute_collide(SortedMove mv, BatchBin b, BatchCollide c,
+                                                                     RouteMix mix) {
+    __shared__ uint32_t nh[2 * kNextReach + 1];
+    __shared__ float2 stage_all[kBlock / 64 * kStage];
+    uint32_t r;
+    if (mix.routes(blockIdx.x, r)) {
+        if (r >= mix.n_route) return;
+        const uint32_t g = xcd_block(r, mix.n_route);
+        const ScenDev sc = b.scen[b.seg_scen[g]];
+        // the counts this tick's move consumed, cleared for the move after next
+        if (threadIdx.x == 0) mv.cur.clear(g);
+        const NextCount nc{nh, mv.next, g - sc.seg_first, sc.n_seg, sc.seg_first, sc.seg_log};
+        route_segment_list<UNIFORM, false>(mv, scen_view(sc, b), nc, g);
+    } else {
+        if (r >= mix.n_collide) return;
+        bcollide_block<P>(c, xcd_block(r, mix.n_collide), stage_all);
     }
 }
+
+// One wave per scenario: fold the slots into the scenario's pair totals.
+static __global__ __launch_bounds__(64) void k_bfinish(BatchFinish f) { bfinish_scenario(f, blockIdx.x); }
 
 }  // namespace msim
 
@@ -404,6 +445,8 @@ struct msim_batch {
     float* arr_spd = nullptr;               // [n] their speeds (per-agent speeds only)
     uint32_t* seg_start = nullptr;          // [n_seg + 1] first slot of each segment (k_seg_scan)
     uint32_t* seg_cnt[2] = {nullptr, nullptr};  // per buffer: agents per segment for the move leaving it
+    uint32_t* seg_group[2] = {nullptr, nullptr};  // and per kGroupSegs segments
+    bool finish_pending = false;  // run_ticks: the last tick's pair totals are folded by the next move
     uint32_t* seg_arr = nullptr;            // [n_seg] arrivals of each segment
     uint32_t bin_unroll = 4;  // window slots per rebinning thread and load round
     uint32_t tick = 1;
@@ -556,7 +599,11 @@ inline GridDev bgrid(const msim_batch* b) {
     return g;
 }
 
-inline int benqueue_collide(msim_batch* b) {
+inline SegCounts bseg_counts(const msim_batch* b, int k) { return SegCounts{b->seg_cnt[k], b->seg_group[k]}; }
+
+inline BatchFinish bfinish_args(const msim_batch* b) { return BatchFinish{b->part, b->totals, b->last, b->n_scen}; }
+
+inline BatchCollide bcollide_args(const msim_batch* b) {
     BatchCollide c{};
     c.blk = b->blk_scen;
     c.scen = b->scen;
@@ -570,6 +617,11 @@ inline int benqueue_collide(msim_batch* b) {
     c.inv_cell = b->inv_cell;
     c.d2_limit = b->d2_limit;
     c.part = b->part;
+    return c;
+}
+
+inline int benqueue_collide(msim_batch* b) {
+    const BatchCollide c = bcollide_args(b);
     bprobe_pre(b);
     if (b->collide_mode == 1) {
         hipLaunchKernelGGL(k_bcollide, dim3(bblocks(b->n)), dim3(kBlock), 0, b->stream, c);
@@ -582,7 +634,7 @@ inline int benqueue_collide(msim_batch* b) {
     }
     bprobe_post(b);
     bprobe_pre(b);
-    hipLaunchKernelGGL(k_bfinish, dim3(b->n_scen), dim3(64), 0, b->stream, b->part, b->totals, b->last);
+    hipLaunchKernelGGL(k_bfinish, dim3(b->n_scen), dim3(64), 0, b->stream, bfinish_args(b));
     bprobe_post(b);
     return bcheck(b, "batched collision dispatch");
 }

@@ -185,12 +185,12 @@ __device__ __forceinline__ bool in_range(float2 pj, float2 pi, float d2_limit) {
 // Workgroup index remapped so that each XCD (workgroups are dealt round-robin
 // over the 8 XCDs) works on one contiguous slice of the index space, keeping
 // neighbouring tiles in the same L2.
+constexpr uint32_t kXcds = 8;
 __device__ __forceinline__ uint32_t xcd_block(uint32_t bid, uint32_t nblocks) {
-    constexpr uint32_t kXcd = 8;
-    const uint32_t xcd = bid % kXcd;
-    const uint32_t local = bid / kXcd;
-    const uint32_t per = nblocks / kXcd;
-    const uint32_t rem = nblocks % kXcd;
+    const uint32_t xcd = bid % kXcds;
+    const uint32_t local = bid / kXcds;
+    const uint32_t per = nblocks / kXcds;
+    const uint32_t rem = nblocks % kXcds;
     return xcd * per + (xcd < rem ? xcd : rem) + local;
 }
 

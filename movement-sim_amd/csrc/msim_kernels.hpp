@@ -655,15 +655,13 @@ __device__ __forceinline__ void wave_count_in_cells(const float2 (&me)[P], const
 }
 
 // Staged neighbour pass (collision dispatch of initialised agents): each
-// wave takes 64 P consecutive slots, P per lane (grid: ceil(n / (kBlock P))
-// workgroups).  At most 64 VGPRs (8 waves per SIMD).
+// wave takes 64 P consecutive slots, P per lane (workgroup blk of
+// ceil(n / (kBlock P))).  lds: kBlock / 64 words, stage_all: kStage positions
+// per wave.
 template <int P>
-static __global__ __launch_bounds__(kBlock, 8) void k_collide_staged(AgentsDev a, GridDev g,
-                                                              const float2* __restrict__ bpos,
-                                                              unsigned long long* __restrict__ part_pairs) {
-    __shared__ uint32_t lds[kBlock / 64];
-    __shared__ float2 stage_all[kBlock / 64 * kStage];
-    const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+__device__ __forceinline__ void collide_block(const AgentsDev& a, const GridDev& g, const float2* __restrict__ bpos,
+                                              unsigned long long* __restrict__ part_pairs, uint32_t blk,
+                                              uint32_t* lds, float2* stage_all) {
     const uint32_t w0 = (blk * (kBlock / 64) + (threadIdx.x >> 6)) * (64u * P);
     const float T = g.d2_limit;
     float2 me[P];
@@ -698,6 +696,17 @@ static __global__ __launch_bounds__(kBlock, 8) void k_collide_staged(AgentsDev a
     if (threadIdx.x == 0) {
         slot_add(part_pairs, blk, kWordPairs, bs);
     }
+}
+
+// The neighbour pass in a launch of its own.  At most 64 VGPRs (8 waves per
+// SIMD).
+template <int P>
+static __global__ __launch_bounds__(kBlock, 8) void k_collide_staged(AgentsDev a, GridDev g,
+                                                              const float2* __restrict__ bpos,
+                                                              unsigned long long* __restrict__ part_pairs) {
+    __shared__ uint32_t lds[kBlock / 64];
+    __shared__ float2 stage_all[kBlock / 64 * kStage];
+    collide_block<P>(a, g, bpos, part_pairs, xcd_block(blockIdx.x, gridDim.x), lds, stage_all);
 }
 
 // Neighbour pass over the binned slots, one slot per lane: count_in_cells.
@@ -812,13 +821,12 @@ static __global__ __launch_bounds__(64) void k_fold_stats(unsigned long long* __
 
 // Folds k_collide's slots into the dispatch's pair total (every pair is found
 // from both ends in the fast path, once in the SLOW path) and, when
-// fold_stats is set, the pending advance statistics; launched with one wave.
+// fold_stats is set, the pending advance statistics; one wave.
 template <bool SLOW>
-static __global__ __launch_bounds__(64) void k_collide_finish(unsigned long long* __restrict__ part_pairs,
-                                                       Counters* __restrict__ ctr, uint32_t* __restrict__ hist,
-                                                       uint32_t hist_mask,
-                                                       unsigned long long* __restrict__ part_stats,
-                                                       uint32_t fold_stats) {
+__device__ __forceinline__ void finish_dispatch(unsigned long long* __restrict__ part_pairs,
+                                                Counters* __restrict__ ctr, uint32_t* __restrict__ hist,
+                                                uint32_t hist_mask, unsigned long long* __restrict__ part_stats,
+                                                uint32_t fold_stats) {
     const unsigned long long tot = take_slots(part_pairs, kWordPairs);
     unsigned long long ins = 0, arr = 0;
     if (fold_stats) {
@@ -833,6 +841,15 @@ static __global__ __launch_bounds__(64) void k_collide_finish(unsigned long long
         ctr->inserts += ins;
         ctr->arrivals += arr;
     }
+}
+
+template <bool SLOW>
+static __global__ __launch_bounds__(64) void k_collide_finish(unsigned long long* __restrict__ part_pairs,
+                                                       Counters* __restrict__ ctr, uint32_t* __restrict__ hist,
+                                                       uint32_t hist_mask,
+                                                       unsigned long long* __restrict__ part_stats,
+                                                       uint32_t fold_stats) {
+    finish_dispatch<SLOW>(part_pairs, ctr, hist, hist_mask, part_stats, fold_stats);
 }
 
 // ---- spatial renumbering -------------------------------------------------

@@ -79,6 +79,8 @@ struct msim_sim {
     float* arr_spd = nullptr;               // [n] their speeds (per-agent speeds only)
     uint32_t* seg_start = nullptr;          // [n_seg + 1] first slot of each segment (k_seg_scan)
     uint32_t* seg_cnt[2] = {nullptr, nullptr};  // per buffer: agents per segment for the move leaving it
+    uint32_t* seg_group[2] = {nullptr, nullptr};  // and per kGroupSegs segments
+    bool finish_pending = false;  // run_ticks: the last tick's statistics are folded by the next move
     uint32_t* seg_arr = nullptr;            // [n_seg] arrivals of each segment
     int ncount_at = 0;  // buffer whose slot order ncount follows (-1: ncount_caller)
     bool route_inline = false;  // arrivals routed inside k_advance instead of k_route
@@ -410,13 +412,13 @@ void flush_stats(msim_sim* s) {
 
 // Move dispatch: advance + bucket table rebuild.  ev (optional) receives an
 // event record after each of the 5 launches of the atomic path.
-int enqueue_move_sorted(msim_sim* s, bool write_dir);
+int enqueue_move_sorted(msim_sim* s, bool write_dir, bool fused);
 
 int enqueue_move(msim_sim* s, int mode, bool write_dir, hipEvent_t* ev = nullptr) {
     flush_stats(s);
     if (mode == kMoveAll) {
         if (s->sorted) {
-            return enqueue_move_sorted(s, write_dir);
+            return enqueue_move_sorted(s, write_dir, false);
         }
         if (s->binning == 3) {
             return fail(s, MSIM_ERR_STATE, "internal: sorted-state move dispatch before the state was sorted");
@@ -543,6 +545,8 @@ SortedBufs sorted_bufs(const msim_sim* s, int k) {
     return SortedBufs{b.pos, s->rec[k], s->nxt[k], b.dir};
 }
 
+SegCounts seg_counts(const msim_sim* s, int k) { return SegCounts{s->seg_cnt[k], s->seg_group[k]}; }
+
 constexpr uint32_t kSortedThreads = 512;
 
 
@@ -563,13 +567,14 @@ int enter_sorted(msim_sim* s) {
     const dim3 gs((s->n_seg + kBlock - 1) / kBlock);
     for (int k = 0; k < 2; k++) {
         hipLaunchKernelGGL(k_fill_u32, gs, dim3(kBlock), 0, s->stream, s->seg_cnt[k], 0u, s->n_seg);
+        hipLaunchKernelGGL(k_fill_u32, gs, dim3(kBlock), 0, s->stream, s->seg_group[k], 0u, seg_groups(s->n_seg));
     }
     if (s->uniform) {
         hipLaunchKernelGGL(k_sorted_next<true>, g, dim3(kBlock), 0, s->stream, sorted_bufs(s, s->cur), s->n,
-                           s->spd_const, gd.inv_cell, gd.lw, gd.wmask, gd.hmask, s->seg_log, s->seg_cnt[s->cur]);
+                           s->spd_const, gd.inv_cell, gd.lw, gd.wmask, gd.hmask, s->seg_log, seg_counts(s, s->cur));
     } else {
         hipLaunchKernelGGL(k_sorted_next<false>, g, dim3(kBlock), 0, s->stream, sorted_bufs(s, s->cur), s->n,
-                           s->spd_const, gd.inv_cell, gd.lw, gd.wmask, gd.hmask, s->seg_log, s->seg_cnt[s->cur]);
+                           s->spd_const, gd.inv_cell, gd.lw, gd.wmask, gd.hmask, s->seg_log, seg_counts(s, s->cur));
     }
     s->ncount_at = s->cur;
     s->sorted = true;
@@ -585,35 +590,59 @@ int ensure_sorted(msim_sim* s) {
 
 constexpr uint32_t kScanThreads = 1024;
 
+// mv.cur.seg null: scan, move and route choice, each in a launch of its own.
+// Otherwise the move alone (the route choice joins the neighbour pass).
+// finish: the previous tick's statistics are folded beside the move.
 template <uint32_t U, bool UN, bool W>
-void launch_sorted(msim_sim* s, const SortedMove& mv, const BinDev& b) {
+void launch_sorted(msim_sim* s, const SortedMove& mv, const BinDev& b, const SortedFinish* finish) {
+    if (!mv.cur.seg) {
+        probe_pre(s);
+        hipLaunchKernelGGL(k_seg_scan<kScanThreads>, dim3(1), dim3(kScanThreads), 0, s->stream, s->seg_cnt[s->cur],
+                           s->seg_group[s->cur], s->seg_start, s->n_seg, s->n, &s->ctr->faults);
+        probe_post(s);
+    }
     probe_pre(s);
-    hipLaunchKernelGGL(k_seg_scan<kScanThreads>, dim3(1), dim3(kScanThreads), 0, s->stream, s->seg_cnt[s->cur],
-                       s->seg_start, s->n_seg, s->n, &s->ctr->faults);
+    hipLaunchKernelGGL((k_move_sorted<U, kSortedThreads, UN, W>), dim3(s->n_seg + (finish ? kXcds : 0u)),
+                       dim3(kSortedThreads), sorted_lds_bytes(s->seg_log), s->stream, mv, b,
+                       finish ? *finish : SortedFinish{});
     probe_post(s);
-    probe_pre(s);
-    hipLaunchKernelGGL((k_move_sorted<U, kSortedThreads, UN, W>), dim3(s->n_seg), dim3(kSortedThreads),
-                       sorted_lds_bytes(s->seg_log), s->stream, mv, b);
-    probe_post(s);
-    probe_pre(s);
-    hipLaunchKernelGGL((k_route_sorted<UN, W>), dim3(s->n_seg), dim3(kBlock), 0, s->stream, mv, b);
-    probe_post(s);
+    if (!mv.cur.seg) {
+        probe_pre(s);
+        hipLaunchKernelGGL((k_route_sorted<UN, W>), dim3(s->n_seg), dim3(kBlock), 0, s->stream, mv, b);
+        probe_post(s);
+    }
 }
 
 template <uint32_t U>
-void launch_sorted_u(msim_sim* s, const SortedMove& mv, const BinDev& b, bool write_dir) {
+void launch_sorted_u(msim_sim* s, const SortedMove& mv, const BinDev& b, bool write_dir,
+                     const SortedFinish* finish) {
     if (s->uniform) {
-        if (write_dir) launch_sorted<U, true, true>(s, mv, b);
-        else launch_sorted<U, true, false>(s, mv, b);
+        if (write_dir) launch_sorted<U, true, true>(s, mv, b, finish);
+        else launch_sorted<U, true, false>(s, mv, b, finish);
     } else {
-        if (write_dir) launch_sorted<U, false, true>(s, mv, b);
-        else launch_sorted<U, false, false>(s, mv, b);
+        if (write_dir) launch_sorted<U, false, true>(s, mv, b, finish);
+        else launch_sorted<U, false, false>(s, mv, b, finish);
+    }
+}
+
+SortedFinish finish_args(const msim_sim* s) {
+    return SortedFinish{s->part_pairs, s->ctr, s->hist, s->hist_cap - 1, stats_buf(s)};
+}
+
+// Folds the statistics a fused tick left to its successor.
+void flush_finish(msim_sim* s) {
+    if (s->finish_pending) {
+        hipLaunchKernelGGL(k_collide_finish<false>, dim3(1), dim3(64), 0, s->stream, s->part_pairs, s->ctr,
+                           s->hist, s->hist_cap - 1, stats_buf(s), 1u);
+        s->finish_pending = false;
     }
 }
 
 // Sorted move dispatch: buf[cur] / binning bcur -> buf[1-cur] / binning
-// 1-bcur in one launch.
-int enqueue_move_sorted(msim_sim* s, bool write_dir) {
+// 1-bcur.  fused (run_ticks): the whole tick in two launches, the move and
+// then the route choice together with the neighbour pass; its statistics are
+// left to the next move (or flush_finish).
+int enqueue_move_sorted(msim_sim* s, bool write_dir, bool fused) {
     const int nb = 1 - s->cur;
     const dim3 g(agent_blocks(s->n));
     if (s->ncount_at == nb) {  // the move overwrites the slot order the last counts follow
@@ -628,13 +657,17 @@ int enqueue_move_sorted(msim_sim* s, bool write_dir) {
     mv.roads = s->roads;
     mv.conns = s->conns;
     mv.spd_const = s->spd_const;
+    const SortedFinish finish = finish_args(s);  // the previous tick's half of the statistics
+    const bool fin = s->finish_pending;
+    s->finish_pending = false;
     s->stats_par ^= 1;  // the next tick's collision dispatch folds this half
     mv.part_stats = stats_buf(s);
     mv.faults = &s->ctr->faults;
     mv.arr_rec = s->arr_rec;
     mv.arr_spd = s->arr_spd;
     mv.seg_start = s->seg_start;
-    mv.seg_next = s->seg_cnt[nb];
+    if (fused) mv.cur = seg_counts(s, s->cur);
+    mv.next = seg_counts(s, nb);
     mv.seg_arr = s->seg_arr;
     mv.n = s->n;
     BinDev b{};
@@ -653,13 +686,44 @@ int enqueue_move_sorted(msim_sim* s, bool write_dir) {
     b.margin = s->margin;
     b.n = s->n;
     s->launch_no = 0;
-    if (s->bin_unroll == 2) launch_sorted_u<2>(s, mv, b, write_dir);
-    else if (s->bin_unroll == 8) launch_sorted_u<8>(s, mv, b, write_dir);
-    else launch_sorted_u<4>(s, mv, b, write_dir);
+    const SortedFinish* pf = fin ? &finish : nullptr;
+    if (s->bin_unroll == 2) launch_sorted_u<2>(s, mv, b, write_dir, pf);
+    else if (s->bin_unroll == 8) launch_sorted_u<8>(s, mv, b, write_dir, pf);
+    else launch_sorted_u<4>(s, mv, b, write_dir, pf);
     s->cur = nb;
     s->bcur = 1 - s->bcur;
-    s->stats_pending = true;  // folded by the next collision dispatch's finish pass
-    return check_launch(s, "sorted move dispatch");
+    if (!fused) {
+        s->stats_pending = true;  // folded by the next collision dispatch's finish pass
+        return check_launch(s, "sorted move dispatch");
+    }
+    GridDev gd = s->grid_cur();
+    gd.bid = nullptr;  // the state itself is in slot order
+    const uint32_t per = kBlock * 2u;
+    const RouteMix mix{s->n_seg, std::max(1u, (s->n + per - 1) / per)};
+    const AgentsDev a = s->agents(s->cur);
+    const float2* bpos = s->buf[s->cur].pos;
+    if (s->uniform) {
+        hipLaunchKernelGGL((k_route_collide<true, 2>), dim3(mix.blocks()), dim3(kBlock), 0, s->stream, mv, b, a, gd,
+                           bpos, s->part_pairs, mix);
+    } else {
+        hipLaunchKernelGGL((k_route_collide<false, 2>), dim3(mix.blocks()), dim3(kBlock), 0, s->stream, mv, b, a, gd,
+                           bpos, s->part_pairs, mix);
+    }
+    s->ncount_at = s->cur;
+    s->finish_pending = true;
+    return check_launch(s, "sorted tick");
+}
+
+// One tick inside a run (not its last): the sorted state with the two-slot
+// staged neighbour pass takes the two-launch form.
+int enqueue_run_tick(msim_sim* s) {
+    if (s->sorted && s->collide_mode == 0) {
+        flush_stats(s);
+        return enqueue_move_sorted(s, false, true);
+    }
+    int rc = enqueue_move(s, kMoveAll, false);
+    if (rc == MSIM_OK) rc = enqueue_collide(s, false);
+    return rc;
 }
 
 // Makes the classic per-slot arrays of buf[cur] (target, speed, caller index,
@@ -721,10 +785,10 @@ int build_graph(msim_sim* s) {
     int rc = MSIM_OK;
     s->capturing = true;  // run segments are always followed by the run's last tick
     for (uint32_t t = 0; t < s->seg_ticks && rc == MSIM_OK; t++) {
-        rc = enqueue_move(s, kMoveAll, false);
-        if (rc == MSIM_OK) rc = enqueue_collide(s, false);
+        rc = enqueue_run_tick(s);
         if (rc == MSIM_OK) rc = after_move(s);
     }
+    flush_finish(s);
     s->capturing = false;
     hipError_t e = hipStreamEndCapture(s->stream, &graph);
     msim_sim::Segment& g = s->gexec[cur0][bcur0][qpar0];
@@ -1000,6 +1064,8 @@ extern "C" int msim_create(const msim_road* roads, uint32_t n_roads, const uint3
         ALLOC(s->seg_start, s->n_seg + 1);
         ALLOC(s->seg_cnt[0], s->n_seg);
         ALLOC(s->seg_cnt[1], s->n_seg);
+        ALLOC(s->seg_group[0], seg_groups(s->n_seg));
+        ALLOC(s->seg_group[1], seg_groups(s->n_seg));
         ALLOC(s->seg_arr, s->n_seg);
     }
     ALLOC(s->seg_total, s->n_seg);
@@ -1099,6 +1165,7 @@ extern "C" int msim_run_ticks(msim_sim* s, uint32_t n_ticks) {
         const uint32_t left = n_ticks - done;
         if (left - 1 >= s->seg_ticks && (s->reorder_interval == 0 || s->since_reorder == 0) &&
             (!s->sorted || s->ncount_at == s->cur)) {
+            flush_finish(s);  // the segment's first move folds nothing
             msim_sim::Segment& g = s->gexec[s->cur][s->bcur][s->qpar];
             if (!g.exec) {
                 rc = build_graph(s);
@@ -1119,8 +1186,12 @@ extern "C" int msim_run_ticks(msim_sim* s, uint32_t n_ticks) {
             done += s->seg_ticks;
         } else {
             // Direction is output-only state: write it on the final tick.
-            rc = enqueue_move(s, kMoveAll, left == 1);
-            if (rc == MSIM_OK) rc = enqueue_collide(s, false);
+            if (left == 1) {
+                rc = enqueue_move(s, kMoveAll, true);
+                if (rc == MSIM_OK) rc = enqueue_collide(s, false);
+            } else {
+                rc = enqueue_run_tick(s);
+            }
             s->pc.tick += 2;
             s->any_collide = true;
             done++;

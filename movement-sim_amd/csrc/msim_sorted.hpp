@@ -16,10 +16,12 @@
 //   * count pass: every window slot carries `nxt`, the bucket of the agent's
 //     next position, computed when the agent was last placed; counting reads
 //     these 4 bytes per slot and no state;
-//   * the segment's first slot is known before the launch: the previous
-//     move and route choice counted, per segment, the agents whose next
-//     bucket lies in it, and k_seg_scan turned those counts into first slots,
-//     so no segment waits for another;
+//   * the segment's first slot follows from counts made before the launch:
+//     the previous move and route choice counted, per segment and per group
+//     of kGroupSegs segments, the agents whose next bucket lies in it, so no
+//     segment waits for another.  Inside run_ticks every workgroup sums the
+//     counts before its segment itself; a single dispatch runs k_seg_scan
+//     first;
 //   * rank: the window slots whose `nxt` lies in the segment take their new
 //     slots from LDS counters; an LDS map records, per new slot, the old
 //     slot's window index and the counted bucket;
@@ -96,13 +98,35 @@ __device__ __forceinline__ uint4 hot_record(float2 tgt, float spd, uint32_t call
 // and the PRNG state.
 __device__ __forceinline__ uint4 cold_word(uint32_t road, uint2 c) { return make_uint4(road, c.x, c.y, 0u); }
 
+// Agents whose next bucket lies in each segment, and the sums of those
+// counts over groups of kGroupSegs consecutive segments: a segment's first
+// slot is then the sum of the groups before its own and of at most
+// kGroupSegs - 1 segments, which the workgroup of the segment adds up while
+// its window is in flight (12,000 segments: 750 + 15 words).  Larger groups
+// would put more of the workgroups' atomics on one word.
+constexpr uint32_t kGroupLog = 4, kGroupSegs = 1u << kGroupLog;
+__host__ __device__ constexpr uint32_t seg_groups(uint32_t n_seg) { return (n_seg + kGroupSegs - 1u) >> kGroupLog; }
+struct SegCounts {
+    uint32_t* seg;    // [n_seg]
+    uint32_t* group;  // [seg_groups(n_seg)]
+    __device__ void add(uint32_t g, uint32_t v) const {
+        atomicAdd(&seg[g], v);
+        atomicAdd(&group[g >> kGroupLog], v);
+    }
+    __device__ void clear(uint32_t g) const {
+        seg[g] = 0u;
+        if ((g & (kGroupSegs - 1u)) == 0u) group[g >> kGroupLog] = 0u;
+    }
+};
+
 struct SortedMove {
     SortedBufs src, dst;
     uint4* arr_rec;      // [n] arrivals {new slot, caller index, x bits, y bits}, segment g's at
                          // [seg_start[g], + seg_arr[g])
     float* arr_spd;      // [n] their speeds; nullptr with spd_const
-    const uint32_t* seg_start;  // [n_seg + 1] first slot of each segment (k_seg_scan)
-    uint32_t* seg_next;         // [n_seg] agents whose next bucket lies in each segment, for the next move
+    uint32_t* seg_start;        // [n_seg + 1] first slot of each segment (k_seg_scan, or written by the move)
+    SegCounts cur;              // counts this move consumes (cur.seg nullptr: k_seg_scan did)
+    SegCounts next;             // counts for the next move
     uint32_t* seg_arr;          // [n_seg] arrivals of each segment
     uint4* cold;                // [2 n] caller order: cold_word, PRNG state
     uint32_t n;
@@ -119,11 +143,11 @@ enum : unsigned int { kFaultNext = 4u };  // an agent's position left the bucket
 // g_local of a table of n_local segments (global index seg_first + g_local);
 // its agents' next buckets lie within the window margin of that segment, so
 // nh[d + kNextReach] counts those d segments away (cyclically) and farther
-// ones go straight to seg_next.  next_flush adds nh to seg_next.
+// ones go straight to the global counts.  next_flush adds nh to them.
 constexpr int kNextReach = 2;
 struct NextCount {
     uint32_t* nh;  // LDS [2 kNextReach + 1]
-    uint32_t* seg_next;
+    SegCounts next;
     uint32_t g_local, n_local, seg_first, seg_log;
 };
 
@@ -148,17 +172,17 @@ __device__ __forceinline__ void next_add(const NextCount& nc, uint32_t bucket, b
         __hip_atomic_fetch_add(&nc.nh[d + kNextReach], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     if (active && !own && !near) {
-        atomicAdd(&nc.seg_next[nc.seg_first + ls], 1u);
+        nc.next.add(nc.seg_first + ls, 1u);
     }
 }
 
-// Workgroup-level, after a barrier: nh into seg_next.
+// Workgroup-level, after a barrier: nh into the global counts.
 __device__ __forceinline__ void next_flush(const NextCount& nc) {
     const int k = static_cast<int>(threadIdx.x);
     if (k < 2 * kNextReach + 1 && nc.nh[k]) {
         const int nl = static_cast<int>(nc.n_local);
         const int l = ((static_cast<int>(nc.g_local) + k - kNextReach) % nl + nl) % nl;
-        atomicAdd(&nc.seg_next[nc.seg_first + static_cast<uint32_t>(l)], nc.nh[k]);
+        nc.next.add(nc.seg_first + static_cast<uint32_t>(l), nc.nh[k]);
     }
 }
 
@@ -411,7 +435,17 @@ __device__ __forceinline__ void sorted_segment(const SortedMove& mv, const Table
                                                uint32_t* total_out) {
     const uint32_t tid = threadIdx.x;
     const uint32_t S = 1u << t.seg_log;
-    const uint32_t st0 = mv.seg_start[g], st1 = mv.seg_start[g + 1];  // loaded while the window is counted
+    // the counts before the segment, or its scanned slots: loaded while the window is counted
+    uint32_t before = 0, st0 = 0, st1 = 0;
+    if (mv.cur.seg) {
+        const uint32_t gg = g >> kGroupLog, in = (gg << kGroupLog) + tid;
+        for (uint32_t k = tid; k < gg; k += T) before += mv.cur.group[k];
+        if (in < g) before += mv.cur.seg[in];  // in < g leaves tid < kGroupSegs
+        st1 = mv.cur.seg[g];
+    } else {
+        st0 = mv.seg_start[g];
+        st1 = mv.seg_start[g + 1];
+    }
     for (uint32_t j = tid; j < S; j += T) {
         hist[j] = 0u;
     }
@@ -455,7 +489,15 @@ __device__ __forceinline__ void sorted_segment(const SortedMove& mv, const Table
         sorted_count<2 * U, T>(mv.src.nxt, s0, S, a0, a1, hist);
         sorted_count<2 * U, T>(mv.src.nxt, s0, S, c0, c1, hist);
     }
+    if (mv.cur.seg) {
+        before = wave_sum(before);
+        if (__lane_id() == 0) sh[1 + (tid >> 6)] = before;
+    }
     __syncthreads();
+    if (mv.cur.seg) {
+        for (uint32_t w = 0; w < T / 64; w++) st0 += sh[1 + w];
+        st1 += st0;
+    }
     const uint32_t per = S / T;
     uint32_t run = 0;
     for (uint32_t q = 0; q < per; q++) {
@@ -471,6 +513,7 @@ __device__ __forceinline__ void sorted_segment(const SortedMove& mv, const Table
     if (tid == 0 && total != limit) {
         atomicOr(mv.faults, kFaultBinCount);
     }
+    if (tid == 0 && mv.cur.seg) mv.seg_start[g] = base;
     for (uint32_t q = 0; q < per; q++) {  // counts -> absolute bucket offsets
         const uint32_t v = hist[tid * per + q];
         hist[tid * per + q] = base + excl;
@@ -537,33 +580,60 @@ __device__ __forceinline__ void sorted_segment(const SortedMove& mv, const Table
 }
 
 
-// Sorted move of one table (grid: n_seg workgroups; dynamic LDS:
+// Statistics of a finished collision dispatch (k_collide_finish's work),
+// done by one extra workgroup of the next tick's move: a launch of its own
+// for one wave took 4.5 us of a 45 us tick (1M agents).
+struct SortedFinish {
+    unsigned long long* part_pairs;
+    Counters* ctr;
+    uint32_t* hist;
+    uint32_t hist_mask;
+    unsigned long long* part_stats;  // the finished tick's half
+};
+
+__device__ __forceinline__ void sorted_finish(const SortedFinish& f) {
+    if (threadIdx.x < 64u) {
+        finish_dispatch<false>(f.part_pairs, f.ctr, f.hist, f.hist_mask, f.part_stats, 1u);
+    }
+}
+
+// Sorted move of one table (grid: n_seg workgroups, after kXcds more when the
+// previous tick's statistics are pending; dynamic LDS:
 // sorted_lds_bytes(seg_log)).
 template <uint32_t U, uint32_t T, bool UNIFORM, bool WRITE_DIR>
-static __global__ __launch_bounds__(T) void k_move_sorted(SortedMove mv, BinDev b) {
+static __global__ __launch_bounds__(T) void k_move_sorted(SortedMove mv, BinDev b, SortedFinish fin) {
     extern __shared__ uint32_t hist[];
     __shared__ uint32_t lds[T / 64];
     __shared__ uint32_t nh[2 * kNextReach + 1];
-    __shared__ uint32_t sh[1];
-    const uint32_t seg = xcd_block(blockIdx.x, gridDim.x);
-    const NextCount nc{nh, mv.seg_next, seg, b.n_seg, 0u, b.seg_log};
+    __shared__ uint32_t sh[1 + T / 64];
+    const uint32_t extra = gridDim.x - b.n_seg;
+    if (blockIdx.x < extra) {  // the previous tick's statistics, beside the move (see sorted_finish)
+        if (blockIdx.x == 0) sorted_finish(fin);
+        return;
+    }
+    const uint32_t seg = xcd_block(blockIdx.x - extra, b.n_seg);
+    const NextCount nc{nh, mv.next, seg, b.n_seg, 0u, b.seg_log};
     uint32_t base, total;
     sorted_segment<U, T, UNIFORM, WRITE_DIR>(mv, table_view(b), nc, seg << b.seg_log, seg, hist, lds, sh,
                                              b.new_start, &base, &total);
     if (seg == b.n_seg - 1 && threadIdx.x == 0) {
         b.new_start[b.m] = base + total;
+        if (base + total != b.n) {
+            atomicOr(mv.faults, kFaultBinCount);
+        }
     }
 }
 
 // First slot of every segment from the per-segment agent counts (the
 // segments of all tables in order): seg_start[g] = cnt[0] + ... + cnt[g - 1],
-// seg_start[n_seg] = the total, which must be n.  cnt is cleared for its next
-// use.  One workgroup: wave w takes the contiguous chunk [w C, (w + 1) C) in
+// seg_start[n_seg] = the total, which must be n.  cnt and its group sums are
+// cleared for their next use.  One workgroup: wave w takes the contiguous chunk [w C, (w + 1) C) in
 // pieces of 64 K entries, each loaded at once (coalesced, K loads in flight
 // per lane) and kept in registers for both the chunk sum and the offsets.
 template <uint32_t T>
-static __global__ __launch_bounds__(T) void k_seg_scan(uint32_t* __restrict__ cnt, uint32_t* __restrict__ seg_start,
-                                                       uint32_t n_seg, uint32_t n, unsigned int* faults) {
+static __global__ __launch_bounds__(T) void k_seg_scan(uint32_t* __restrict__ cnt, uint32_t* __restrict__ group,
+                                                       uint32_t* __restrict__ seg_start, uint32_t n_seg, uint32_t n,
+                                                       unsigned int* faults) {
     constexpr uint32_t W = T / 64, K = 16;
     __shared__ uint32_t wsum[W];
     const uint32_t lane = __lane_id(), w = threadIdx.x >> 6;
@@ -609,6 +679,9 @@ static __global__ __launch_bounds__(T) void k_seg_scan(uint32_t* __restrict__ cn
             }
             run += static_cast<uint32_t>(__shfl(static_cast<int>(inc), 63, 64));
         }
+    }
+    for (uint32_t k = threadIdx.x; k < seg_groups(n_seg); k += T) {
+        group[k] = 0u;
     }
     if (threadIdx.x == 0) {
         seg_start[n_seg] = total;
@@ -664,33 +737,79 @@ template <bool UNIFORM, bool WRITE_DIR>
 static __global__ __launch_bounds__(kBlock) void k_route_sorted(SortedMove mv, BinDev b) {
     __shared__ uint32_t nh[2 * kNextReach + 1];
     const uint32_t g = xcd_block(blockIdx.x, gridDim.x);
-    route_segment_list<UNIFORM, WRITE_DIR>(mv, table_view(b), NextCount{nh, mv.seg_next, g, b.n_seg, 0u, b.seg_log},
-                                           g);
+    route_segment_list<UNIFORM, WRITE_DIR>(mv, table_view(b), NextCount{nh, mv.next, g, b.n_seg, 0u, b.seg_log}, g);
+}
+
+// Route choice and neighbour pass in one launch (run_ticks only).  Neither
+// reads what the other writes: the neighbour pass needs the positions and
+// bucket offsets the move left, the route choice rewrites targets, next
+// buckets and route state.  Groups of kXcds workgroups (one per XCD) are
+// dealt to the two in turn while both have some left: a route workgroup
+// waits on random cache lines most of its time, and spreading the routes
+// through the whole launch made it as long as their chain of waits.
+// Measured (kernel trace, us; apart -> together in turn): 8M agents
+// 55 + 77 -> 131 (129 with all routes first, 142 spread evenly), 64
+// scenarios of 5.8M agents 33 + 77 -> 99 (103, 93 to 104), 1M agents
+// 4.9 + 13.0 -> 16.4 (16.9, 17.3).
+struct RouteMix {
+    uint32_t n_route, n_collide;
+    __host__ __device__ static uint32_t groups(uint32_t n) { return (n + kXcds - 1u) / kXcds; }
+    __host__ uint32_t blocks() const { return kXcds * (groups(n_route) + groups(n_collide)); }
+    // Workgroup bid's part: route workgroup r, or neighbour workgroup r (r may
+    // lie past the last one).
+    __device__ bool routes(uint32_t bid, uint32_t& r) const {
+        const uint32_t grp = bid / kXcds, rg = groups(n_route), cg = groups(n_collide);
+        const uint32_t both = 2u * min(rg, cg);
+        r = (grp < both ? grp / 2u : grp - both / 2u) * kXcds + bid % kXcds;
+        return grp < both ? (grp & 1u) == 0u : rg > cg;
+    }
+};
+
+template <bool UNIFORM, int P>
+static __global__ __launch_bounds__(kBlock, 8) void k_route_collide(SortedMove mv, BinDev b, AgentsDev a, GridDev g,
+                                                                    const float2* __restrict__ bpos,
+                                                                    unsigned long long* __restrict__ part_pairs,
+                                                                    RouteMix mix) {
+    __shared__ uint32_t lds[kBlock / 64];
+    __shared__ uint32_t nh[2 * kNextReach + 1];
+    __shared__ float2 stage_all[kBlock / 64 * kStage];
+    uint32_t r;
+    if (mix.routes(blockIdx.x, r)) {
+        if (r >= mix.n_route) return;
+        const uint32_t seg = xcd_block(r, mix.n_route);
+        // the counts this tick's move consumed, cleared for the move after next
+        if (threadIdx.x == 0) mv.cur.clear(seg);
+        route_segment_list<UNIFORM, false>(mv, table_view(b), NextCount{nh, mv.next, seg, b.n_seg, 0u, b.seg_log},
+                                           seg);
+    } else {
+        if (r >= mix.n_collide) return;
+        collide_block<P>(a, g, bpos, part_pairs, xcd_block(r, mix.n_collide), lds, stage_all);
+    }
 }
 
 // Wave-level: one count per distinct segment among the active lanes' gseg
 // (the lanes of a wave hold consecutive slots in bucket order, so there are
 // few).
-__device__ __forceinline__ void count_next_segment(uint32_t* seg_next, uint32_t gseg, bool active) {
+__device__ __forceinline__ void count_next_segment(const SegCounts& next, uint32_t gseg, bool active) {
     unsigned long long todo = __ballot(active);
     while (todo) {
         const int leader = __ffsll(static_cast<long long>(todo)) - 1;
         const uint32_t k = static_cast<uint32_t>(__shfl(static_cast<int>(gseg), leader, 64));
         const unsigned long long peers = __ballot(active && gseg == k) & todo;
         if (static_cast<int>(__lane_id()) == leader) {
-            atomicAdd(&seg_next[k], static_cast<uint32_t>(__popcll(peers)));
+            next.add(k, static_cast<uint32_t>(__popcll(peers)));
         }
         todo &= ~peers;
     }
 }
 
 // nxt for every slot of one table: the bucket of the agent's next position;
-// seg_next (cleared before) counts them per segment.
+// next (cleared before) counts them per segment.
 template <bool UNIFORM>
 static __global__ __launch_bounds__(kBlock) void k_sorted_next(SortedBufs st, uint32_t n, float spd_const,
                                                                float inv_cell, uint32_t lw, uint32_t wmask,
                                                                uint32_t hmask, uint32_t seg_log,
-                                                               uint32_t* __restrict__ seg_next) {
+                                                               SegCounts next) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     uint32_t b = 0;
     if (i < n) {
@@ -700,7 +819,7 @@ static __global__ __launch_bounds__(kBlock) void k_sorted_next(SortedBufs st, ui
         b = bucket_of(cell_coord(np.x, inv_cell), cell_coord(np.y, inv_cell), lw, wmask, hmask);
         st.nxt[i] = b;
     }
-    count_next_segment(seg_next, b >> seg_log, i < n);
+    count_next_segment(next, b >> seg_log, i < n);
 }
 
 // p[0, n) = v (in graphs too, where memset nodes are avoided).

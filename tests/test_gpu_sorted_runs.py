@@ -1,0 +1,49 @@
+"""Runs on the sorted state: the two-launch tick (move; route choice with the
+neighbour pass) at the sizes where its workgroup dealing and its folded
+statistics can go wrong, against the CPU oracle bit for bit."""
+import numpy as np
+import pytest
+
+import msim
+import orc
+from msim import scenarios as S
+from test_gpu_parity import assert_same, pair
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("agents", [1, 64, 511, 513, 5000])
+@pytest.mark.parametrize("opts", [dict(table_log2=12), dict(table_log2=12, segment_log2=9),
+                                  dict(table_log2=19, segment_log2=9), dict(segment_log2=10, graph_ticks=7)])
+def test_run_matches_oracle(agents, opts):
+    """More route than neighbour workgroups and the reverse, counts that are
+    no multiple of eight, one segment and many, direct and captured ticks."""
+    sc = S.config(1, scale=0.5)
+    sc.entities, sc.speed = sc.entities[:agents], sc.speed[:agents]
+    g, o = pair(sc, binning=3, **opts)
+    for ticks in (1, 45, 2, 33):
+        g.run_ticks(ticks)
+        o.run_ticks(ticks)
+        assert_same(g.state(), o.st, f"{agents} agents, {opts}")
+    total, hist = g.pairs()
+    assert total == o.pairs_total
+    assert hist.tolist() == o.pair_hist
+    g.sync()
+
+
+@pytest.mark.parametrize("n_scen", [1, 8, 63, 65])
+def test_batch_run_folds_every_scenarios_pairs(n_scen):
+    """Pair totals and the last tick's pairs of every scenario, the earlier
+    ticks' totals folded by the moves that follow them."""
+    scs = S.batch_config(n_scen, scale=0.004, seed=11)
+    b = msim.Batch(scs, binning=3, graph_ticks=6)
+    b.run_ticks(31)
+    tot, last = b.pairs()
+    for s, sc in enumerate(scs):
+        o = orc.OracleSim(sc.roads, sc.conns, sc.entities, sc.pc, speed=sc.speed)
+        o.run_ticks(31)
+        assert int(tot[s]) == o.pairs_total and int(last[s]) == o.pair_hist[-1], f"scenario {s}"
+        st = b.state(s)
+        np.testing.assert_array_equal(st["pos"].view(np.uint32), o.st.pos.view(np.uint32), err_msg=f"scenario {s}")
+        np.testing.assert_array_equal(st["rng"], o.st.rng, err_msg=f"scenario {s}")
+    b.sync()
