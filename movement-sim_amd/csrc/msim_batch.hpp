@@ -156,7 +156,7 @@ static __global__ __launch_bounds__(T) void k_bmove_sorted(SortedMove mv, BatchB
         if (sidx < fin.n_scen) bfinish_scenario(fin, sidx);
         return;
     }
-    const uint32_t g = xcd_block(blockIdx.x - extra, b.n_seg);
+    const uint32_t g = seg_order(blockIdx.x - extra, b.n_seg);
     const ScenDev sc = b.scen[b.seg_scen[g]];
     const uint32_t gl = g - sc.seg_first;
     const NextCount nc{nh, mv.next, gl, sc.n_seg, sc.seg_first, sc.seg_log};
@@ -197,7 +197,7 @@ struct BatchCollide {
 template <bool UNIFORM, bool WRITE_DIR>
 static __global__ __launch_bounds__(kBlock) void k_broute_sorted(SortedMove mv, BatchBin b) {
     __shared__ uint32_t nh[2 * kNextReach + 1];
-    const uint32_t g = xcd_block(blockIdx.x, gridDim.x);
+    const uint32_t g = seg_order(blockIdx.x, gridDim.x);
     const ScenDev sc = b.scen[b.seg_scen[g]];
     const NextCount nc{nh, mv.next, g - sc.seg_first, sc.n_seg, sc.seg_first, sc.seg_log};
     route_segment_list<UNIFORM, WRITE_DIR>(mv, scen_view(sc, b), nc, g);
@@ -355,7 +355,7 @@ __device__ __forceinline__ void bcollide_block(const BatchCollide& c, uint32_t b
 template <int P>
 static __global__ __launch_bounds__(kBlock, P == 1 ? 8 : 6) void k_bcollide_staged(BatchCollide c) {
     __shared__ float2 stage_all[kBlock / 64 * kStage];
-    bcollide_block<P>(c, xcd_block(blockIdx.x, gridDim.x), stage_all);
+    bcollide_block<P>(c, collide_order(blockIdx.x, gridDim.x), stage_all);
 }
 
 // k_route_collide for every scenario.
@@ -367,7 +367,7 @@ static __global__ __launch_bounds__(kBlock, 6) void k_broute_collide(SortedMove 
     uint32_t r;
     if (mix.routes(blockIdx.x, r)) {
         if (r >= mix.n_route) return;
-        const uint32_t g = xcd_block(r, mix.n_route);
+        const uint32_t g = seg_order(r, mix.n_route);
         const ScenDev sc = b.scen[b.seg_scen[g]];
         // the counts this tick's move consumed, cleared for the move after next
         if (threadIdx.x == 0) mv.cur.clear(g);
@@ -375,7 +375,7 @@ static __global__ __launch_bounds__(kBlock, 6) void k_broute_collide(SortedMove 
         route_segment_list<UNIFORM, false>(mv, scen_view(sc, b), nc, g);
     } else {
         if (r >= mix.n_collide) return;
-        bcollide_block<P>(c, xcd_block(r, mix.n_collide), stage_all);
+        bcollide_block<P>(c, collide_order(r, mix.n_collide), stage_all);
     }
 }
 

@@ -706,7 +706,7 @@ static __global__ __launch_bounds__(kBlock, 8) void k_collide_staged(AgentsDev a
                                                               unsigned long long* __restrict__ part_pairs) {
     __shared__ uint32_t lds[kBlock / 64];
     __shared__ float2 stage_all[kBlock / 64 * kStage];
-    collide_block<P>(a, g, bpos, part_pairs, xcd_block(blockIdx.x, gridDim.x), lds, stage_all);
+    collide_block<P>(a, g, bpos, part_pairs, collide_order(blockIdx.x, gridDim.x), lds, stage_all);
 }
 
 // Neighbour pass over the binned slots, one slot per lane: count_in_cells.

@@ -8,8 +8,7 @@
 //
 //   * the toroidal bucket table is cut into segments; workgroup `seg` owns
 //     the slots of the agents whose new bucket lies in its segment (segments
-//     dealt to the XCDs in contiguous runs, so that neighbouring windows
-//     share an L2);
+//     dealt to the XCDs in runs, so that neighbouring windows share an L2);
 //   * an agent moves at most D cells per axis, so it lands within `margin`
 //     buckets of its previous bucket: the segment's agents all sit in a
 //     window of the previous slot order;
@@ -412,6 +411,13 @@ __device__ __forceinline__ void sorted_store(const SortedMove& mv, const TableVi
     }
 }
 
+// Order of the segments' workgroups: three move workgroups of 512 threads and
+// 50 KB of LDS share a CU.  The route choice takes the same order, so that a
+// segment's arrival records are in the L2 of the XCD that reads them.
+__device__ __forceinline__ uint32_t seg_order(uint32_t bid, uint32_t n_seg) {
+    return xcd_deal<4>(bid, n_seg, 3u * kCus);
+}
+
 // LDS of the sorted move: the segment's counters (4 bytes per bucket) and,
 // for its first sorted_map_cap new slots, each agent's window index and its
 // bucket in the segment (2 + 2 bytes).  Segments of up to 2^12 buckets map 2
@@ -611,7 +617,7 @@ static __global__ __launch_bounds__(T) void k_move_sorted(SortedMove mv, BinDev 
         if (blockIdx.x == 0) sorted_finish(fin);
         return;
     }
-    const uint32_t seg = xcd_block(blockIdx.x - extra, b.n_seg);
+    const uint32_t seg = seg_order(blockIdx.x - extra, b.n_seg);
     const NextCount nc{nh, mv.next, seg, b.n_seg, 0u, b.seg_log};
     uint32_t base, total;
     sorted_segment<U, T, UNIFORM, WRITE_DIR>(mv, table_view(b), nc, seg << b.seg_log, seg, hist, lds, sh,
@@ -736,7 +742,7 @@ __device__ __forceinline__ void route_segment_list(const SortedMove& mv, const T
 template <bool UNIFORM, bool WRITE_DIR>
 static __global__ __launch_bounds__(kBlock) void k_route_sorted(SortedMove mv, BinDev b) {
     __shared__ uint32_t nh[2 * kNextReach + 1];
-    const uint32_t g = xcd_block(blockIdx.x, gridDim.x);
+    const uint32_t g = seg_order(blockIdx.x, gridDim.x);
     route_segment_list<UNIFORM, WRITE_DIR>(mv, table_view(b), NextCount{nh, mv.next, g, b.n_seg, 0u, b.seg_log}, g);
 }
 
@@ -776,14 +782,14 @@ static __global__ __launch_bounds__(kBlock, 8) void k_route_collide(SortedMove m
     uint32_t r;
     if (mix.routes(blockIdx.x, r)) {
         if (r >= mix.n_route) return;
-        const uint32_t seg = xcd_block(r, mix.n_route);
+        const uint32_t seg = seg_order(r, mix.n_route);
         // the counts this tick's move consumed, cleared for the move after next
         if (threadIdx.x == 0) mv.cur.clear(seg);
         route_segment_list<UNIFORM, false>(mv, table_view(b), NextCount{nh, mv.next, seg, b.n_seg, 0u, b.seg_log},
                                            seg);
     } else {
         if (r >= mix.n_collide) return;
-        collide_block<P>(a, g, bpos, part_pairs, xcd_block(r, mix.n_collide), lds, stage_all);
+        collide_block<P>(a, g, bpos, part_pairs, collide_order(r, mix.n_collide), lds, stage_all);
     }
 }
 
