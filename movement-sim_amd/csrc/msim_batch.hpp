@@ -161,7 +161,7 @@ static __global__ __launch_bounds__(T) void k_bmove_sorted(SortedMove mv, BatchB
     const uint32_t gl = g - sc.seg_first;
     const NextCount nc{nh, mv.next, gl, sc.n_seg, sc.seg_first, sc.seg_log};
     uint32_t base, total;
-    sorted_segment<U, T, UNIFORM, WRITE_DIR>(mv, scen_view(sc, b), nc, gl << sc.seg_log, g, hist, lds, sh,
+    sorted_segment<U, T, UNIFORM, WRITE_DIR, false>(mv, scen_view(sc, b), nc, gl << sc.seg_log, g, hist, lds, sh,
                                              b.new_start + sc.start_base, &base, &total);
     if (gl == sc.n_seg - 1 && threadIdx.x == 0) {
         const uint32_t end = base + total;
@@ -200,7 +200,7 @@ static __global__ __launch_bounds__(kBlock) void k_broute_sorted(SortedMove mv, 
     const uint32_t g = seg_order(blockIdx.x, gridDim.x);
     const ScenDev sc = b.scen[b.seg_scen[g]];
     const NextCount nc{nh, mv.next, g - sc.seg_first, sc.n_seg, sc.seg_first, sc.seg_log};
-    route_segment_list<UNIFORM, WRITE_DIR>(mv, scen_view(sc, b), nc, g);
+    route_segment_list<UNIFORM, WRITE_DIR, false>(mv, scen_view(sc, b), nc, g);
 }
 
 // nxt for every slot of every scenario: the bucket of the agent's next
@@ -372,7 +372,7 @@ static __global__ __launch_bounds__(kBlock, 6) void k_broute_collide(SortedMove 
         // the counts this tick's move consumed, cleared for the move after next
         if (threadIdx.x == 0) mv.cur.clear(g);
         const NextCount nc{nh, mv.next, g - sc.seg_first, sc.n_seg, sc.seg_first, sc.seg_log};
-        route_segment_list<UNIFORM, false>(mv, scen_view(sc, b), nc, g);
+        route_segment_list<UNIFORM, false, false>(mv, scen_view(sc, b), nc, g);
     } else {
         if (r >= mix.n_collide) return;
         bcollide_block<P>(c, collide_order(r, mix.n_collide), stage_all);

@@ -9,19 +9,22 @@
 //   * the toroidal bucket table is cut into segments; workgroup `seg` owns
 //     the slots of the agents whose new bucket lies in its segment (segments
 //     dealt to the XCDs in runs, so that neighbouring windows share an L2);
-//   * an agent moves at most D cells per axis, so it lands within `margin`
-//     buckets of its previous bucket: the segment's agents all sit in a
-//     window of the previous slot order;
-//   * count pass: every window slot carries `nxt`, the bucket of the agent's
-//     next position, computed when the agent was last placed; counting reads
+//   * every slot carries `nxt`, the bucket of its agent's next position,
+//     computed when the agent was last placed; counting and ranking read
 //     these 4 bytes per slot and no state;
+//   * an agent moves at most D cells per axis, so it lands within `margin`
+//     buckets of its previous bucket.  With lists (LISTS), whoever placed an agent that will leave its segment also
+//     listed it (slot, next bucket) for the segment above or below: the
+//     segment's agents are among its own previous slots and its two
+//     neighbours' lists.  Otherwise they are sought in a window of the
+//     previous slot order, the segment and the margin on both sides;
 //   * the segment's first slot follows from counts made before the launch:
 //     the previous move and route choice counted, per segment and per group
 //     of kGroupSegs segments, the agents whose next bucket lies in it, so no
 //     segment waits for another.  Inside run_ticks every workgroup sums the
 //     counts before its segment itself; a single dispatch runs k_seg_scan
 //     first;
-//   * rank: the window slots whose `nxt` lies in the segment take their new
+//   * rank: the window entries whose `nxt` lies in the segment take their new
 //     slots from LDS counters; an LDS map records, per new slot, the old
 //     slot's window index and the counted bucket;
 //   * store pass: the new slots in order (whole lines written per wave),
@@ -118,8 +121,21 @@ struct SegCounts {
     }
 };
 
+// What one segment hands to the next move (LISTS): its slots [x, y) and the
+// lengths of its two lists of agents whose next bucket lies in another
+// segment.  Both lists use the segment's own range of the list array, an
+// entry {slot, next bucket} for each: the z agents going to the segment
+// above from the front, the w agents going below from the back.  An agent is
+// listed at most once, so the range holds them all.  "Above" and "below" are
+// cyclic in the table; with two segments everything goes above.
+struct SegLists {
+    uint4* rec;    // [n_seg]
+    uint2* leave;  // [n]
+};
+
 struct SortedMove {
     SortedBufs src, dst;
+    SegLists from, to;   // LISTS: the lists this move reads, and those it and the route choice write
     uint4* arr_rec;      // [n] arrivals {new slot, caller index, x bits, y bits}, segment g's at
                          // [seg_start[g], + seg_arr[g])
     float* arr_spd;      // [n] their speeds; nullptr with spd_const
@@ -185,24 +201,125 @@ __device__ __forceinline__ void next_flush(const NextCount& nc) {
     }
 }
 
-// Count pass over window slots [lo, hi): agents whose next bucket lies in
-// [s0, s0 + S) bump their LDS counter.
-template <uint32_t U, uint32_t T>
-__device__ __forceinline__ void sorted_count(const uint32_t* __restrict__ nxt, uint32_t s0, uint32_t S, uint32_t lo,
-                                             uint32_t hi, uint32_t* hist) {
-    for (uint32_t base = lo; base < hi; base += U * T) {
+// The agents that may land in a segment, numbered from 0: old slots [a0, a1),
+// then (LISTS) the entries of the lower neighbour's list of agents going up
+// and of the upper neighbour's list of agents going down, or (windows) old
+// slots [c0, c1).
+constexpr uint32_t kListCap = 1024;  // list entries whose slots are kept in LDS (later ones are read again)
+template <bool LISTS>
+struct Window {
+    uint32_t a0, a1, c0, c1;
+    const uint2 *up, *down;  // first entry of the one list, last entry of the other
+    uint32_t n_up, n_list;
+    uint32_t* lslot;  // LDS [kListCap]
+    __device__ uint32_t own() const { return a1 - a0; }
+    __device__ uint32_t size() const { return own() + (LISTS ? n_list : c1 - c0); }
+    __device__ uint2 entry(uint32_t e) const { return e < n_up ? up[e] : *(down - (e - n_up)); }
+    // Next bucket of agent r < size(); keep: note a list entry's slot.
+    __device__ uint32_t bucket(const uint32_t* __restrict__ nxt, uint32_t r, bool keep) const {
+        if (!LISTS) return nxt[slot(r)];
+        if (r < own()) return nxt[a0 + r];
+        const uint32_t k = r - own();
+        const uint2 e = entry(k);
+        if (keep && k < kListCap) lslot[k] = e.x;
+        return e.y;
+    }
+    __device__ uint32_t slot(uint32_t r) const {
+        if (r < own()) return a0 + r;
+        const uint32_t k = r - own();
+        if (!LISTS) return c0 + k;
+        return k < kListCap ? lslot[k] : entry(k).x;
+    }
+};
+
+// Count pass over a window: agents whose next bucket lies in [s0, s0 + S)
+// bump their LDS counter.
+template <uint32_t U, uint32_t T, bool LISTS>
+__device__ __forceinline__ void sorted_count(const Window<LISTS>& win, const uint32_t* __restrict__ nxt, uint32_t s0,
+                                             uint32_t S, uint32_t* hist) {
+    const uint32_t size = win.size();
+    for (uint32_t base = 0; base < size; base += U * T) {
         uint32_t b[U];
 #pragma unroll
         for (uint32_t u = 0; u < U; u++) {
-            b[u] = nxt[min(base + u * T + threadIdx.x, hi - 1u)];
+            const uint32_t r = base + u * T + threadIdx.x;
+            b[u] = win.bucket(nxt, min(r, size - 1u), r < size);
         }
 #pragma unroll
         for (uint32_t u = 0; u < U; u++) {
-            const uint32_t k = base + u * T + threadIdx.x;
             const uint32_t off = b[u] - s0;
-            (void)wave_rank_add(hist, off, k < hi && off < S);
+            (void)wave_rank_add(hist, off, base + u * T + threadIdx.x < size && off < S);
         }
     }
+}
+
+// Lists agents that will leave the segment (LISTS).  g, above, below: the
+// segment and its neighbours in its table; n: LDS [2], the two lists'
+// lengths; [base, end): the segment's new slots.
+struct Leavers {
+    uint32_t* n;
+    uint2* leave;
+    uint32_t base, end;
+    uint32_t g, above, below, seg_log;
+    unsigned int* faults;
+};
+
+// Wave-level (every lane of the wave calls it): lists the agents of new slots
+// q[u] and next buckets b[u] where active[u]; one LDS atomic per wave and
+// direction.
+template <uint32_t U>
+__device__ __forceinline__ void leave_round(const Leavers& lv, const uint32_t (&q)[U], const uint32_t (&b)[U],
+                                            const bool (&active)[U]) {
+    const unsigned long long lt = (1ull << __lane_id()) - 1ull;
+    unsigned long long mu[U], md[U];
+    uint32_t nu = 0, nd = 0;
+    bool far = false;
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) {
+        const uint32_t s = b[u] >> lv.seg_log;
+        const bool out = active[u] && s != lv.g;
+        mu[u] = __ballot(out && s == lv.above);
+        md[u] = __ballot(out && s != lv.above && s == lv.below);
+        far = far || (out && s != lv.above && s != lv.below);
+        nu += static_cast<uint32_t>(__popcll(mu[u]));
+        nd += static_cast<uint32_t>(__popcll(md[u]));
+    }
+    if (far) {
+        atomicOr(lv.faults, kFaultBinCount);  // beyond the margin: the next move would not find it
+    }
+    if (nu + nd == 0u) {  // wave-uniform
+        return;
+    }
+    uint32_t au = 0, ad = 0;
+    if (__lane_id() == 0) {
+        au = atomicAdd(&lv.n[0], nu);
+        ad = atomicAdd(&lv.n[1], nd);
+    }
+    au = lv.base + static_cast<uint32_t>(__shfl(static_cast<int>(au), 0, 64));
+    ad = lv.end - 1u - static_cast<uint32_t>(__shfl(static_cast<int>(ad), 0, 64));
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) {
+        if ((mu[u] >> __lane_id()) & 1ull) lv.leave[au + static_cast<uint32_t>(__popcll(mu[u] & lt))] = make_uint2(q[u], b[u]);
+        if ((md[u] >> __lane_id()) & 1ull) lv.leave[ad - static_cast<uint32_t>(__popcll(md[u] & lt))] = make_uint2(q[u], b[u]);
+        au += static_cast<uint32_t>(__popcll(mu[u]));
+        ad -= static_cast<uint32_t>(__popcll(md[u]));
+    }
+}
+
+// Workgroup-level, after a barrier: adds the next segments of `placed` agents
+// to the next move's counts, of whom the lists received lv.n less n0 (up)
+// and n1 (down); the rest stay.
+__device__ __forceinline__ void leave_flush(const Leavers& lv, const SegCounts& next, uint32_t seg_first,
+                                            uint32_t placed, uint32_t n0, uint32_t n1) {
+    const uint32_t up = lv.n[0] - n0, down = lv.n[1] - n1;
+    if (threadIdx.x == 0u && placed != up + down) next.add(seg_first + lv.g, placed - up - down);
+    if (threadIdx.x == 1u && up) next.add(seg_first + lv.above, up);
+    if (threadIdx.x == 2u && down) next.add(seg_first + lv.below, down);
+}
+
+__device__ __forceinline__ Leavers leavers_of(const SortedMove& mv, const NextCount& nc, uint32_t base, uint32_t end) {
+    return Leavers{nc.nh, mv.to.leave, base, end, nc.g_local, nc.g_local + 1u == nc.n_local ? 0u : nc.g_local + 1u,
+                   nc.g_local ? nc.g_local - 1u : nc.n_local - 1u, nc.seg_log, mv.faults};
 }
 
 // Hot state of the agent in one old slot: next bucket, position, target,
@@ -285,16 +402,21 @@ __device__ __forceinline__ void put_arrival(const SortedMove& mv, uint32_t i, co
     if (!UNIFORM) mv.arr_spd[i] = spd;
 }
 
-// The segment's window: old slots [a0, a1) then [c0, c1), numbered from 0.
-struct Window {
-    uint32_t a0, a1, c0, c1;
-    __device__ uint32_t slot(uint32_t r) const { return r < a1 - a0 ? a0 + r : c0 + (r - (a1 - a0)); }
-    __device__ uint32_t size() const { return (a1 - a0) + (c1 - c0); }
-};
+// Wave-level: the next segment of one placed agent per lane.
+template <bool LISTS>
+__device__ __forceinline__ void next_one(const NextCount& nc, const Leavers& lv, uint32_t q, uint32_t bucket,
+                                         bool active) {
+    if (LISTS) {
+        const uint32_t qs[1] = {q}, bs[1] = {bucket};
+        const bool as[1] = {active};
+        leave_round<1>(lv, qs, bs, as);
+    } else {
+        next_add(nc, bucket, active);
+    }
+}
 
-// Rank pass over window slots [lo, hi) (window-relative index rel0 for lo):
-// each agent whose next bucket lies in the segment takes cursor[bucket]++,
-// its new slot.  The segment's output position j = slot - base records the
+// Rank pass over a window: each agent whose next bucket lies in the segment
+// takes cursor[bucket]++, its new slot.  The segment's output position j = slot - base records the
 // agent's window index in map[j] and its bucket in the segment in mapb[j]
 // when j < cap; past cap (a segment more
 // crowded than the map holds) the agent is moved and stored at once.  A
@@ -303,37 +425,38 @@ struct Window {
 // only the next buckets; the next round's are loaded before this round is
 // ranked.  Waves run the rounds independently (the rank helper needs whole
 // waves, no workgroup barrier).
-template <uint32_t U, uint32_t T, bool UNIFORM, bool WRITE_DIR>
+template <uint32_t U, uint32_t T, bool UNIFORM, bool WRITE_DIR, bool LISTS>
 __device__ __forceinline__ void sorted_rank(const SortedMove& mv, const TableView& t, const NextCount& nc,
-                                            uint32_t s0, uint32_t lo, uint32_t hi, uint32_t rel0, uint32_t* cursor,
-                                            uint16_t* map, uint16_t* mapb, uint32_t base, uint32_t cap,
-                                            uint32_t limit,
-                                            uint32_t* arr_count, uint32_t arr_base, uint32_t& n_ins) {
-    if (lo >= hi) {
+                                            const Leavers& lv, const Window<LISTS>& win, uint32_t s0,
+                                            uint32_t* cursor, uint16_t* map, uint16_t* mapb, uint32_t base,
+                                            uint32_t cap, uint32_t limit, uint32_t* arr_count, uint32_t arr_base,
+                                            uint32_t& n_ins) {
+    const uint32_t size = win.size();
+    if (size == 0u) {
         return;
     }
     const uint32_t S = 1u << t.seg_log;
     uint32_t bn[U];
 #pragma unroll
     for (uint32_t u = 0; u < U; u++) {
-        bn[u] = mv.src.nxt[min(lo + u * T + threadIdx.x, hi - 1u)];
+        bn[u] = win.bucket(mv.src.nxt, min(u * T + threadIdx.x, size - 1u), false);
     }
-    for (uint32_t r0 = lo; r0 < hi; r0 += U * T) {
+    for (uint32_t r0 = 0; r0 < size; r0 += U * T) {
         uint32_t b[U];
 #pragma unroll
         for (uint32_t u = 0; u < U; u++) {
             b[u] = bn[u];
         }
-        if (r0 + U * T < hi) {
+        if (r0 + U * T < size) {
 #pragma unroll
             for (uint32_t u = 0; u < U; u++) {
-                bn[u] = mv.src.nxt[min(r0 + U * T + u * T + threadIdx.x, hi - 1u)];
+                bn[u] = win.bucket(mv.src.nxt, min(r0 + U * T + u * T + threadIdx.x, size - 1u), false);
             }
         }
 #pragma unroll
         for (uint32_t u = 0; u < U; u++) {
             const uint32_t k = r0 + u * T + threadIdx.x;
-            const bool mine = k < hi && b[u] - s0 < S;
+            const bool mine = k < size && b[u] - s0 < S;
             const uint32_t j = wave_rank_add(cursor, b[u] - s0, mine) - base;
             bool moved = false, arr = false;
             uint32_t nb = 0;
@@ -343,15 +466,15 @@ __device__ __forceinline__ void sorted_rank(const SortedMove& mv, const TableVie
                 if (j >= limit) {
                     atomicOr(mv.faults, kFaultBinCount);
                 } else if (j < cap) {
-                    map[j] = static_cast<uint16_t>(rel0 + (k - lo));
+                    map[j] = static_cast<uint16_t>(k);
                     mapb[j] = static_cast<uint16_t>(b[u] - s0);
                 } else {
                     moved = true;
-                    arr = move_agent<UNIFORM, WRITE_DIR>(mv, t, k, b[u], base + j, n_ins, rec, rs, nb);
+                    arr = move_agent<UNIFORM, WRITE_DIR>(mv, t, win.slot(k), b[u], base + j, n_ins, rec, rs, nb);
                     if (arr) put_arrival<UNIFORM>(mv, arr_base + atomicAdd(arr_count, 1u), rec, rs);
                 }
             }
-            next_add(nc, nb, moved && !arr);
+            next_one<LISTS>(nc, lv, base + j, nb, moved && !arr);
         }
     }
 }
@@ -363,9 +486,10 @@ __device__ __forceinline__ void sorted_rank(const SortedMove& mv, const TableVie
 // the first agent is stepped (its stores would otherwise hold back the
 // next agent's loads).  Arrivals are listed for k_route_sorted (one LDS
 // atomic per wave and round).
-template <uint32_t U, uint32_t T, bool UNIFORM, bool WRITE_DIR>
+template <uint32_t U, uint32_t T, bool UNIFORM, bool WRITE_DIR, bool LISTS>
 __device__ __forceinline__ void sorted_store(const SortedMove& mv, const TableView& t, const NextCount& nc,
-                                             const Window& win, const uint16_t* map, const uint16_t* mapb,
+                                             const Leavers& lv, const Window<LISTS>& win, const uint16_t* map,
+                                             const uint16_t* mapb,
                                              uint32_t s0, uint32_t base, uint32_t count,
                                              uint32_t* arr_count, uint32_t arr_base, uint32_t& n_ins) {
     const unsigned long long lt = (1ull << __lane_id()) - 1ull;
@@ -374,6 +498,8 @@ __device__ __forceinline__ void sorted_store(const SortedMove& mv, const TableVi
         uint4 rec[U];
         float rs[U];
         HotAgent ag[U];
+        uint32_t nb[U], q[U];
+        bool stays[U];
 #pragma unroll
         for (uint32_t u = 0; u < U; u++) {  // j0 < count: slot count - 1 is mapped
             const uint32_t j = min(j0 + u * T + threadIdx.x, count - 1u);
@@ -383,12 +509,15 @@ __device__ __forceinline__ void sorted_store(const SortedMove& mv, const TableVi
         for (uint32_t u = 0; u < U; u++) {
             const uint32_t j = j0 + u * T + threadIdx.x;
             arr[u] = false;
-            uint32_t nb = 0;
+            nb[u] = 0;
+            q[u] = base + j;
             if (j < count) {
-                arr[u] = step_agent<UNIFORM, WRITE_DIR>(mv, t, ag[u], base + j, n_ins, rec[u], rs[u], nb);
+                arr[u] = step_agent<UNIFORM, WRITE_DIR>(mv, t, ag[u], q[u], n_ins, rec[u], rs[u], nb[u]);
             }
-            next_add(nc, nb, j < count && !arr[u]);
+            stays[u] = j < count && !arr[u];
+            if (!LISTS) next_add(nc, nb[u], stays[u]);
         }
+        if (LISTS) leave_round<U>(lv, q, nb, stays);
         unsigned long long am[U];
         uint32_t round_arr = 0;
 #pragma unroll
@@ -422,11 +551,12 @@ __device__ __forceinline__ uint32_t seg_order(uint32_t bid, uint32_t n_seg) {
 // for its first sorted_map_cap new slots, each agent's window index and its
 // bucket in the segment (2 + 2 bytes).  Segments of up to 2^12 buckets map 2
 // slots per bucket (12 bytes per bucket in all), larger ones 1 (8 bytes).
+// The slots of list entries follow the maps.
 __host__ __device__ constexpr uint32_t sorted_map_cap(uint32_t seg_log) {
     return seg_log <= 12u ? (2u << seg_log) : (1u << seg_log);
 }
 __host__ __device__ constexpr size_t sorted_lds_bytes(uint32_t seg_log) {
-    return (size_t{4} << seg_log) + size_t{4} * sorted_map_cap(seg_log);
+    return (size_t{4} << seg_log) + size_t{4} * sorted_map_cap(seg_log) + size_t{4} * kListCap;
 }
 
 // Count and place segment g (global index; s0 its first bucket in table t).
@@ -434,7 +564,7 @@ __host__ __device__ constexpr size_t sorted_lds_bytes(uint32_t seg_log) {
 // *base_out / *total_out receive the segment's first slot and agent count
 // (all threads).  The segment's insert and arrival counts go to the
 // statistics slots; its agents' next segments are counted for the next move.
-template <uint32_t U, uint32_t T, bool UNIFORM, bool WRITE_DIR>
+template <uint32_t U, uint32_t T, bool UNIFORM, bool WRITE_DIR, bool LISTS>
 __device__ __forceinline__ void sorted_segment(const SortedMove& mv, const TableView& t, const NextCount& nc,
                                                uint32_t s0, uint32_t g, uint32_t* hist, uint32_t* lds,
                                                uint32_t* sh, uint32_t* __restrict__ start_out, uint32_t* base_out,
@@ -462,17 +592,31 @@ __device__ __forceinline__ void sorted_segment(const SortedMove& mv, const Table
         sh[0] = 0u;  // the segment's arrivals so far
     }
     __syncthreads();
-    uint32_t a0, a1, c0, c1;
-    bin_window(t, s0, a0, a1, c0, c1);
-    const Window win{a0, a1, c0, c1};
+    uint16_t* map = reinterpret_cast<uint16_t*>(hist + S);
+    uint16_t* mapb = map + sorted_map_cap(t.seg_log);
+    Window<LISTS> win{};
+    if (LISTS) {
+        const uint32_t first = g - nc.g_local;
+        const Leavers at = leavers_of(mv, nc, 0u, 0u);
+        const uint4 me = mv.from.rec[g], lo = mv.from.rec[first + at.below], hi = mv.from.rec[first + at.above];
+        win.a0 = me.x;
+        win.a1 = me.y;
+        win.up = mv.from.leave + lo.x;
+        win.down = mv.from.leave + hi.y - 1;
+        win.n_up = nc.n_local > 1u ? lo.z : 0u;
+        win.n_list = win.n_up + (nc.n_local > 1u ? hi.w : 0u);
+        win.lslot = reinterpret_cast<uint32_t*>(mapb + sorted_map_cap(t.seg_log));
+    } else {
+        bin_window(t, s0, win.a0, win.a1, win.c0, win.c1);
+    }
     const uint32_t wsize = win.size();
     // A window of at most R T slots is counted in one round whose LDS
     // atomics also give each agent its rank in its bucket (kept in
     // registers, so no rank pass is needed); larger windows are counted,
     // then ranked, in rounds.
-    // (U = 4: 12 slots per thread, 6,144 per round, so that more windows
-    // take one round; the registers stay within the same occupancy)
-    constexpr uint32_t R = U == 4 ? 12 : 2 * U;
+    // (U <= 4: 3 U slots per thread, 6,144 per round at U = 4, so that more
+    // windows take one round; the registers stay within the same occupancy)
+    constexpr uint32_t R = U <= 4 ? 3 * U : 2 * U;
     const bool one_round = wsize <= R * T;  // workgroup-uniform
     // (bucket offset << 16) | rank in the bucket, ~0 when not the segment's
     // agent (segments have at most 2^14 buckets, windows here R T <= 2^13 slots)
@@ -482,7 +626,7 @@ __device__ __forceinline__ void sorted_segment(const SortedMove& mv, const Table
 #pragma unroll
         for (uint32_t r = 0; r < R; r++) {
             const uint32_t idx = r * T + tid;
-            b[r] = idx < wsize ? mv.src.nxt[win.slot(idx)] : 0u;
+            b[r] = idx < wsize ? win.bucket(mv.src.nxt, idx, true) : 0u;
         }
 #pragma unroll
         for (uint32_t r = 0; r < R; r++) {
@@ -492,8 +636,7 @@ __device__ __forceinline__ void sorted_segment(const SortedMove& mv, const Table
             pk[r] = mine ? (off << 16) | rank : ~0u;
         }
     } else {
-        sorted_count<2 * U, T>(mv.src.nxt, s0, S, a0, a1, hist);
-        sorted_count<2 * U, T>(mv.src.nxt, s0, S, c0, c1, hist);
+        sorted_count<2 * U, T>(win, mv.src.nxt, s0, S, hist);
     }
     if (mv.cur.seg) {
         before = wave_sum(before);
@@ -532,8 +675,7 @@ __device__ __forceinline__ void sorted_segment(const SortedMove& mv, const Table
         start_out[s0 + j] = min(hist[j], base + limit);
     }
     uint32_t n_ins = 0;
-    uint16_t* map = reinterpret_cast<uint16_t*>(hist + S);
-    uint16_t* mapb = map + sorted_map_cap(t.seg_log);
+    const Leavers lv = leavers_of(mv, nc, base, end);
     // window indices must fit the map's 16 bits; a window past that moves
     // every agent straight from the rank pass
     const uint32_t cap = wsize <= 65536u ? sorted_map_cap(t.seg_log) : 0u;
@@ -542,9 +684,10 @@ __device__ __forceinline__ void sorted_segment(const SortedMove& mv, const Table
         for (uint32_t r = 0; r < R; r++) {
             const uint32_t idx = r * T + tid;
             bool moved = false, arr = false;
-            uint32_t nb = 0;
+            uint32_t nb = 0, q = 0;
             if (pk[r] != ~0u) {
                 const uint32_t j = hist[pk[r] >> 16] - base + (pk[r] & 0xffffu);
+                q = base + j;
                 if (j >= limit) {
                     atomicOr(mv.faults, kFaultBinCount);
                 } else if (j < cap) {
@@ -559,20 +702,23 @@ __device__ __forceinline__ void sorted_segment(const SortedMove& mv, const Table
                     if (arr) put_arrival<UNIFORM>(mv, base + atomicAdd(&sh[0], 1u), rec, rs);
                 }
             }
-            next_add(nc, nb, moved && !arr);
+            next_one<LISTS>(nc, lv, q, nb, moved && !arr);
         }
     } else {
         __syncthreads();  // the rank pass advances the offsets the stores above read
-        sorted_rank<U, T, UNIFORM, WRITE_DIR>(mv, t, nc, s0, a0, a1, 0u, hist, map, mapb, base, cap, limit,
-                                              &sh[0], base, n_ins);
-        sorted_rank<U, T, UNIFORM, WRITE_DIR>(mv, t, nc, s0, c0, c1, a1 - a0, hist, map, mapb, base, cap, limit,
-                                              &sh[0], base, n_ins);
+        sorted_rank<U, T, UNIFORM, WRITE_DIR, LISTS>(mv, t, nc, lv, win, s0, hist, map, mapb, base, cap, limit,
+                                                     &sh[0], base, n_ins);
     }
     __syncthreads();
-    sorted_store<U, T, UNIFORM, WRITE_DIR>(mv, t, nc, win, map, mapb, s0, base, min(min(total, cap), limit),
-                                           &sh[0], base, n_ins);
+    sorted_store<U, T, UNIFORM, WRITE_DIR, LISTS>(mv, t, nc, lv, win, map, mapb, s0, base,
+                                                  min(min(total, cap), limit), &sh[0], base, n_ins);
     __syncthreads();
-    next_flush(nc);
+    if (LISTS) {
+        leave_flush(lv, nc.next, g - nc.g_local, min(total, limit) - sh[0], 0u, 0u);
+        if (tid == 0) mv.to.rec[g] = make_uint4(base, end, lv.n[0], lv.n[1]);
+    } else {
+        next_flush(nc);
+    }
     // block totals of insertions and arrivals, one slot update each
     const uint32_t si = block_sum<T>(n_ins, lds);
     if (tid == 0) {
@@ -606,7 +752,7 @@ __device__ __forceinline__ void sorted_finish(const SortedFinish& f) {
 // Sorted move of one table (grid: n_seg workgroups, after kXcds more when the
 // previous tick's statistics are pending; dynamic LDS:
 // sorted_lds_bytes(seg_log)).
-template <uint32_t U, uint32_t T, bool UNIFORM, bool WRITE_DIR>
+template <uint32_t U, uint32_t T, bool UNIFORM, bool WRITE_DIR, bool LISTS>
 static __global__ __launch_bounds__(T) void k_move_sorted(SortedMove mv, BinDev b, SortedFinish fin) {
     extern __shared__ uint32_t hist[];
     __shared__ uint32_t lds[T / 64];
@@ -620,7 +766,7 @@ static __global__ __launch_bounds__(T) void k_move_sorted(SortedMove mv, BinDev 
     const uint32_t seg = seg_order(blockIdx.x - extra, b.n_seg);
     const NextCount nc{nh, mv.next, seg, b.n_seg, 0u, b.seg_log};
     uint32_t base, total;
-    sorted_segment<U, T, UNIFORM, WRITE_DIR>(mv, table_view(b), nc, seg << b.seg_log, seg, hist, lds, sh,
+    sorted_segment<U, T, UNIFORM, WRITE_DIR, LISTS>(mv, table_view(b), nc, seg << b.seg_log, seg, hist, lds, sh,
                                              b.new_start, &base, &total);
     if (seg == b.n_seg - 1 && threadIdx.x == 0) {
         b.new_start[b.m] = base + total;
@@ -703,21 +849,24 @@ static __global__ __launch_bounds__(T) void k_seg_scan(uint32_t* __restrict__ cn
 // (random_move.comp:778-828) updates the caller-order route state and gives
 // the new target, the bucket of the next move and (last tick of a batch) the
 // heading.
-template <bool UNIFORM, bool WRITE_DIR>
+template <bool UNIFORM, bool WRITE_DIR, bool LISTS>
 __device__ __forceinline__ void route_segment_list(const SortedMove& mv, const TableView& t, const NextCount& nc,
                                                    uint32_t g) {
     const SortedBufs& dst = mv.dst;
+    const uint4 sr = LISTS ? mv.to.rec[g] : make_uint4(0u, 0u, 0u, 0u);
+    const uint32_t base = LISTS ? sr.x : min(mv.seg_start[g], mv.n), cnt = mv.seg_arr[g];
+    const Leavers lv = leavers_of(mv, nc, base, sr.y);
     if (threadIdx.x < 2 * kNextReach + 1) {
-        nc.nh[threadIdx.x] = 0u;
+        nc.nh[threadIdx.x] = !LISTS || threadIdx.x > 1u ? 0u : (threadIdx.x ? sr.w : sr.z);
     }
     __syncthreads();
-    const uint32_t base = min(mv.seg_start[g], mv.n), cnt = mv.seg_arr[g];
     for (uint32_t j0 = 0; j0 < cnt; j0 += blockDim.x) {  // whole-block rounds: next_add is wave-level
         const uint32_t j = j0 + threadIdx.x;
-        uint32_t nb = 0;
+        uint32_t nb = 0, q = 0;
         if (j < cnt) {
             const uint4 a = mv.arr_rec[base + j];
-            const uint32_t q = a.x, hh = a.y;
+            const uint32_t hh = a.y;
+            q = a.x;
             const float2 at = make_float2(__uint_as_float(a.z), __uint_as_float(a.w));
             const float s = UNIFORM ? mv.spd_const : mv.arr_spd[base + j];
             const uint4 w = mv.cold[2u * hh];
@@ -733,17 +882,22 @@ __device__ __forceinline__ void route_segment_list(const SortedMove& mv, const T
             dst.nxt[q] = nb;
             if (WRITE_DIR) dst.dir[q] = heading(nt, at, s);
         }
-        next_add(nc, nb, j < cnt);
+        next_one<LISTS>(nc, lv, q, nb, j < cnt);
     }
     __syncthreads();
-    next_flush(nc);
+    if (LISTS) {
+        leave_flush(lv, nc.next, g - nc.g_local, cnt, sr.z, sr.w);
+        if (threadIdx.x == 0) mv.to.rec[g] = make_uint4(sr.x, sr.y, lv.n[0], lv.n[1]);
+    } else {
+        next_flush(nc);
+    }
 }
 
-template <bool UNIFORM, bool WRITE_DIR>
+template <bool UNIFORM, bool WRITE_DIR, bool LISTS>
 static __global__ __launch_bounds__(kBlock) void k_route_sorted(SortedMove mv, BinDev b) {
     __shared__ uint32_t nh[2 * kNextReach + 1];
     const uint32_t g = seg_order(blockIdx.x, gridDim.x);
-    route_segment_list<UNIFORM, WRITE_DIR>(mv, table_view(b), NextCount{nh, mv.next, g, b.n_seg, 0u, b.seg_log}, g);
+    route_segment_list<UNIFORM, WRITE_DIR, LISTS>(mv, table_view(b), NextCount{nh, mv.next, g, b.n_seg, 0u, b.seg_log}, g);
 }
 
 // Route choice and neighbour pass in one launch (run_ticks only).  Neither
@@ -771,7 +925,7 @@ struct RouteMix {
     }
 };
 
-template <bool UNIFORM, int P>
+template <bool UNIFORM, int P, bool LISTS>
 static __global__ __launch_bounds__(kBlock, 8) void k_route_collide(SortedMove mv, BinDev b, AgentsDev a, GridDev g,
                                                                     const float2* __restrict__ bpos,
                                                                     unsigned long long* __restrict__ part_pairs,
@@ -785,7 +939,7 @@ static __global__ __launch_bounds__(kBlock, 8) void k_route_collide(SortedMove m
         const uint32_t seg = seg_order(r, mix.n_route);
         // the counts this tick's move consumed, cleared for the move after next
         if (threadIdx.x == 0) mv.cur.clear(seg);
-        route_segment_list<UNIFORM, false>(mv, table_view(b), NextCount{nh, mv.next, seg, b.n_seg, 0u, b.seg_log},
+        route_segment_list<UNIFORM, false, LISTS>(mv, table_view(b), NextCount{nh, mv.next, seg, b.n_seg, 0u, b.seg_log},
                                            seg);
     } else {
         if (r >= mix.n_collide) return;
@@ -809,21 +963,55 @@ __device__ __forceinline__ void count_next_segment(const SegCounts& next, uint32
     }
 }
 
+// Entering the sorted state (LISTS): lists the agent of slot q, in segment gl
+// of n_seg, if its next bucket lies in another segment.
+__device__ __forceinline__ void init_leave(const SegLists& to, unsigned int* faults, uint32_t q, uint32_t bucket,
+                                           uint32_t gl, uint32_t n_seg, uint32_t seg_log) {
+    const uint32_t s = bucket >> seg_log;
+    if (s == gl) {
+        return;
+    }
+    uint4* r = &to.rec[gl];
+    if (s == (gl + 1u == n_seg ? 0u : gl + 1u)) {
+        to.leave[r->x + atomicAdd(&r->z, 1u)] = make_uint2(q, bucket);
+    } else if (s == (gl ? gl - 1u : n_seg - 1u)) {
+        to.leave[r->y - 1u - atomicAdd(&r->w, 1u)] = make_uint2(q, bucket);
+    } else {
+        atomicOr(faults, kFaultBinCount);
+    }
+}
+
+// Entering the sorted state (LISTS): the segments' slots, both lists empty.
+static __global__ __launch_bounds__(kBlock) void k_seg_records(SegLists to, const uint32_t* __restrict__ start,
+                                                               uint32_t n_seg, uint32_t seg_log) {
+    const uint32_t g = blockIdx.x * kBlock + threadIdx.x;
+    if (g < n_seg) {
+        to.rec[g] = make_uint4(start[g << seg_log], start[(g + 1u) << seg_log], 0u, 0u);
+    }
+}
+
 // nxt for every slot of one table: the bucket of the agent's next position;
-// next (cleared before) counts them per segment.
+// next (cleared before) counts them per segment, and to (LISTS; null
+// otherwise, records initialised) lists those that leave theirs.
 template <bool UNIFORM>
 static __global__ __launch_bounds__(kBlock) void k_sorted_next(SortedBufs st, uint32_t n, float spd_const,
                                                                float inv_cell, uint32_t lw, uint32_t wmask,
                                                                uint32_t hmask, uint32_t seg_log,
-                                                               SegCounts next) {
+                                                               SegCounts next, SegLists to, uint32_t n_seg,
+                                                               unsigned int* faults) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     uint32_t b = 0;
     if (i < n) {
         const uint4 r = st.rec[i];
-        const float2 np = next_position(st.pos[i], make_float2(__uint_as_float(r.x), __uint_as_float(r.y)),
+        const float2 p = st.pos[i];
+        const float2 np = next_position(p, make_float2(__uint_as_float(r.x), __uint_as_float(r.y)),
                                         UNIFORM ? spd_const : __uint_as_float(r.z));
         b = bucket_of(cell_coord(np.x, inv_cell), cell_coord(np.y, inv_cell), lw, wmask, hmask);
         st.nxt[i] = b;
+        if (to.rec) {
+            const uint32_t at = bucket_of(cell_coord(p.x, inv_cell), cell_coord(p.y, inv_cell), lw, wmask, hmask);
+            init_leave(to, faults, i, b, at >> seg_log, n_seg, seg_log);
+        }
     }
     count_next_segment(next, b >> seg_log, i < n);
 }

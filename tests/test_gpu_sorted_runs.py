@@ -47,3 +47,27 @@ def test_batch_run_folds_every_scenarios_pairs(n_scen):
         np.testing.assert_array_equal(st["pos"].view(np.uint32), o.st.pos.view(np.uint32), err_msg=f"scenario {s}")
         np.testing.assert_array_equal(st["rng"], o.st.rng, err_msg=f"scenario {s}")
     b.sync()
+
+
+@pytest.mark.parametrize("opts,agents", [
+    (dict(table_log2=12, segment_log2=12, table_width_log2=8), 4000),   # one segment: nothing leaves it
+    (dict(table_log2=12, segment_log2=11, table_width_log2=7), 4000),   # two: each is above and below the other
+    (dict(table_log2=12, segment_log2=10, table_width_log2=6), 4000),   # four, a few rows each
+    (dict(table_log2=13, segment_log2=9, table_width_log2=7), 4000),    # margin wider than 3/4 of a segment
+    (dict(table_log2=14, segment_log2=12, table_width_log2=10), 60000),  # more leavers than their slots fit in LDS
+    (dict(table_log2=13, segment_log2=12, table_width_log2=9), 60000),  # crowded past the map and its 16-bit window
+])
+def test_lists_of_leaving_agents_match_oracle(opts, agents):
+    sc = S.config(1)
+    sc.entities, sc.speed = S.place_agents(sc.roads, agents, 5)
+    g, o = pair(sc, threads=4, binning=3, graph_ticks=6, **opts)
+    for ticks in (1, 20):
+        g.run_ticks(ticks)
+        o.run_ticks(ticks)
+        assert_same(g.state(), o.st, f"{opts}")
+    for _ in range(6):  # the same lists through single dispatches
+        g.dispatch()
+        o.dispatch()
+    assert_same(g.state(), o.st, f"{opts}, dispatches")
+    assert g.pairs()[0] == o.pairs_total
+    g.sync()
