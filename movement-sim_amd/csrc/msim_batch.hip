@@ -453,26 +453,35 @@ extern "C" int msim_batch_create(uint32_t n_scen, const uint32_t* road_off, cons
         for (uint32_t i = 0; i < n; i++) smax = std::max(smax, speed[i]);
     }
     const uint32_t D = static_cast<uint32_t>(std::floor(smax * (1.0f + 1.0f / 1048576.0f) / cell)) + 1u;
+    uint64_t buckets = 0;
     for (uint32_t s = 0; s < n_scen; s++) {
         ScenDev& d = sc[s];
         d.agent_off = agent_off[s];
         d.n = agent_off[s + 1] - agent_off[s];
-        const uint32_t tlog = auto_table_log2(d.n);
-        const uint32_t rows_log = extent_rows_log2(roads + road_off[s], road_off[s + 1] - road_off[s],
-                                                   entities + agent_off[s], d.n, cell);
+        uint32_t tlog = auto_table_log2(d.n);
+        const Extent ext = extent_of(roads + road_off[s], road_off[s + 1] - road_off[s], entities + agent_off[s], d.n);
+        const uint32_t rows_log = extent_rows_log2(ext, cell);
         d.lw = o.table_width_log2 ? std::max(2u, std::min(o.table_width_log2, tlog - 2u))
                                   : auto_width_log2(tlog, rows_log);
-        uint32_t seg_log = auto_segment_log2(tlog, d.lw);
+        if (!o.table_width_log2 && !o.segment_log2) {
+            (void)whole_world_table(d.n, ext.rows(cell), ext.cols(cell), &tlog, &d.lw);
+        }
+        d.m = 1u << tlog;
+        d.wmask = (1u << d.lw) - 1u;
+        d.hmask = (1u << (tlog - d.lw)) - 1u;
+        d.margin = (D + 1u) * (d.wmask + 1u) + D;
+        buckets += d.m;
+    }
+    for (uint32_t s = 0; s < n_scen; s++) {
+        ScenDev& d = sc[s];
+        const uint32_t tlog = ceil_log2_u64(d.m);
+        uint32_t seg_log = auto_batch_segment_log2(buckets, tlog, d.lw);
         if (o.segment_log2) seg_log = std::min(std::max(o.segment_log2, 9u), tlog);
         auto lds_need = [&](uint32_t l) {
             return (o.binning == 3 ? sorted_lds_bytes(l) : (static_cast<size_t>(4) << l)) + 1024;
         };
         while (seg_log > 9 && lds_need(seg_log) > static_cast<size_t>(lds_max)) seg_log--;
         d.seg_log = seg_log;
-        d.m = 1u << tlog;
-        d.wmask = (1u << d.lw) - 1u;
-        d.hmask = (1u << (tlog - d.lw)) - 1u;
-        d.margin = (D + 1u) * (d.wmask + 1u) + D;
         d.start_base = start_len;
         start_len += d.m + 1u;
         d.seg_first = static_cast<uint32_t>(seg_scen.size());

@@ -2,6 +2,7 @@
 // map/agent validation, grid sizing and the exact squared-radius threshold.
 #pragma once
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -49,11 +50,32 @@ inline uint32_t auto_width_log2(uint32_t tlog, uint32_t rows_log) {
     return l;
 }
 
-// Segment owned by one rebinning workgroup: 16 table rows, 512..16384
-// buckets (at most 64 KB of LDS counters).
+// Segment owned by one rebinning workgroup: about 128 segments of 2^9 to
+// 2^11 buckets (2^12 in tables of 2^22 and more), or two table rows where
+// those are longer (a window adds one to three rows on both sides), up to
+// 2^14 buckets (64 KB of LDS counters).  Ticks of the classic layout, us: 1M
+// agents on 2^20 buckets in rows of 2^10: 61.5 at 2^12, 62.5 at 2^11, 74 at
+// 2^10, 71 at 2^13; in rows of 2^11, 88 at 2^14 (64 segments, most CUs idle)
+// against 73; in rows of 2^7, 56 at 2^11, 58 at 2^12; 123k agents on 2^17: 33
+// at 2^9 and 2^10, 34 at 2^11, 39 at 2^12.
 inline uint32_t auto_segment_log2(uint32_t tlog, uint32_t lw) {
-    uint32_t l = lw + 4;
-    if (l < 9) l = 9;
+    uint32_t l = tlog > 21u ? 12u : (tlog > 18u ? 11u : (tlog > 16u ? tlog - 7u : 9u));
+    if (l < lw + 1u) l = lw + 1u;
+    if (l > 14) l = 14;
+    if (l > tlog) l = tlog;
+    return l;
+}
+
+// The same for one of many tables in a launch, of `buckets` in all, whose
+// segments fill the GPU together: 2^11 buckets, fewer while that leaves less
+// than 384 segments.  Count + place of 64 scenarios of 5.8M agents: 210 us at
+// 2^9 buckets (16 rows), 127 at 2^10, 92 at 2^11 and 2^12, 118 at 2^13; a
+// differentiable run of 7 scenarios on 2^16 buckets each was 2% slower at 2^11
+// (224 segments) than at 2^10.
+inline uint32_t auto_batch_segment_log2(uint64_t buckets, uint32_t tlog, uint32_t lw) {
+    uint32_t l = 11;
+    while (l > 9 && (buckets >> l) < 384u) l--;
+    if (l < lw + 1u) l = lw + 1u;
     if (l > 14) l = 14;
     if (l > tlog) l = tlog;
     return l;
@@ -64,30 +86,63 @@ inline uint32_t auto_segment_log2(uint32_t tlog, uint32_t lw) {
 // per CU) measured faster with 4.
 inline uint32_t auto_bin_unroll(uint32_t seg_log) { return seg_log <= 13 ? 8u : 4u; }
 
-// floor(log2(rows spanned by the roads and agents, in cells)), at least 2.
-inline uint32_t extent_rows_log2(const msim_road* roads, uint32_t n_roads, const msim_entity* e, uint32_t n,
-                                 float cell) {
-    double lo = 0, hi = 0;
-    bool any = false;
-    auto add = [&](float y) {
-        if (!any) {
-            lo = hi = y;
-            any = true;
-        }
-        lo = y < lo ? y : lo;
-        hi = y > hi ? y : hi;
+// Bounding box of the roads and agents.
+struct Extent {
+    float x0 = 0.0f, x1 = 0.0f, y0 = 0.0f, y1 = 0.0f;
+    // Cells spanned (one past the last).
+    double cols(float cell) const { return std::floor(double{x1} / cell) - std::floor(double{x0} / cell) + 1.0; }
+    double rows(float cell) const { return std::floor(double{y1} / cell) - std::floor(double{y0} / cell) + 1.0; }
+};
+
+inline Extent extent_of(const msim_road* roads, uint32_t n_roads, const msim_entity* e, uint32_t n) {
+    Extent b;
+    auto add = [&](float x, float y) {
+        b.x0 = std::min(b.x0, x);
+        b.x1 = std::max(b.x1, x);
+        b.y0 = std::min(b.y0, y);
+        b.y1 = std::max(b.y1, y);
     };
+    if (n_roads) {
+        b = Extent{roads[0].start.pos.x, roads[0].start.pos.x, roads[0].start.pos.y, roads[0].start.pos.y};
+    } else if (n) {
+        b = Extent{e[0].pos.x, e[0].pos.x, e[0].pos.y, e[0].pos.y};
+    }
     for (uint32_t r = 0; r < n_roads; r++) {
-        add(roads[r].start.pos.y);
-        add(roads[r].end.pos.y);
+        add(roads[r].start.pos.x, roads[r].start.pos.y);
+        add(roads[r].end.pos.x, roads[r].end.pos.y);
     }
     for (uint32_t i = 0; i < n; i++) {
-        add(e[i].pos.y);
+        add(e[i].pos.x, e[i].pos.y);
     }
-    const double rows = (hi - lo) / cell + 1.0;
+    return b;
+}
+
+// floor(log2(rows spanned, in cells)), at least 2.
+inline uint32_t extent_rows_log2(const Extent& b, float cell) {
+    const double rows = (double{b.y1} - double{b.y0}) / cell + 1.0;
     uint32_t l = 2;
     while (l < 30 && static_cast<double>(1ull << (l + 1)) <= rows) l++;
     return l;
+}
+
+// A table that holds the whole world, one bucket per cell, where that takes
+// no more buckets than the agents' own table (2^tlog): its rows are as short
+// as the world, so the rebinning windows are narrow, and no bucket mixes far
+// cells.  (Folded onto rows of 2^11, 1M agents in a world of 781 x 781 cells
+// had 62% of each row empty.)  Crowded worlds, with more than 8,192 agents per
+// 512 buckets, keep the agents' own table for its number of segments.
+inline bool whole_world_table(uint32_t n, double rows, double cols, uint32_t* tlog, uint32_t* lw) {
+    auto ceil_log2 = [](double v) {
+        uint32_t l = 0;
+        while (l < 31 && static_cast<double>(1ull << l) < v) l++;
+        return l;
+    };
+    const uint32_t cr = std::max(2u, ceil_log2(rows)), cc = std::max(2u, ceil_log2(cols));
+    const uint32_t t = std::max(12u, cr + cc);
+    if (t > *tlog || (static_cast<uint64_t>(n) >> 13) > (1ull << (t - 9u))) return false;
+    *tlog = t;
+    *lw = cc;
+    return true;
 }
 
 // Ticks per captured segment: whole reorder periods (at least one), about

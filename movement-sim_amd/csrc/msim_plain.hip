@@ -952,8 +952,12 @@ extern "C" int msim_create(const msim_road* roads, uint32_t n_roads, const uint3
     if (tlog < 12 || tlog > 28) {
         return fail(nullptr, MSIM_ERR_INVALID, "table_log2 must be in [12, 28]");
     }
-    const uint32_t rows_log = extent_rows_log2(roads, n_roads, entities, n_entities, cell);
-    const uint32_t lw = o.table_width_log2 ? o.table_width_log2 : auto_width_log2(tlog, rows_log);
+    const Extent ext = extent_of(roads, n_roads, entities, n_entities);
+    const uint32_t rows_log = extent_rows_log2(ext, cell);
+    uint32_t lw = o.table_width_log2 ? o.table_width_log2 : auto_width_log2(tlog, rows_log);
+    if (!o.table_log2 && !o.table_width_log2 && !o.segment_log2) {
+        (void)whole_world_table(n_entities, ext.rows(cell), ext.cols(cell), &tlog, &lw);
+    }
     if (lw < 2 || lw + 2 > tlog) {
         return fail(nullptr, MSIM_ERR_INVALID, "table_width_log2 must be in [2, table_log2 - 2]");
     }
