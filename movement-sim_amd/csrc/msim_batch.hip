@@ -438,10 +438,9 @@ extern "C" int msim_batch_create(uint32_t n_scen, const uint32_t* road_off, cons
         delete b;
         return bfail(nullptr, MSIM_ERR_HIP, "hipStreamCreate failed");
     }
-    int dev = 0;
-    (void)hipGetDevice(&dev);
+    (void)hipGetDevice(&b->device);
     int lds_max = 65536;
-    (void)hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
+    (void)hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, b->device);
 
     // per-scenario table layout
     std::vector<ScenDev> sc(n_scen);
@@ -546,6 +545,15 @@ extern "C" int msim_batch_create(uint32_t n_scen, const uint32_t* road_off, cons
     BALLOC(b->last, n_scen);
     BALLOC(b->faults, 1);
     BALLOC(b->qdummy, kQueues * kQueueStride);
+    uint32_t n_max = 0;
+    for (const ScenDev& d : sc) n_max = std::max(n_max, d.n);
+    BALLOC(b->read_stage, StateOut::kWords * static_cast<size_t>(n_max));
+    if (rc == MSIM_OK && hipHostMalloc(reinterpret_cast<void**>(&b->box), sizeof(Mailbox), hipHostMallocDefault) !=
+                             hipSuccess) {
+        b->box = nullptr;
+        rc = bfail(b, MSIM_ERR_OOM, "hipHostMalloc(%zu) failed", sizeof(Mailbox));
+    }
+    if (rc == MSIM_OK) b->box->word = 0;
 #undef BALLOC
     if (rc != MSIM_OK) {
         std::string e = b->err;
@@ -686,11 +694,12 @@ extern "C" int msim_batch_run_ticks(msim_batch* b, uint32_t n_ticks) {
 
 extern "C" int msim_batch_sync(msim_batch* b) {
     if (!b) return bfail(b, MSIM_ERR_INVALID, "NULL handle");
-    unsigned int f = 0;
-    hipError_t e = hipMemcpyAsync(&f, b->faults, sizeof(f), hipMemcpyDeviceToHost, b->stream);
-    if (e != hipSuccess) return bfail(b, MSIM_ERR_HIP, "fault readback: %s", hipGetErrorString(e));
-    int rc = bwait(b);
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, b->stream, b->faults, b->box, ++b->reports);
+    int rc = bcheck(b, "k_report");
     if (rc != MSIM_OK) return rc;
+    if (!await_report(b->box, b->reports)) rc = bwait(b);
+    if (rc != MSIM_OK) return rc;
+    const unsigned int f = static_cast<unsigned int>(b->box->word);
     if (f) {
         return bfail(b, MSIM_ERR_STATE, "device-side check failed (fault bits 0x%x%s%s%s)", f,
                      (f & kFaultBinCount) ? ": binned agent count != agent count" : "",
@@ -703,85 +712,37 @@ extern "C" int msim_batch_sync(msim_batch* b) {
 extern "C" int msim_batch_read_state(msim_batch* b, uint32_t scen, float* pos, float* target, float* direction,
                                      uint32_t* road_index, uint32_t* rand_state, uint32_t* neighbour_count) {
     if (!b || scen >= b->n_scen) return bfail(b, MSIM_ERR_INVALID, "bad handle or scenario index");
-    int rc = msim_batch_sync(b);
-    if (rc != MSIM_OK) return rc;
-    const uint32_t off = b->agent_off_h[scen], na = b->agent_off_h[scen + 1] - off;
-    const BBuffers& bb = b->buf[b->cur];
-    std::vector<float2> p(na), t(na), d(na);
-    std::vector<uint32_t> r(na), c(na), pm(na);
-    std::vector<uint4> g(na);
-    auto dn = [&](void* dst, const void* src, size_t bytes) {
-        if (rc == MSIM_OK && bytes) {
-            hipError_t e = hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
-            if (e != hipSuccess) rc = bfail(b, MSIM_ERR_HIP, "readback failed: %s", hipGetErrorString(e));
-        }
-    };
     // a scenario's agents stay inside its slot range through every reorder
-    dn(p.data(), bb.pos + off, sizeof(float2) * na);
-    dn(d.data(), bb.dir + off, sizeof(float2) * na);
-    // sorted state: target and caller index in the slots' records, road and
-    // PRNG state in caller order
+    const uint32_t off = b->agent_off_h[scen], na = b->agent_off_h[scen + 1] - off;
+    if (na == 0) return msim_batch_sync(b);
+    void* to = b->readback.small(StateOut::kWords * sizeof(uint4) * na);
+    const StateOut o = StateOut::at(to ? to : b->read_stage, na);
+    const dim3 g(bblocks(na));
     if (b->sorted) {
-        std::vector<uint4> rc4(na);
-        dn(rc4.data(), b->rec[b->cur] + off, sizeof(uint4) * na);
-        for (uint32_t k = 0; k < na; k++) {
-            std::memcpy(&t[k], &rc4[k], sizeof(float2));  // the record's first 8 bytes: the target
-            pm[k] = rc4[k].w;
-        }
-        std::vector<uint4> cw(2 * static_cast<size_t>(na));
-        dn(cw.data(), b->cold + 2 * static_cast<size_t>(off), sizeof(uint4) * 2 * na);
-        for (uint32_t k = 0; k < na; k++) {
-            r[k] = cw[2 * k].x;
-            g[k] = cw[2 * k + 1];
-        }
+        hipLaunchKernelGGL(k_export_state_rec, g, dim3(kBlock), 0, b->stream, b->agents(b->cur), b->rec[b->cur],
+                           b->cold, off, na, b->road_off_h[scen], o);
     } else {
-        dn(t.data(), bb.tgt + off, sizeof(float2) * na);
-        dn(pm.data(), bb.perm + off, sizeof(uint32_t) * na);
-        dn(r.data(), bb.road + off, sizeof(uint32_t) * na);
-        dn(g.data(), bb.rng + off, sizeof(uint4) * na);
+        hipLaunchKernelGGL(k_export_state, g, dim3(kBlock), 0, b->stream, b->agents(b->cur), off, na,
+                           b->road_off_h[scen], o);
     }
-    dn(c.data(), bb.ncount + off, sizeof(uint32_t) * na);
+    int rc = bcheck(b, "k_export_state");
     if (rc != MSIM_OK) return rc;
-    const uint32_t road_base = b->road_off_h[scen];
-    for (uint32_t k = 0; k < na; k++) {
-        const uint32_t i = pm[k] - off;
-        if (pos) {
-            pos[2 * i] = p[k].x;
-            pos[2 * i + 1] = p[k].y;
-        }
-        if (target) {
-            target[2 * i] = t[k].x;
-            target[2 * i + 1] = t[k].y;
-        }
-        if (direction) {
-            direction[2 * i] = d[k].x;
-            direction[2 * i + 1] = d[k].y;
-        }
-        const uint32_t c_i = b->sorted ? i : k;  // caller-order arrays are indexed by agent
-        if (road_index) road_index[i] = r[c_i] - road_base;
-        if (rand_state) {
-            rand_state[4 * i] = g[c_i].x;
-            rand_state[4 * i + 1] = g[c_i].y;
-            rand_state[4 * i + 2] = g[c_i].z;
-            rand_state[4 * i + 3] = g[c_i].w;
-        }
-        if (neighbour_count) neighbour_count[i] = c[k];
-    }
-    return MSIM_OK;
+    std::vector<ReadPart> parts;
+    if (pos) parts.push_back({pos, o.pos, sizeof(float2) * na});
+    if (target) parts.push_back({target, o.tgt, sizeof(float2) * na});
+    if (direction) parts.push_back({direction, o.dir, sizeof(float2) * na});
+    if (road_index) parts.push_back({road_index, o.road, sizeof(uint32_t) * na});
+    if (rand_state) parts.push_back({rand_state, o.rng, sizeof(uint4) * na});
+    if (neighbour_count) parts.push_back({neighbour_count, o.ncount, sizeof(uint32_t) * na});
+    return bread_parts(b, parts);
 }
 
 extern "C" int msim_batch_read_pairs(msim_batch* b, uint64_t* totals, uint32_t* last) {
     if (!b) return bfail(b, MSIM_ERR_INVALID, "NULL handle");
-    int rc = msim_batch_sync(b);
-    if (rc != MSIM_OK) return rc;
-    if (totals &&
-        hipMemcpy(totals, b->totals, sizeof(uint64_t) * b->n_scen, hipMemcpyDeviceToHost) != hipSuccess) {
-        return bfail(b, MSIM_ERR_HIP, "pair readback failed");
-    }
-    if (last && hipMemcpy(last, b->last, sizeof(uint32_t) * b->n_scen, hipMemcpyDeviceToHost) != hipSuccess) {
-        return bfail(b, MSIM_ERR_HIP, "pair readback failed");
-    }
-    return MSIM_OK;
+    std::vector<ReadPart> parts;
+    if (totals) parts.push_back({totals, b->totals, sizeof(uint64_t) * b->n_scen});
+    if (last) parts.push_back({last, b->last, sizeof(uint32_t) * b->n_scen});
+    return bread_parts(b, parts);
 }
 
 extern "C" int msim_batch_time_ticks(msim_batch* b, uint32_t n_ticks, float* ms_total, float* kernel_ms,
@@ -847,6 +808,7 @@ extern "C" int msim_batch_destroy(msim_batch* b) {
         for (auto& g : row)
             if (g.exec) (void)hipGraphExecDestroy(g.exec);
     for (void* p : b->allocs) (void)hipFree(p);
+    if (b->box) (void)hipHostFree(b->box);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
     return MSIM_OK;

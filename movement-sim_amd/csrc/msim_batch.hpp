@@ -17,6 +17,7 @@
 #include "msim_bin.hpp"
 #include "msim_host.hpp"
 #include "msim_kernels.hpp"
+#include "msim_read.hpp"
 #include "msim_sorted.hpp"
 
 namespace msim {
@@ -464,6 +465,11 @@ struct msim_batch {
     hipEvent_t probe_ev[2] = {nullptr, nullptr};
     std::vector<void*> allocs;
     std::string err;
+    int device = 0;
+    msim::ReadBack readback;
+    uint4* read_stage = nullptr;      // [StateOut::kWords * largest scenario] a scenario's state in caller order
+    msim::Mailbox* box = nullptr;     // pinned fault report (msim_batch_sync)
+    unsigned int reports = 0;
     DiffState* diff = nullptr;
 
     AgentsDev agents(int k) const {
@@ -577,18 +583,24 @@ inline void blaunch_bins(msim_batch* b, const float2* pos, const BatchBin& bb, s
 }
 
 inline int bwait(msim_batch* b) {
-    const auto t0 = std::chrono::steady_clock::now();
-    for (;;) {
-        hipError_t e = hipStreamQuery(b->stream);
-        if (e == hipSuccess) return MSIM_OK;
-        if (e != hipErrorNotReady) return bfail(b, MSIM_ERR_HIP, "stream failed: %s", hipGetErrorString(e));
-        const auto ms =
-            std::chrono::duration_cast<std::chrono::milliseconds>(std::chrono::steady_clock::now() - t0).count();
-        if (ms > static_cast<long long>(b->watchdog_ms)) {
-            return bfail(b, MSIM_ERR_TIMEOUT, "stream did not drain within %u ms", b->watchdog_ms);
-        }
-        std::this_thread::sleep_for(std::chrono::microseconds(ms < 10 ? 20 : 500));
+    const hipError_t e = bounded_wait(b->watchdog_ms, [&] { return hipStreamQuery(b->stream); });
+    if (e == hipErrorNotReady) {
+        return bfail(b, MSIM_ERR_TIMEOUT, "stream did not drain within %u ms", b->watchdog_ms);
     }
+    if (e != hipSuccess) return bfail(b, MSIM_ERR_HIP, "stream failed: %s", hipGetErrorString(e));
+    return MSIM_OK;
+}
+
+// The parts into the caller's memory, after the stream's work and the
+// device-side checks.
+inline int bread_parts(msim_batch* b, const std::vector<ReadPart>& parts) {
+    hipError_t e = hipSuccess;
+    const int rc = b->readback.read(b->device, b->stream, parts, b->watchdog_ms, &e, [&] { return msim_batch_sync(b); });
+    if (rc >= 0) return rc;
+    if (e == hipErrorNotReady) {
+        return bfail(b, MSIM_ERR_TIMEOUT, "readback did not finish within %u ms", b->watchdog_ms);
+    }
+    return bfail(b, MSIM_ERR_HIP, "readback failed: %s", hipGetErrorString(e));
 }
 
 inline GridDev bgrid(const msim_batch* b) {

@@ -1016,6 +1016,42 @@ static __global__ __launch_bounds__(kBlock) void k_pack_entities(AgentsDev a, co
     r[3] = make_uint4(__float_as_uint(d.x), __float_as_uint(d.y), a.road[k], a.init[k]);
 }
 
+// State of n agents in caller order, for the readbacks: one array after the
+// other, each of n entries (the widest first, so that every one is aligned).
+struct StateOut {
+    uint4* rng;
+    float2 *pos, *tgt, *dir;
+    uint32_t *road, *ncount;
+    static constexpr size_t kWords = 3;  // 16-byte words per agent
+    __host__ static StateOut at(void* p, size_t n) {
+        StateOut o;
+        o.rng = static_cast<uint4*>(p);
+        o.pos = reinterpret_cast<float2*>(o.rng + n);
+        o.tgt = o.pos + n;
+        o.dir = o.tgt + n;
+        o.road = reinterpret_cast<uint32_t*>(o.dir + n);
+        o.ncount = o.road + n;
+        return o;
+    }
+};
+
+// Slots [off, off + n) of a, whose agents have the caller indices
+// [off, off + n), into out; road indices relative to road_base.
+static __global__ __launch_bounds__(kBlock) void k_export_state(AgentsDev a, uint32_t off, uint32_t n,
+                                                                uint32_t road_base, StateOut out) {
+    const uint32_t j = blockIdx.x * kBlock + threadIdx.x;
+    if (j >= n) {
+        return;
+    }
+    const uint32_t k = off + j, i = a.perm[k] - off;
+    out.pos[i] = a.pos[k];
+    out.tgt[i] = a.tgt[k];
+    out.dir[i] = a.dir[k];
+    out.road[i] = a.road[k] - road_base;
+    out.rng[i] = a.rng[k];
+    out.ncount[i] = a.ncount[k];
+}
+
 // Per-agent cell export in caller order.
 static __global__ __launch_bounds__(kBlock) void k_export_cells(AgentsDev a, float inv_cell, int2* out) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;

@@ -21,6 +21,7 @@
 #include "msim_bin.hpp"
 #include "msim_host.hpp"
 #include "msim_kernels.hpp"
+#include "msim_read.hpp"
 #include "msim_sorted.hpp"
 
 using namespace msim;
@@ -132,6 +133,10 @@ struct msim_sim {
     uint64_t bytes = 0;
     std::vector<void*> allocs;
     std::string err;
+    ReadBack readback;
+    Counters* ctr_host = nullptr;  // pinned copy of ctr
+    Mailbox* box = nullptr;        // pinned fault report (check_faults)
+    unsigned int reports = 0;
 
     GridDev grid_cur() const {
         GridDev g = grid;
@@ -747,15 +752,11 @@ int enqueue_run_tick(msim_sim* s) {
     return rc;
 }
 
-// Makes the classic per-slot arrays of buf[cur] (target, speed, caller index,
-// road, rng, init, ncount) readable for the readbacks; the sorted state stays
-// in force.
-int publish_sorted(msim_sim* s) {
+// Sorted state: neighbour counts in the current slot order, in buf[cur].
+int settle_ncount(msim_sim* s) {
     if (!s->sorted) return MSIM_OK;
     const Buffers& b = s->buf[s->cur];
     const dim3 g(agent_blocks(s->n));
-    hipLaunchKernelGGL(k_unpack_rec, g, dim3(kBlock), 0, s->stream, s->rec[s->cur], b.tgt,
-                       s->uniform ? nullptr : b.spd, b.perm, s->n);
     if (s->ncount_at == 1 - s->cur) {
         const Buffers& o = s->buf[1 - s->cur];
         hipLaunchKernelGGL(k_scatter_rec<uint32_t>, g, dim3(kBlock), 0, s->stream, s->rec[1 - s->cur], o.ncount,
@@ -763,33 +764,38 @@ int publish_sorted(msim_sim* s) {
         s->ncount_at = -1;
     }
     if (s->ncount_at == -1) {
-        hipLaunchKernelGGL(k_gather_perm<uint32_t>, g, dim3(kBlock), 0, s->stream, b.perm, s->ncount_caller,
+        hipLaunchKernelGGL(k_gather_rec<uint32_t>, g, dim3(kBlock), 0, s->stream, s->rec[s->cur], s->ncount_caller,
                            b.ncount, s->n);
         s->ncount_at = s->cur;
     }
+    return check_launch(s, "neighbour counts");
+}
+
+// Makes the classic per-slot arrays of buf[cur] (target, speed, caller index,
+// road, rng, init, ncount) readable for the readbacks; the sorted state stays
+// in force.
+int publish_sorted(msim_sim* s) {
+    if (!s->sorted) return MSIM_OK;
+    int rc = settle_ncount(s);
+    if (rc != MSIM_OK) return rc;
+    const Buffers& b = s->buf[s->cur];
+    const dim3 g(agent_blocks(s->n));
+    hipLaunchKernelGGL(k_unpack_rec, g, dim3(kBlock), 0, s->stream, s->rec[s->cur], b.tgt,
+                       s->uniform ? nullptr : b.spd, b.perm, s->n);
     hipLaunchKernelGGL(k_cold_publish, g, dim3(kBlock), 0, s->stream, b.perm, s->cold, b.road, b.rng, s->n);
     hipLaunchKernelGGL(k_set_init, g, dim3(kBlock), 0, s->stream, b.init, s->n);
     return check_launch(s, "sorted state readback");
 }
 
 int wait_stream(msim_sim* s) {
-    const auto t0 = std::chrono::steady_clock::now();
-    for (;;) {
-        hipError_t e = hipStreamQuery(s->stream);
-        if (e == hipSuccess) {
-            return MSIM_OK;
-        }
-        if (e != hipErrorNotReady) {
-            return fail(s, MSIM_ERR_HIP, "stream failed: %s", hipGetErrorString(e));
-        }
-        const auto ms = std::chrono::duration_cast<std::chrono::milliseconds>(
-                            std::chrono::steady_clock::now() - t0)
-                            .count();
-        if (ms > static_cast<long long>(s->watchdog_ms)) {
-            return fail(s, MSIM_ERR_TIMEOUT, "stream did not drain within %u ms", s->watchdog_ms);
-        }
-        std::this_thread::sleep_for(std::chrono::microseconds(ms < 10 ? 20 : 500));
+    const hipError_t e = bounded_wait(s->watchdog_ms, [&] { return hipStreamQuery(s->stream); });
+    if (e == hipErrorNotReady) {
+        return fail(s, MSIM_ERR_TIMEOUT, "stream did not drain within %u ms", s->watchdog_ms);
     }
+    if (e != hipSuccess) {
+        return fail(s, MSIM_ERR_HIP, "stream failed: %s", hipGetErrorString(e));
+    }
+    return MSIM_OK;
 }
 
 int after_move(msim_sim* s);
@@ -885,14 +891,6 @@ int single_dispatch(msim_sim* s, uint32_t tick) {
         s->any_collide = true;
     }
     return rc;
-}
-
-template <class T>
-int download(msim_sim* s, std::vector<T>& host, const T* dev, size_t count) {
-    host.resize(count);
-    if (count == 0) return MSIM_OK;
-    MSIM_TRY_HIP(s, hipMemcpyAsync(host.data(), dev, count * sizeof(T), hipMemcpyDeviceToHost, s->stream));
-    return MSIM_OK;
 }
 
 }  // namespace
@@ -1162,6 +1160,16 @@ extern "C" int msim_create(const msim_road* roads, uint32_t n_roads, const uint3
                            reinterpret_cast<const uint4*>(s->ent_stage), s->agents(0), s->color0);
         rc = check_launch(s, "k_unpack_entities");
     }
+    if (rc == MSIM_OK && hipHostMalloc(reinterpret_cast<void**>(&s->ctr_host), 256 + sizeof(Mailbox),
+                                       hipHostMallocDefault) != hipSuccess) {
+        s->ctr_host = nullptr;
+        rc = fail(s, MSIM_ERR_OOM, "hipHostMalloc(%zu) failed", 256 + sizeof(Mailbox));
+    }
+    if (rc == MSIM_OK) {
+        static_assert(sizeof(Counters) <= 256, "counters before the mailbox");
+        s->box = reinterpret_cast<Mailbox*>(reinterpret_cast<char*>(s->ctr_host) + 256);
+        s->box->word = 0;
+    }
     // Initial binning, then renumber agents into bucket order for locality.
     if (rc == MSIM_OK) rc = enqueue_move(s, kBinOnly, false);
     if (rc == MSIM_OK) rc = reorder(s);
@@ -1236,16 +1244,26 @@ extern "C" int msim_run_ticks(msim_sim* s, uint32_t n_ticks) {
     return rc;
 }
 
-int check_faults(msim_sim* s) {
-    Counters c{};
-    MSIM_TRY_HIP(s, hipMemcpyAsync(&c, s->ctr, sizeof(c), hipMemcpyDeviceToHost, s->stream));
-    int rc = wait_stream(s);
+// The fault word as of the stream's last work, which has ended on return.
+int wait_report(msim_sim* s, unsigned int* f) {
+    const unsigned int no = ++s->reports;
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, s->stream, &s->ctr->faults, s->box, no);
+    int rc = check_launch(s, "k_report");
     if (rc != MSIM_OK) return rc;
-    if (c.faults) {
-        return fail(s, MSIM_ERR_STATE, "device-side check failed (fault bits 0x%x%s%s%s)", c.faults,
-                    (c.faults & kFaultBinCount) ? ": binned agent count != agent count" : "",
-                    (c.faults & kFaultLookback) ? ": rebinning look-back timed out" : "",
-                    (c.faults & kFaultNext) ? ": an agent's position left its counted bucket" : "");
+    if (!await_report(s->box, no)) rc = wait_stream(s);
+    *f = static_cast<unsigned int>(s->box->word);
+    return rc;
+}
+
+int check_faults(msim_sim* s) {
+    unsigned int f = 0;
+    int rc = wait_report(s, &f);
+    if (rc != MSIM_OK) return rc;
+    if (f) {
+        return fail(s, MSIM_ERR_STATE, "device-side check failed (fault bits 0x%x%s%s%s)", f,
+                    (f & kFaultBinCount) ? ": binned agent count != agent count" : "",
+                    (f & kFaultLookback) ? ": rebinning look-back timed out" : "",
+                    (f & kFaultNext) ? ": an agent's position left its counted bucket" : "");
     }
     return MSIM_OK;
 }
@@ -1257,25 +1275,21 @@ extern "C" int msim_sync(msim_sim* s) {
 
 namespace {
 
-struct HostState {
-    std::vector<float2> pos, tgt, dir;
-    std::vector<uint32_t> road, init, ncount, perm;
-    std::vector<uint4> rng;
-};
+// The parts into the caller's memory, after the stream's work and the
+// device-side checks.
+template <class Ready>
+int read_parts(msim_sim* s, const std::vector<ReadPart>& parts, Ready&& ready) {
+    hipError_t e = hipSuccess;
+    const int rc = s->readback.read(s->device, s->stream, parts, s->watchdog_ms, &e, ready);
+    if (rc >= 0) return rc;
+    if (e == hipErrorNotReady) {
+        return fail(s, MSIM_ERR_TIMEOUT, "readback did not finish within %u ms", s->watchdog_ms);
+    }
+    return fail(s, MSIM_ERR_HIP, "readback failed: %s", hipGetErrorString(e));
+}
 
-int fetch_state(msim_sim* s, HostState& h, bool need_dir, bool need_rng) {
-    const Buffers& b = s->buf[s->cur];
-    int rc = publish_sorted(s);
-    if (rc == MSIM_OK) rc = download(s, h.pos, b.pos, s->n);
-    if (rc == MSIM_OK) rc = download(s, h.tgt, b.tgt, s->n);
-    if (rc == MSIM_OK && need_dir) rc = download(s, h.dir, b.dir, s->n);
-    if (rc == MSIM_OK) rc = download(s, h.road, b.road, s->n);
-    if (rc == MSIM_OK && need_rng) rc = download(s, h.rng, b.rng, s->n);
-    if (rc == MSIM_OK) rc = download(s, h.init, b.init, s->n);
-    if (rc == MSIM_OK) rc = download(s, h.ncount, b.ncount, s->n);
-    if (rc == MSIM_OK) rc = download(s, h.perm, b.perm, s->n);
-    if (rc == MSIM_OK) rc = check_faults(s);
-    return rc;
+int read_parts(msim_sim* s, const std::vector<ReadPart>& parts) {
+    return read_parts(s, parts, [&] { return check_faults(s); });
 }
 
 }  // namespace
@@ -1289,55 +1303,52 @@ extern "C" int msim_read_entities(msim_sim* s, msim_entity* out, uint32_t first,
     flush_stats(s);
     int rc0 = publish_sorted(s);
     if (rc0 != MSIM_OK) return rc0;
+    void* to = s->readback.small(sizeof(msim_entity) * count);
+    if (!to) to = s->ent_stage;
     hipLaunchKernelGGL(k_pack_entities, dim3(agent_blocks(s->n)), dim3(kBlock), 0, s->stream, s->agents(s->cur),
-                       s->color0, s->any_collide ? 1u : 0u, first, count, reinterpret_cast<uint4*>(s->ent_stage));
+                       s->color0, s->any_collide ? 1u : 0u, first, count, static_cast<uint4*>(to));
     int rc = check_launch(s, "k_pack_entities");
     if (rc != MSIM_OK) return rc;
-    MSIM_TRY_HIP(s, hipMemcpyAsync(out, s->ent_stage, sizeof(msim_entity) * count, hipMemcpyDeviceToHost,
-                                   s->stream));
-    rc = check_faults(s);
-    return rc;
+    return read_parts(s, {{out, to, sizeof(msim_entity) * count}});
 }
 
 extern "C" int msim_read_state(msim_sim* s, float* pos, float* target, float* direction,
                                uint32_t* road_index, uint32_t* rand_state, uint32_t* neighbour_count) {
     if (!s) return fail(s, MSIM_ERR_INVALID, "NULL handle");
-    HostState h;
-    int rc = fetch_state(s, h, direction != nullptr, rand_state != nullptr);
+    const size_t n = s->n;
+    if (n == 0) return msim_sync(s);
+    int rc = settle_ncount(s);
     if (rc != MSIM_OK) return rc;
-    for (uint32_t k = 0; k < s->n; k++) {
-        const uint32_t i = h.perm[k];
-        if (pos) {
-            pos[2 * i] = h.pos[k].x;
-            pos[2 * i + 1] = h.pos[k].y;
-        }
-        if (target) {
-            target[2 * i] = h.tgt[k].x;
-            target[2 * i + 1] = h.tgt[k].y;
-        }
-        if (direction) {
-            direction[2 * i] = h.dir[k].x;
-            direction[2 * i + 1] = h.dir[k].y;
-        }
-        if (road_index) road_index[i] = h.road[k];
-        if (rand_state) {
-            rand_state[4 * i] = h.rng[k].x;
-            rand_state[4 * i + 1] = h.rng[k].y;
-            rand_state[4 * i + 2] = h.rng[k].z;
-            rand_state[4 * i + 3] = h.rng[k].w;
-        }
-        if (neighbour_count) neighbour_count[i] = h.ncount[k];
+    // caller order on the device, in the entity staging buffer (64 bytes per agent)
+    static_assert(StateOut::kWords * sizeof(uint4) <= sizeof(msim_entity), "state fits the staging buffer");
+    void* to = s->readback.small(StateOut::kWords * sizeof(uint4) * n);
+    const StateOut o = StateOut::at(to ? to : s->ent_stage, n);
+    const dim3 g(agent_blocks(s->n));
+    if (s->sorted) {
+        hipLaunchKernelGGL(k_export_state_rec, g, dim3(kBlock), 0, s->stream, s->agents(s->cur), s->rec[s->cur],
+                           s->cold, 0u, s->n, 0u, o);
+    } else {
+        hipLaunchKernelGGL(k_export_state, g, dim3(kBlock), 0, s->stream, s->agents(s->cur), 0u, s->n, 0u, o);
     }
-    return MSIM_OK;
+    rc = check_launch(s, "k_export_state");
+    if (rc != MSIM_OK) return rc;
+    std::vector<ReadPart> parts;
+    if (pos) parts.push_back({pos, o.pos, sizeof(float2) * n});
+    if (target) parts.push_back({target, o.tgt, sizeof(float2) * n});
+    if (direction) parts.push_back({direction, o.dir, sizeof(float2) * n});
+    if (road_index) parts.push_back({road_index, o.road, sizeof(uint32_t) * n});
+    if (rand_state) parts.push_back({rand_state, o.rng, sizeof(uint4) * n});
+    if (neighbour_count) parts.push_back({neighbour_count, o.ncount, sizeof(uint32_t) * n});
+    return read_parts(s, parts);
 }
 
 extern "C" int msim_read_debug(msim_sim* s, uint32_t out[10]) {
     if (!s || !out) return fail(s, MSIM_ERR_INVALID, "NULL argument");
     flush_stats(s);
-    Counters c{};
-    MSIM_TRY_HIP(s, hipMemcpyAsync(&c, s->ctr, sizeof(c), hipMemcpyDeviceToHost, s->stream));
+    MSIM_TRY_HIP(s, hipMemcpyAsync(s->ctr_host, s->ctr, sizeof(Counters), hipMemcpyDeviceToHost, s->stream));
     int rc = wait_stream(s);
     if (rc != MSIM_OK) return rc;
+    const Counters c = *s->ctr_host;
     std::memset(out, 0, sizeof(uint32_t) * 10);
     out[0] = static_cast<uint32_t>(c.inserts);
     out[1] = static_cast<uint32_t>(c.pairs_total);
@@ -1347,13 +1358,15 @@ extern "C" int msim_read_debug(msim_sim* s, uint32_t out[10]) {
 extern "C" int msim_read_pairs(msim_sim* s, uint64_t* total, uint32_t* per_tick, uint32_t n,
                                uint32_t* n_out) {
     if (!s) return fail(s, MSIM_ERR_INVALID, "NULL handle");
-    Counters c{};
     std::vector<uint32_t> hist(s->hist_cap);
-    MSIM_TRY_HIP(s, hipMemcpyAsync(&c, s->ctr, sizeof(c), hipMemcpyDeviceToHost, s->stream));
-    MSIM_TRY_HIP(s, hipMemcpyAsync(hist.data(), s->hist, sizeof(uint32_t) * s->hist_cap,
-                                   hipMemcpyDeviceToHost, s->stream));
-    int rc = wait_stream(s);
+    // the counters come with the history; a device-side fault is msim_sync's to report
+    auto counters = [&]() -> int {
+        MSIM_TRY_HIP(s, hipMemcpyAsync(s->ctr_host, s->ctr, sizeof(Counters), hipMemcpyDeviceToHost, s->stream));
+        return wait_stream(s);
+    };
+    int rc = read_parts(s, {{hist.data(), s->hist, sizeof(uint32_t) * s->hist_cap}}, counters);
     if (rc != MSIM_OK) return rc;
+    const Counters c = *s->ctr_host;
     if (total) *total = c.pairs_total;
     const uint64_t avail = std::min<uint64_t>(c.collides, s->hist_cap);
     const uint32_t k = static_cast<uint32_t>(std::min<uint64_t>(avail, per_tick ? n : 0));
@@ -1388,12 +1401,8 @@ extern "C" int msim_read_cells(msim_sim* s, int32_t* cell_xy) {
     MSIM_TRY_HIP(s, hipMallocAsync(reinterpret_cast<void**>(&d), sizeof(int2) * s->n, s->stream));
     launch_export_cells(s, d);
     int rc = check_launch(s, "k_export_cells");
-    if (rc == MSIM_OK) {
-        hipError_t e = hipMemcpyAsync(cell_xy, d, sizeof(int2) * s->n, hipMemcpyDeviceToHost, s->stream);
-        if (e != hipSuccess) rc = fail(s, MSIM_ERR_HIP, "cell readback: %s", hipGetErrorString(e));
-    }
+    if (rc == MSIM_OK) rc = read_parts(s, {{cell_xy, d, sizeof(int2) * s->n}}, [&] { return wait_stream(s); });
     (void)hipFreeAsync(d, s->stream);
-    if (rc == MSIM_OK) rc = wait_stream(s);
     return rc;
 }
 
@@ -1583,6 +1592,7 @@ extern "C" int msim_destroy(msim_sim* s) {
     if (s->stream) (void)hipStreamSynchronize(s->stream);
     drop_graphs(s);
     for (void* p : s->allocs) (void)hipFree(p);
+    if (s->ctr_host) (void)hipHostFree(s->ctr_host);
     if (s->stream) (void)hipStreamDestroy(s->stream);
     delete s;
     return MSIM_OK;

@@ -1057,14 +1057,14 @@ static __global__ __launch_bounds__(kBlock) void k_cold_publish(const uint32_t* 
     rng[i] = cold[2u * h + 1u];
 }
 
-// dst[i] = src[perm[i]]
+// dst[i] = src[caller index of slot i], the caller index from the slot's record.
 template <class V>
-static __global__ __launch_bounds__(kBlock) void k_gather_perm(const uint32_t* __restrict__ perm,
-                                                               const V* __restrict__ src, V* __restrict__ dst,
-                                                               uint32_t n) {
+static __global__ __launch_bounds__(kBlock) void k_gather_rec(const uint4* __restrict__ rec,
+                                                              const V* __restrict__ src, V* __restrict__ dst,
+                                                              uint32_t n) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i < n) {
-        dst[i] = src[perm[i]];
+        dst[i] = src[rec[i].w];
     }
 }
 
@@ -1089,6 +1089,26 @@ static __global__ __launch_bounds__(kBlock) void k_export_cells_rec(const float2
         const float2 p = pos[i];
         out[rec[i].w] = make_int2(cell_coord(p.x, inv_cell), cell_coord(p.y, inv_cell));
     }
+}
+
+// k_export_state for the sorted state: target and caller index in the
+// records, road and PRNG state in caller order already.
+static __global__ __launch_bounds__(kBlock) void k_export_state_rec(AgentsDev a, const uint4* __restrict__ rec,
+                                                                    const uint4* __restrict__ cold, uint32_t off,
+                                                                    uint32_t n, uint32_t road_base, StateOut out) {
+    const uint32_t j = blockIdx.x * kBlock + threadIdx.x;
+    if (j >= n) {
+        return;
+    }
+    const uint32_t k = off + j;
+    const uint4 r = rec[k];
+    const uint32_t i = r.w - off;
+    out.pos[i] = a.pos[k];
+    out.tgt[i] = make_float2(__uint_as_float(r.x), __uint_as_float(r.y));
+    out.dir[i] = a.dir[k];
+    out.ncount[i] = a.ncount[k];
+    out.road[j] = cold[2u * k].x - road_base;
+    out.rng[j] = cold[2u * k + 1u];
 }
 
 // Records from the classic per-slot arrays (entering the sorted state); spd

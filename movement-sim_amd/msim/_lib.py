@@ -246,19 +246,19 @@ class Simulation:
     # -- readback ----------------------------------------------------------
     def entities(self, first=0, count=None):
         count = self.n - first if count is None else count
-        out = np.zeros(count, ENTITY_DTYPE)
+        out = np.empty(count, ENTITY_DTYPE)
         self._check(self.lib.msim_read_entities(self.h, _ptr(out), first, count))
         return out
 
     def state(self):
         n = self.n
         st = {
-            "pos": np.zeros((n, 2), np.float32),
-            "tgt": np.zeros((n, 2), np.float32),
-            "dir": np.zeros((n, 2), np.float32),
-            "road": np.zeros(n, np.uint32),
-            "rng": np.zeros((n, 4), np.uint32),
-            "ncount": np.zeros(n, np.uint32),
+            "pos": np.empty((n, 2), np.float32),
+            "tgt": np.empty((n, 2), np.float32),
+            "dir": np.empty((n, 2), np.float32),
+            "road": np.empty(n, np.uint32),
+            "rng": np.empty((n, 4), np.uint32),
+            "ncount": np.empty(n, np.uint32),
         }
         self._check(self.lib.msim_read_state(self.h, _ptr(st["pos"]), _ptr(st["tgt"]), _ptr(st["dir"]),
                                              _ptr(st["road"]), _ptr(st["rng"]), _ptr(st["ncount"])))
@@ -277,7 +277,7 @@ class Simulation:
         return int(total[0]), per[: got.value].copy()
 
     def cells(self):
-        out = np.zeros((self.n, 2), np.int32)
+        out = np.empty((self.n, 2), np.int32)
         self._check(self.lib.msim_read_cells(self.h, _ptr(out)))
         return out
 
@@ -399,12 +399,12 @@ class Batch:
         """Scenario s's state in its own agent order and road numbering."""
         n = int(self.agent_off[s + 1] - self.agent_off[s])
         st = {
-            "pos": np.zeros((n, 2), np.float32),
-            "tgt": np.zeros((n, 2), np.float32),
-            "dir": np.zeros((n, 2), np.float32),
-            "road": np.zeros(n, np.uint32),
-            "rng": np.zeros((n, 4), np.uint32),
-            "ncount": np.zeros(n, np.uint32),
+            "pos": np.empty((n, 2), np.float32),
+            "tgt": np.empty((n, 2), np.float32),
+            "dir": np.empty((n, 2), np.float32),
+            "road": np.empty(n, np.uint32),
+            "rng": np.empty((n, 4), np.uint32),
+            "ncount": np.empty(n, np.uint32),
         }
         self._check(self.lib.msim_batch_read_state(self.h, s, _ptr(st["pos"]), _ptr(st["tgt"]), _ptr(st["dir"]),
                                                    _ptr(st["road"]), _ptr(st["rng"]), _ptr(st["ncount"])))
