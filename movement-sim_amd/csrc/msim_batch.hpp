@@ -300,7 +300,7 @@ __device__ __forceinline__ uint32_t bcount_slot(const BatchCollide& c, uint32_t 
 }
 
 // Staged neighbour pass: each wave takes 64 P consecutive slots, P per
-// lane; a wave whose slots all lie in one scenario runs wave_count_in_cells
+// lane; a wave whose slots all lie in one scenario runs wave_visit_cells
 // on that scenario's table, a wave across a scenario boundary walks per slot
 // (workgroup blk of ceil(n / (kBlock P)); stage_all: kStage positions per
 // wave).
@@ -334,9 +334,9 @@ __device__ __forceinline__ void bcollide_block(const BatchCollide& c, uint32_t b
     const bool one = __ballot(later) == 0ull;
     if (one) {
         const uint32_t last = min(64u * P, c.n - w0) - 1u;
-        wave_count_in_cells<P>(me, valid, 0u, 0u, last >> 6, last & 63u, cx, cy, c.start + bs.start_base, bs.lw,
-                               bs.wmask, bs.hmask, c.bpos, c.d2_limit, stage_all + (threadIdx.x >> 6) * kStage,
-                               cnt);
+        wave_visit_cells<P>(valid, 0u, 0u, last >> 6, last & 63u, cx, cy, c.start + bs.start_base, bs.lw, bs.wmask,
+                            bs.hmask, c.bpos, stage_all + (threadIdx.x >> 6) * kStage,
+                            CountVisitor<P>{cnt, me, c.d2_limit});
     }
 #pragma unroll
     for (int p = 0; p < P; p++) {

@@ -30,7 +30,9 @@ using namespace msim;
 
 namespace msim {
 
-enum DiffFlag : uint8_t { kDiffArrived = 1, kDiffNoMove = 2 };
+// kDiffNear (on the segment tape only): the agent had a neighbour in the
+// tick's avoidance.
+enum DiffFlag : uint8_t { kDiffArrived = 1, kDiffNoMove = 2, kDiffNear = 4 };
 
 struct DiffTapeDev {
     float2* pos;     // [n] position before the move
@@ -110,6 +112,17 @@ struct DiffCells {
     float push_allow;  // largest push per axis the rebinning windows were sized for
 };
 
+// The slots of a tick that have neighbours: each group of kNearGroup slots
+// (one wave's width) lists its own, as offsets into the group.
+// The adjoint of the avoidance changes nothing for the others, at the
+// calibration's density four agents in five.
+constexpr uint32_t kNearGroup = 64;
+struct DiffNear {
+    uint8_t* list;   // [n rounded up to whole groups]; nullptr: not recorded
+    uint8_t* count;  // per group
+    uint8_t* flag;   // [n] the tape's flags, agent order
+};
+
 // Calls f(slot) for every other slot within the d2 limit of slot s, over the
 // 3x3 cells of s's scenario table.  The order of the slots inside a bucket
 // follows the rebinning's LDS atomics and is not reproducible: callers sum in
@@ -134,15 +147,26 @@ __device__ __forceinline__ void for_neighbours(const DiffCells& c, uint32_t s, f
     const uint32_t c0 = static_cast<uint32_t>(cx - 1) & wmask;
     const uint32_t c2 = static_cast<uint32_t>(cx + 1) & wmask;
     const bool wrap = c0 > c2;
-#pragma unroll 1
-    for (int r = -1; r <= 1; r++) {
-        const uint32_t rowb = (static_cast<uint32_t>(cy + r) & hmask) << lw;
-        const uint32_t lo = start[rowb + c0];
-        const uint32_t hi = start[rowb + (wrap ? wmask + 1u : c2 + 1u)];
-        for (uint32_t k = lo; k < hi; k++) {
-            if (k != s && in_range(c.bpos[k], me, c.d2_limit)) f(k);
+    uint32_t lo[3], hi[3];
+#pragma unroll
+    for (uint32_t r = 0; r < 3u; r++) {  // the rows' bounds in one round trip
+        const uint32_t rowb = (static_cast<uint32_t>(cy - 1 + static_cast<int32_t>(r)) & hmask) << lw;
+        lo[r] = start[rowb + c0];
+        hi[r] = start[rowb + (wrap ? wmask + 1u : c2 + 1u)];
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < 3u; r++) {
+        for (uint32_t k = lo[r]; k < hi[r]; k += 2u) {  // two candidates in flight
+            const float2 q0 = c.bpos[k];
+            const float2 q1 = c.bpos[min(k + 1u, hi[r] - 1u)];
+            if (k != s && in_range(q0, me, c.d2_limit)) f(k);
+            if (k + 1u < hi[r] && k + 1u != s && in_range(q1, me, c.d2_limit)) f(k + 1u);
         }
-        if (wrap) {
+    }
+    if (wrap) {
+#pragma unroll 1
+        for (int32_t r = -1; r <= 1; r++) {
+            const uint32_t rowb = (static_cast<uint32_t>(cy + r) & hmask) << lw;
             const uint32_t hi2 = start[rowb + c2 + 1u];
             for (uint32_t k = start[rowb]; k < hi2; k++) {
                 if (k != s && in_range(c.bpos[k], me, c.d2_limit)) f(k);
@@ -151,63 +175,211 @@ __device__ __forceinline__ void for_neighbours(const DiffCells& c, uint32_t s, f
     }
 }
 
-// Forward avoidance: pos[agent] = p~ + alpha * A over the tick's binning.
+// Sums the pushes of a slot's neighbours; cnt counts all candidates in range
+// (the slot itself among them).  A candidate whose squared distance is 0 adds
+// exactly nothing (its terms are below half a unit of the sums).  The others
+// wait in a short queue per slot: one lane in five has a neighbour at all, so
+// summed where they are met, nearly every step of the scan would run the
+// costly part for one lane or two.
+template <int P>
+struct PushVisitor {
+    static constexpr uint32_t kQueue = 3;
+    long long ix[P], iy[P];
+    uint32_t cnt[P], waiting[P];
+    float2 queue[P][kQueue];
+    const float2 (&me)[P];
+    float T, inv_r2;
+    double sc;
+    __device__ __forceinline__ PushVisitor(const float2 (&m)[P], const DiffCells& c)
+        : me(m), T(c.d2_limit), inv_r2(c.inv_r2), sc(c.fix_scale) {
+#pragma unroll
+        for (int p = 0; p < P; p++) {
+            ix[p] = 0;
+            iy[p] = 0;
+            cnt[p] = 0u;
+            waiting[p] = 0u;
+#pragma unroll
+            for (uint32_t k = 0; k < kQueue; k++) queue[p][k] = make_float2(0.0f, 0.0f);
+        }
+    }
+    __device__ __forceinline__ void add(int p, float2 q) {
+        const float x = me[p].x - q.x;
+        const float y = me[p].y - q.y;
+        const float w = avoid_w(x * x + y * y, inv_r2);
+        ix[p] += __double2ll_rn(static_cast<double>(w * x) * sc);
+        iy[p] += __double2ll_rn(static_cast<double>(w * y) * sc);
+    }
+    __device__ __forceinline__ float dist2(int p, float2 q) const {  // in_range's
+        const float ddx = q.x - me[p].x;
+        const float ddy = q.y - me[p].y;
+        return opaque(ddx * ddx) + opaque(ddy * ddy);
+    }
+    __device__ __forceinline__ void note(int p, float2 q, float d2) {
+        cnt[p] += d2 < T ? 1u : 0u;
+        if (d2 < T && d2 > 0.0f) {
+            if (waiting[p] == kQueue) {
+                add(p, queue[p][kQueue - 1]);
+                waiting[p]--;
+            }
+#pragma unroll
+            for (uint32_t k = kQueue - 1; k > 0; k--) queue[p][k] = queue[p][k - 1];
+            queue[p][0] = q;
+            waiting[p]++;
+        }
+    }
+    __device__ __forceinline__ void one(int p, float2 q) { note(p, q, dist2(p, q)); }
+    __device__ __forceinline__ void staged(int p, const float2* stage, uint32_t j0, uint32_t j1) {
+        const float2* q = stage + j0;
+        const float2* const pair_end = stage + (j0 + ((j1 - j0) & ~1u));
+        for (; q != pair_end; q += 2) {
+            const float2 q0 = q[0], q1 = q[1];
+            const float d0 = dist2(p, q0), d1 = dist2(p, q1);
+            note(p, q0, d0);
+            note(p, q1, d1);
+        }
+        if ((j1 - j0) & 1u) one(p, *q);
+    }
+    // The sums, when all candidates were seen.
+    __device__ __forceinline__ void finish() {
+#pragma unroll
+        for (int p = 0; p < P; p++) {
+#pragma unroll
+            for (uint32_t k = 0; k < kQueue; k++) {
+                if (waiting[p] > k) add(p, queue[p][k]);
+            }
+        }
+    }
+};
+
+// Forward avoidance: pos[agent] = p~ + alpha * A over the tick's binning, each
+// wave staging the candidates of its 64 P slots as the neighbour pass does.
 // Each binary32 term w x is rounded to a multiple of 1/fix_scale (a power of
 // two with |w x| * fix_scale < 2^40, at most 2^-40 R) and the terms are
 // summed as 64-bit integers, so A does not depend on the order in which the
 // neighbours are visited and two runs with the same parameters are
 // bit-identical.  A push beyond the windows' allowance raises kFaultBinCount
 // (the run then fails instead of rebinning an agent outside its window).
-static __global__ __launch_bounds__(kBlock) void k_davoid(DiffCells c, float alpha, float2* __restrict__ pos,
-                                                   unsigned int* __restrict__ faults) {
-    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
-    if (s >= c.n) {
-        return;
+// Positions without a neighbour stay as the move left them (p + 0 differs
+// from p only for p = -0).  move = 0: only near is recorded.
+// (One slot per lane: with two, 110 registers and half the waves, 800k agents
+// took 41 us against 28; a lane walking its cells in global memory, without
+// staging, 33.)
+template <int P>
+static __global__ __launch_bounds__(kBlock, 4) void k_davoid(DiffCells c, float alpha, uint32_t move,
+                                                             float2* __restrict__ pos, DiffNear near,
+                                                             unsigned int* __restrict__ faults) {
+    __shared__ float2 stage_all[kBlock / 64 * kStage];
+    const uint32_t blk = collide_order(blockIdx.x, gridDim.x);
+    const uint32_t wave = blk * (kBlock / 64) + (threadIdx.x >> 6);
+    const uint32_t w0 = wave * (64u * P);
+    if (w0 >= c.n) {
+        return;  // wave-uniform: no barrier follows
     }
-    const float2 me = c.bpos[s];
-    long long ix = 0, iy = 0;
-    const double sc = c.fix_scale;
-    for_neighbours(c, s, me, [&](uint32_t k) {
-        const float2 q = c.bpos[k];
-        const float x = me.x - q.x;
-        const float y = me.y - q.y;
-        const float w = avoid_w(x * x + y * y, c.inv_r2);
-        ix += __double2ll_rn(static_cast<double>(w * x) * sc);
-        iy += __double2ll_rn(static_cast<double>(w * y) * sc);
-    });
-    const float ax = static_cast<float>(static_cast<double>(ix) / sc);
-    const float ay = static_cast<float>(static_cast<double>(iy) / sc);
-    const float px = alpha * ax, py = alpha * ay;
-    if (!(fabsf(px) <= c.push_allow) || !(fabsf(py) <= c.push_allow)) {
-        atomicOr(faults, kFaultBinCount);
+    const uint32_t lane = __lane_id();
+    const BlockScen bs = c.blk[w0 / kBlock];
+    float2 me[P];
+    bool valid[P];
+    int32_t cx[P], cy[P];
+    bool later = false;  // some valid slot lies past scenario bs.sid
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+        const uint32_t s = w0 + 64u * p + lane;
+        valid[p] = s < c.n;
+        me[p] = valid[p] ? c.bpos[s] : make_float2(0.0f, 0.0f);
+        cx[p] = cell_coord(me[p].x, c.inv_cell);
+        cy[p] = cell_coord(me[p].y, c.inv_cell);
+        later = later || (valid[p] && s >= bs.end);
     }
-    pos[c.bid[s]] = make_float2(me.x + px, me.y + py);
+    PushVisitor<P> v(me, c);
+    if (__ballot(later) == 0ull) {
+        const uint32_t last = min(64u * P, c.n - w0) - 1u;
+        wave_visit_cells<P>(valid, 0u, 0u, last >> 6, last & 63u, cx, cy, c.start + bs.start_base, bs.lw, bs.wmask,
+                            bs.hmask, c.bpos, stage_all + (threadIdx.x >> 6) * kStage, v);
+    } else {  // across a scenario boundary: per slot
+#pragma unroll
+        for (int p = 0; p < P; p++) {
+            const uint32_t s = w0 + 64u * p + lane;
+            if (valid[p]) {
+                for_neighbours(c, s, me[p], [&](uint32_t k) { v.one(p, c.bpos[k]); });
+                v.cnt[p]++;  // its own
+            }
+        }
+    }
+    v.finish();
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+        const uint32_t s = w0 + 64u * p + lane;
+        const bool has = valid[p] && v.cnt[p] > 1u;
+        const bool moves = move && valid[p] && (has || me[p].x == 0.0f || me[p].y == 0.0f);
+        const unsigned long long hm = __ballot(has);
+        if (has || moves) {
+            const uint32_t i = c.bid[s];
+            if (near.list && has) {
+                near.list[w0 + kNearGroup * p + static_cast<uint32_t>(__popcll(hm & ((1ull << lane) - 1ull)))] =
+                    static_cast<uint8_t>(lane);
+                near.flag[i] |= kDiffNear;
+            }
+            if (moves) {
+                const float px = alpha * static_cast<float>(static_cast<double>(v.ix[p]) / v.sc);
+                const float py = alpha * static_cast<float>(static_cast<double>(v.iy[p]) / v.sc);
+                if (!(fabsf(px) <= c.push_allow) || !(fabsf(py) <= c.push_allow)) {
+                    atomicOr(faults, kFaultBinCount);
+                }
+                pos[i] = make_float2(me[p].x + px, me[p].y + py);
+            }
+        }
+        if (near.list && lane == 0 && w0 + kNearGroup * p < c.n) {
+            near.count[wave * P + p] = static_cast<uint8_t>(__popcll(hm));
+        }
+    }
 }
 
+// The alpha derivative is summed into kAlphaSlots words a line apart, one
+// atomic per workgroup (on one word the workgroups' atomics queue up).
+constexpr uint32_t kAlphaSlots = 64, kAlphaStride = 16;
+
 // Avoidance adjoint over the tick's binning, in binary64 from the run's
-// binary32 positions: lam_out = lam + alpha * sum J dl, and the alpha
-// derivative sum lam . A (one atomic per block).
-static __global__ __launch_bounds__(kBlock) void k_davoid_adj(DiffCells c, double alpha,
+// binary32 positions, for the listed slots: lam_out = lam + alpha * sum J dl
+// at their agents, and the alpha derivative sum lam . A.  A workgroup takes
+// GROUPS groups.
+template <uint32_t GROUPS>
+static __global__ __launch_bounds__(kBlock) void k_davoid_adj(DiffCells c, DiffNear near, double alpha,
                                                        const double2* __restrict__ lam,
                                                        double2* __restrict__ lam_out,
                                                        double* __restrict__ galpha) {
     __shared__ double red[kBlock / 64];
-    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
+    const uint32_t blk = collide_order(blockIdx.x, gridDim.x);
+    const uint32_t n_groups = (c.n + kNearGroup - 1u) / kNearGroup, g0 = blk * GROUPS;
+    uint32_t end[GROUPS];
+    uint32_t m = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < GROUPS; k++) {
+        m += g0 + k < n_groups ? near.count[g0 + k] : 0u;
+        end[k] = m;
+    }
     double ga = 0.0;
-    if (s < c.n) {
+    for (uint32_t e = threadIdx.x; e < m; e += kBlock) {
+        uint32_t k = 0, first = 0;
+#pragma unroll
+        for (uint32_t u = 0; u + 1u < GROUPS; u++) {
+            if (e >= end[u]) {
+                k = u + 1u;
+                first = end[u];
+            }
+        }
+        const uint32_t base = (g0 + k) * kNearGroup;
+        const uint32_t s = base + near.list[base + (e - first)];
         const float2 me = c.bpos[s];
         const uint32_t i = c.bid[s];
         const double2 li = lam[i];
         const double inv_r2 = c.inv_r2_d;
         double gx = 0.0, gy = 0.0, ax = 0.0, ay = 0.0;
-        for_neighbours(c, s, me, [&](uint32_t k) {
-            const float2 q = c.bpos[k];
+        auto add = [&](float2 q, double2 lj) {
             const double x = static_cast<double>(me.x) - q.x;
             const double y = static_cast<double>(me.y) - q.y;
             const double h = 1.0 - (x * x + y * y) * inv_r2;
             const double w = h * h * h;
             const double wp = -3.0 * inv_r2 * h * h;  // dw/dq
-            const double2 lj = lam[c.bid[k]];
             const double dlx = li.x - lj.x;
             const double dly = li.y - lj.y;
             const double xd = 2.0 * wp * (x * dlx + y * dly);
@@ -215,9 +387,39 @@ static __global__ __launch_bounds__(kBlock) void k_davoid_adj(DiffCells c, doubl
             gy += w * dly + xd * y;
             ax += w * x;
             ay += w * y;
+        };
+        // neighbours wait in a queue, so that their loads go out together
+        uint32_t queue[4] = {s, s, s, s}, waiting = 0;
+        for_neighbours(c, s, me, [&](uint32_t k) {
+            if (waiting == 4u) {
+                add(c.bpos[queue[3]], lam[c.bid[queue[3]]]);
+                waiting--;
+            }
+            queue[3] = queue[2];
+            queue[2] = queue[1];
+            queue[1] = queue[0];
+            queue[0] = k;
+            waiting++;
         });
+        uint32_t id[4];
+        float2 q[4];
+        double2 lj[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; k++) {
+            id[k] = c.bid[queue[k]];
+            q[k] = c.bpos[queue[k]];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; k++) lj[k] = lam[id[k]];
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; k++) {
+            if (waiting > k) add(q[k], lj[k]);
+        }
         lam_out[i] = make_double2(li.x + alpha * gx, li.y + alpha * gy);
-        ga = li.x * ax + li.y * ay;
+        ga += li.x * ax + li.y * ay;
+    }
+    if (m == 0u) {
+        return;  // workgroup-uniform
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
@@ -229,63 +431,37 @@ static __global__ __launch_bounds__(kBlock) void k_davoid_adj(DiffCells c, doubl
         double t = 0.0;
 #pragma unroll
         for (uint32_t k = 0; k < kBlock / 64; k++) t += red[k];
-        if (t != 0.0) atomicAdd(galpha, t);
+        if (t != 0.0) atomicAdd(&galpha[(blk % kAlphaSlots) * kAlphaStride], t);
     }
 }
 
 // Move adjoint in agent order, binary64 from the run's binary32 values.
+// lam2 holds the avoidance adjoint's result for the agents flagged kDiffNear.
 // An arrival's snap is constant under frozen decisions (λ = 0).  With carry,
 // it is differentiated as if the arrival carried its leftover time onto the
 // next road (nxt_tgt, nxt_road: the decisions after this tick),
 // p' = T + (1 - L/s) s2 u2 with L = |T - p|, u2 the next road's direction and
 // s, s2 the two roads' speeds: λ = (s2/s) u (u2·λ'), ∂/∂θ[road] += v L s2/s²
 // (u2·λ'), ∂/∂θ[next road] += v (1 - L/s)(u2·λ').
+// An agent's terms for the road it is on are summed in acc and added to
+// gtheta where, going back in time, it leaves the road (its arrival, about one
+// tick in 25; k_dflush for the first road): 800k agents, one atomic each per
+// tick, took 40 us.
 template <bool UNIFORM>
 static __global__ __launch_bounds__(kBlock) void k_dmove_adj(uint32_t n, const float* __restrict__ spd,
                                                       float spd_const, const float* __restrict__ theta,
                                                       DiffTapeDev tp, const float2* __restrict__ nxt_tgt,
                                                       const uint32_t* __restrict__ nxt_road, uint32_t carry,
-                                                      const double2* __restrict__ lam_in,
-                                                      double2* __restrict__ lam_out,
-                                                      double* __restrict__ gtheta) {
+                                                      double2* __restrict__ lam, const double2* __restrict__ lam2,
+                                                      double* __restrict__ acc, double* __restrict__ gtheta) {
     const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
     if (k >= n) {
         return;
     }
-    const double2 l = lam_in[k];
     const uint8_t flag = tp.flag[k];
-    if (flag & kDiffArrived) {
-        double2 out = make_double2(0.0, 0.0);
-        if (carry) {
-            const float2 p = tp.pos[k];
-            const float2 T = tp.tgt[k];
-            const float2 T2 = nxt_tgt[k];
-            const double ex = static_cast<double>(T2.x) - T.x;
-            const double ey = static_cast<double>(T2.y) - T.y;
-            const double E = sqrt(ex * ex + ey * ey);
-            const uint32_t r = tp.road[k];
-            const uint32_t r2 = nxt_road[k];
-            const float v = UNIFORM ? spd_const : spd[k];
-            const double s = static_cast<double>(v * theta[r]);
-            const double s2 = static_cast<double>(v * theta[r2]);
-            // a zero speed (theta[r] == 0) carries nothing: the frozen snap
-            if (E > 0.0 && s > 0.0) {
-                const double dx = static_cast<double>(T.x) - p.x;
-                const double dy = static_cast<double>(T.y) - p.y;
-                const double L = sqrt(dx * dx + dy * dy);
-                const double ux = L > 0.0 ? dx / L : 0.0;
-                const double uy = L > 0.0 ? dy / L : 0.0;
-                const double g2 = (ex / E) * l.x + (ey / E) * l.y;
-                out = make_double2(ux * (s2 / s) * g2, uy * (s2 / s) * g2);
-                atomicAdd(&gtheta[r], static_cast<double>(v) * (L * s2 / (s * s)) * g2);
-                atomicAdd(&gtheta[r2], static_cast<double>(v) * (1.0 - L / s) * g2);
-            }
-        }
-        lam_out[k] = out;
-        return;
-    }
+    const double2 l = (flag & kDiffNear) ? lam2[k] : lam[k];
     if (flag & kDiffNoMove) {
-        lam_out[k] = l;
+        if (flag & kDiffNear) lam[k] = l;
         return;
     }
     const float2 p = tp.pos[k];
@@ -296,12 +472,55 @@ static __global__ __launch_bounds__(kBlock) void k_dmove_adj(uint32_t n, const f
     const double dx = static_cast<double>(T.x) - p.x;
     const double dy = static_cast<double>(T.y) - p.y;
     const double len = sqrt(dx * dx + dy * dy);
+    if (flag & kDiffArrived) {
+        double2 out = make_double2(0.0, 0.0);
+        const uint32_t r2 = nxt_road[k];
+        double on_next = acc[k], on_this = 0.0;
+        if (carry) {
+            const float2 T2 = nxt_tgt[k];
+            const double ex = static_cast<double>(T2.x) - T.x;
+            const double ey = static_cast<double>(T2.y) - T.y;
+            const double E = sqrt(ex * ex + ey * ey);
+            const double s2 = static_cast<double>(v * theta[r2]);
+            // a zero speed (theta[r] == 0) carries nothing: the frozen snap
+            if (E > 0.0 && s > 0.0) {
+                const double ux = len > 0.0 ? dx / len : 0.0;
+                const double uy = len > 0.0 ? dy / len : 0.0;
+                const double g2 = (ex / E) * l.x + (ey / E) * l.y;
+                out = make_double2(ux * (s2 / s) * g2, uy * (s2 / s) * g2);
+                on_this = static_cast<double>(v) * (len * s2 / (s * s)) * g2;
+                on_next += static_cast<double>(v) * (1.0 - len / s) * g2;
+            }
+        }
+        lam[k] = out;
+        acc[k] = on_this;
+        if (on_next != 0.0) atomicAdd(&gtheta[r2], on_next);
+        return;
+    }
     const double ux = dx / len;
     const double uy = dy / len;
     const double ul = ux * l.x + uy * l.y;
     const double f = s / len;
-    lam_out[k] = make_double2(l.x - f * (l.x - ux * ul), l.y - f * (l.y - uy * ul));
-    atomicAdd(&gtheta[r], static_cast<double>(v) * ul);
+    lam[k] = make_double2(l.x - f * (l.x - ux * ul), l.y - f * (l.y - uy * ul));
+    acc[k] += static_cast<double>(v) * ul;
+}
+
+// The sums of the roads the agents start on, and the alpha derivative.
+static __global__ __launch_bounds__(kBlock) void k_dflush(uint32_t n, const uint32_t* __restrict__ road,
+                                                   const double* __restrict__ acc, double* __restrict__ gtheta,
+                                                   const double* __restrict__ alpha_slots,
+                                                   double* __restrict__ galpha) {
+    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+    if (k < n && acc[k] != 0.0) atomicAdd(&gtheta[road[k]], acc[k]);
+    if (blockIdx.x == 0 && threadIdx.x < 64u) {
+        static_assert(kAlphaSlots == 64u, "one wave sums the slots");
+        double v = alpha_slots[threadIdx.x * kAlphaStride];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            v += __shfl_xor(v, o, 64);
+        }
+        if (threadIdx.x == 0) *galpha = v;
+    }
 }
 
 // Caller order <-> internal order (perm: internal slot -> caller index).
@@ -312,11 +531,13 @@ static __global__ __launch_bounds__(kBlock) void k_dscatter(uint32_t n, const ui
 }
 
 static __global__ __launch_bounds__(kBlock) void k_dgather(uint32_t n, const uint32_t* __restrict__ perm,
-                                                    const float2* __restrict__ in, double2* __restrict__ out) {
+                                                    const float2* __restrict__ in, double2* __restrict__ out,
+                                                    double* __restrict__ acc) {
     const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
     if (k < n) {
         const float2 v = in[perm[k]];
         out[k] = make_double2(v.x, v.y);
+        acc[k] = 0.0;
     }
 }
 
@@ -354,11 +575,17 @@ struct DiffState {
     uint32_t* tp_start = nullptr;  // [C][start_len]
     uint32_t* tp_bid = nullptr;    // [C][n]
     float2* tp_bpos = nullptr;     // [C][n + 2]
+    uint8_t* tp_near = nullptr;    // [C][near_bytes(n)] lists and counts of the slots with neighbours
+    // the tape holds the last segment of the latest forward run (recorded as
+    // it ran, so that the backward pass need not replay it)
+    bool tape_is_last = false;
     DiffTapeDev sched{};     // [T + 1][n] decisions of the whole run and those after it (keep_schedule)
     double2* lam = nullptr;  // adjoint state, agent order
     double2* lam2 = nullptr;
+    double* acc = nullptr;   // [n] theta terms of the road each agent is on
     double* gtheta = nullptr;
     double* galpha = nullptr;
+    double* alpha_slots = nullptr;  // [kAlphaSlots * kAlphaStride]
     ScenDev* scen = nullptr;  // scenario tables with the differentiable tick's margins
     std::vector<ScenDev> scen_h;
     float smax = 0.0f;  // largest base speed
@@ -371,6 +598,15 @@ namespace {
 
 DiffTapeDev tape_at(const DiffTapeDev& t, size_t n, uint32_t k) {
     return DiffTapeDev{t.pos + n * k, t.tgt + n * k, t.road + n * k, t.flag + n * k};
+}
+
+size_t near_groups(uint32_t n) { return (static_cast<size_t>(n) + kNearGroup - 1) / kNearGroup; }
+size_t near_bytes(uint32_t n) { return near_groups(n) * (kNearGroup + 1); }
+
+// Tape entry k's neighbour lists.
+DiffNear near_at(const msim_batch* b, const DiffState& d, uint32_t k) {
+    uint8_t* p = d.tp_near + near_bytes(b->n) * k;
+    return DiffNear{p, p + near_groups(b->n) * kNearGroup, d.tape.flag + static_cast<size_t>(b->n) * k};
 }
 
 int alloc_snapshot(msim_batch* b, DiffSnapshot& s) {
@@ -483,7 +719,7 @@ DiffCells dcells(msim_batch* b, const uint32_t* start, const float2* bpos, const
 // rebin into (start, bpos, bid), avoidance.
 void dtick(msim_batch* b, DiffState& d, const float* theta, float alpha, uint32_t t, bool replay, DiffTapeDev rec,
            const uint32_t* old_start, const uint32_t* old_bid, uint32_t* new_start, float2* new_bpos,
-           uint32_t* new_bid) {
+           uint32_t* new_bid, DiffNear near = DiffNear{}) {
     const AgentsDev a = b->agents(b->cur);
     const uint32_t no_move = (t == 0 && d.no_move_first) ? 1u : 0u;
     const DiffTapeDev in = replay ? tape_at(d.sched, b->n, t) : DiffTapeDev{};
@@ -506,9 +742,32 @@ void dtick(msim_batch* b, DiffState& d, const float* theta, float alpha, uint32_
         }
     }
     dbins(b, d, old_start, old_bid, new_start, new_bpos, new_bid);
-    if (alpha != 0.0f) {
-        hipLaunchKernelGGL(k_davoid, g, dim3(kBlock), 0, b->stream, dcells(b, new_start, new_bpos, new_bid), alpha,
-                           a.pos, b->faults);
+    if (alpha != 0.0f || near.list) {
+        const DiffCells c = dcells(b, new_start, new_bpos, new_bid);
+        const uint32_t move = alpha != 0.0f ? 1u : 0u;
+        hipLaunchKernelGGL(k_davoid<1>, g, dim3(kBlock), 0, b->stream, c, alpha, move, a.pos, near, b->faults);
+    }
+}
+
+// Tick t as entry j of the segment tape; the segment starts from (start, bid).
+void dtick_taped(msim_batch* b, DiffState& d, uint32_t t, uint32_t j, const uint32_t* start, const uint32_t* bid) {
+    const size_t n = b->n, m = b->start_len;
+    dtick(b, d, d.theta, d.alpha, t, false, tape_at(d.tape, n, j), j ? d.tp_start + m * (j - 1) : start,
+          j ? d.tp_bid + n * (j - 1) : bid, d.tp_start + m * j, d.tp_bpos + (n + 2) * j, d.tp_bid + n * j,
+          near_at(b, d, j));
+}
+
+// 512 slots a workgroup, so that the listed fifth of them fills its lanes
+// better (800k agents: 36 us at 256 slots, 30 at 512); small runs need the
+// workgroups (3k agents: 8.6 us at 256, 9.3 at 512).
+void launch_davoid_adj(msim_batch* b, DiffState& d, const DiffCells& c, const DiffNear& near) {
+    const double alpha = static_cast<double>(d.alpha);
+    if (b->n <= (1u << 17)) {
+        hipLaunchKernelGGL(k_davoid_adj<4>, dim3(bblocks(b->n)), dim3(kBlock), 0, b->stream, c, near, alpha, d.lam,
+                           d.lam2, d.alpha_slots);
+    } else {
+        hipLaunchKernelGGL(k_davoid_adj<8>, dim3((bblocks(b->n) + 1u) / 2u), dim3(kBlock), 0, b->stream, c, near,
+                           alpha, d.lam, d.lam2, d.alpha_slots);
     }
 }
 
@@ -564,6 +823,7 @@ extern "C" int msim_batch_diff_setup(msim_batch* b, uint32_t n_ticks, uint32_t c
     if (rc == MSIM_OK) rc = balloc_n(b, &d->tp_start, static_cast<size_t>(b->start_len) * d->C);
     if (rc == MSIM_OK) rc = balloc_n(b, &d->tp_bid, n * d->C);
     if (rc == MSIM_OK) rc = balloc_n(b, &d->tp_bpos, (n + 2) * d->C);
+    if (rc == MSIM_OK) rc = balloc_n(b, &d->tp_near, near_bytes(b->n) * d->C);
     if (rc == MSIM_OK && d->keep_schedule) {
         rc = balloc_n(b, &d->sched.pos, n * (n_ticks + 1u));
         if (rc == MSIM_OK) rc = balloc_n(b, &d->sched.tgt, n * (n_ticks + 1u));
@@ -574,6 +834,8 @@ extern "C" int msim_batch_diff_setup(msim_batch* b, uint32_t n_ticks, uint32_t c
     if (rc == MSIM_OK) rc = balloc_n(b, &d->lam2, n);
     if (rc == MSIM_OK) rc = balloc_n(b, &d->gtheta, b->n_roads);
     if (rc == MSIM_OK) rc = balloc_n(b, &d->galpha, 1);
+    if (rc == MSIM_OK) rc = balloc_n(b, &d->acc, n);
+    if (rc == MSIM_OK) rc = balloc_n(b, &d->alpha_slots, kAlphaSlots * kAlphaStride);
     if (rc == MSIM_OK) rc = balloc_n(b, &d->scen, b->n_scen);
     if (rc == MSIM_OK) {
         d->scen_h.resize(b->n_scen);
@@ -668,8 +930,16 @@ extern "C" int msim_batch_diff_forward(msim_batch* b, const float* theta, float 
         d.have_forward = false;
     }
     load_initial(b, d.init);
+    d.tape_is_last = false;
+    const uint32_t t_last = (d.n_ck - 1) * d.C;  // the last segment's first tick
     for (uint32_t t = 0; t < d.T && rc == MSIM_OK; t++) {
         if (!replay && t % d.C == 0) save_snapshot(b, d.ck[t / d.C]);
+        if (!replay && !d.keep_schedule && t >= t_last) {
+            // on the tape, binning included (the working one ends here)
+            dtick_taped(b, d, t, t - t_last, b->bstart[b->bcur], b->bbid[b->bcur]);
+            rc = bcheck(b, "differentiable tick");
+            continue;
+        }
         const DiffTapeDev rec = (!replay && d.keep_schedule) ? tape_at(d.sched, b->n, t) : DiffTapeDev{};
         const int nb = 1 - b->bcur;
         dtick(b, d, th, alpha, t, replay != 0, rec, b->bstart[b->bcur], b->bbid[b->bcur], b->bstart[nb],
@@ -699,6 +969,7 @@ extern "C" int msim_batch_diff_forward(msim_batch* b, const float* theta, float 
     if (rc == MSIM_OK) rc = check_diff_faults(b);
     if (rc == MSIM_OK && !replay) {
         d.have_forward = true;
+        d.tape_is_last = !d.keep_schedule;
         d.generation++;
     }
     return rc;
@@ -724,29 +995,24 @@ extern "C" int msim_batch_diff_backward(msim_batch* b, const float* grad_pos, do
     const dim3 g(bblocks(b->n));
     const uint32_t* perm = b->buf[b->cur].perm;
     hipLaunchKernelGGL(k_dgather, g, dim3(kBlock), 0, b->stream, b->n, perm,
-                       reinterpret_cast<const float2*>(grad_pos), d.lam);
+                       reinterpret_cast<const float2*>(grad_pos), d.lam, d.acc);
     (void)hipMemsetAsync(d.gtheta, 0, sizeof(double) * std::max(1u, b->n_roads), b->stream);
-    (void)hipMemsetAsync(d.galpha, 0, sizeof(double), b->stream);
+    (void)hipMemsetAsync(d.alpha_slots, 0, sizeof(double) * kAlphaSlots * kAlphaStride, b->stream);
     for (int seg = static_cast<int>(d.n_ck) - 1; seg >= 0 && rc == MSIM_OK; seg--) {
         const uint32_t t0 = static_cast<uint32_t>(seg) * d.C;
         const uint32_t t1 = std::min(d.T, t0 + d.C);
-        // replay the segment from its checkpoint, recording the tape
-        load_agents(b, d.ck[seg]);
-        for (uint32_t t = t0; t < t1; t++) {
-            const uint32_t j = t - t0;
-            const uint32_t* os = j ? d.tp_start + static_cast<size_t>(b->start_len) * (j - 1) : d.ck[seg].start;
-            const uint32_t* ob = j ? d.tp_bid + n * (j - 1) : d.ck[seg].bid;
-            dtick(b, d, d.theta, d.alpha, t, false, tape_at(d.tape, n, j), os, ob,
-                  d.tp_start + static_cast<size_t>(b->start_len) * j, d.tp_bpos + (n + 2) * j, d.tp_bid + n * j);
+        if (!d.tape_is_last) {  // replay the segment from its checkpoint, recording the tape
+            load_agents(b, d.ck[seg]);
+            for (uint32_t t = t0; t < t1; t++) dtick_taped(b, d, t, t - t0, d.ck[seg].start, d.ck[seg].bid);
         }
+        d.tape_is_last = false;
         rc = bcheck(b, "differentiable tick (segment replay)");
         // reverse through the segment
         for (uint32_t t = t1; t-- > t0 && rc == MSIM_OK;) {
             const uint32_t j = t - t0;
             const DiffCells c = dcells(b, d.tp_start + static_cast<size_t>(b->start_len) * j, d.tp_bpos + (n + 2) * j,
                                        d.tp_bid + n * j);
-            hipLaunchKernelGGL(k_davoid_adj, g, dim3(kBlock), 0, b->stream, c, static_cast<double>(d.alpha), d.lam,
-                               d.lam2, d.galpha);
+            launch_davoid_adj(b, d, c, near_at(b, d, j));
             const AgentsDev a = b->agents(b->cur);
             // the decisions after tick t: the tape's next entry, or after the
             // segment's last tick the agent state its replay ended in
@@ -755,15 +1021,18 @@ extern "C" int msim_batch_diff_backward(msim_batch* b, const float* grad_pos, do
             const uint32_t carry = d.carry ? 1u : 0u;
             if (b->uniform) {
                 hipLaunchKernelGGL(k_dmove_adj<true>, g, dim3(kBlock), 0, b->stream, b->n, a.spd, a.spd_const,
-                                   d.theta, tape_at(d.tape, n, j), nt, nr, carry, d.lam2, d.lam, d.gtheta);
+                                   d.theta, tape_at(d.tape, n, j), nt, nr, carry, d.lam, d.lam2, d.acc, d.gtheta);
             } else {
                 hipLaunchKernelGGL(k_dmove_adj<false>, g, dim3(kBlock), 0, b->stream, b->n, a.spd, a.spd_const,
-                                   d.theta, tape_at(d.tape, n, j), nt, nr, carry, d.lam2, d.lam, d.gtheta);
+                                   d.theta, tape_at(d.tape, n, j), nt, nr, carry, d.lam, d.lam2, d.acc, d.gtheta);
             }
             rc = bcheck(b, "adjoint tick");
         }
     }
     if (rc == MSIM_OK) {
+        // the tape's first entry is the run's first tick now
+        hipLaunchKernelGGL(k_dflush, g, dim3(kBlock), 0, b->stream, b->n, d.tape.road, d.acc, d.gtheta,
+                           d.alpha_slots, d.galpha);
         dcopy(b, grad_theta, d.gtheta, b->n_roads);
         dcopy(b, grad_alpha, d.galpha, 1);
         rc = check_diff_faults(b);

@@ -494,11 +494,24 @@ __device__ __forceinline__ void stage_rows(float2* stage, const float2* __restri
     }
 }
 
-// count_in_cells for a whole wave whose lanes hold P slots each: slot
+// What a wave does with the candidates of its slots: counts those in range.
+template <int P>
+struct CountVisitor {
+    uint32_t (&cnt)[P];
+    const float2 (&me)[P];
+    float T;
+    __device__ __forceinline__ void staged(int p, const float2* stage, uint32_t j0, uint32_t j1) const {
+        cnt[p] += count_staged(stage, j0, j1, me[p], T);
+    }
+    __device__ __forceinline__ void one(int p, float2 q) const { cnt[p] += in_range(q, me[p], T) ? 1u : 0u; }
+};
+
+// The candidates of a whole wave whose lanes hold P slots each: slot
 // w0 + 64 p + lane in element p.  The valid slots (consecutive slots of one
 // bucket table, the first in element first_p of lane first_lane, the last
-// in element last_p of lane last_lane) have nondecreasing buckets; their
-// counts are added to cnt.  Each slot's main
+// in element last_p of lane last_lane) have nondecreasing buckets; v.staged
+// gets their candidates in LDS (a range of the staged positions at a time),
+// v.one those read from global memory.  Each slot's main
 // range in a row, its columns clipped to the row ([col-1, col+1] within
 // [0, wmask]), then starts and ends no earlier than the previous slot's, so
 // the first slot's start and the last slot's end bound the wave's
@@ -509,15 +522,14 @@ __device__ __forceinline__ void stage_rows(float2* stage, const float2* __restri
 // Rows where a slot's neighbour row wraps around the table's top or bottom
 // edge, and the wrapped column of slots in the first or last table column,
 // are read per lane from global memory.  Each slot's own position is
-// included in its count.
-template <int P>
-__device__ __forceinline__ void wave_count_in_cells(const float2 (&me)[P], const bool (&valid)[P], uint32_t first_p,
-                                                    uint32_t first_lane, uint32_t last_p, uint32_t last_lane,
-                                                    const int32_t (&cx)[P],
-                                                    const int32_t (&cy)[P], const uint32_t* __restrict__ start,
-                                                    uint32_t lw, uint32_t wmask, uint32_t hmask,
-                                                    const float2* __restrict__ bpos, float T, float2* stage,
-                                                    uint32_t (&cnt)[P]) {
+// among its candidates.
+template <int P, class V>
+__device__ __forceinline__ void wave_visit_cells(const bool (&valid)[P], uint32_t first_p,
+                                                 uint32_t first_lane, uint32_t last_p, uint32_t last_lane,
+                                                 const int32_t (&cx)[P],
+                                                 const int32_t (&cy)[P], const uint32_t* __restrict__ start,
+                                                 uint32_t lw, uint32_t wmask, uint32_t hmask,
+                                                 const float2* __restrict__ bpos, float2* stage, V&& v) {
     uint32_t col[P], row[P], lo[P][3], hi[P][3];
 #pragma unroll
     for (int p = 0; p < P; p++) {
@@ -569,7 +581,7 @@ __device__ __forceinline__ void wave_count_in_cells(const float2 (&me)[P], const
             for (int p = 0; p < P; p++) {
                 if (valid[p]) {
                     for (uint32_t k = lo[p][r]; k < hi[p][r]; k++) {
-                        cnt[p] += in_range(bpos[k], me[p], T) ? 1u : 0u;
+                        v.one(p, bpos[k]);
                     }
                 }
             }
@@ -600,7 +612,7 @@ __device__ __forceinline__ void wave_count_in_cells(const float2 (&me)[P], const
 #pragma unroll
                 for (int r = 0; r < 3; r++) {
                     if (n[r]) {
-                        cnt[p] += count_staged(stage, off[r] + lo[p][r] - a[r], off[r] + hi[p][r] - a[r], me[p], T);
+                        v.staged(p, stage, off[r] + lo[p][r] - a[r], off[r] + hi[p][r] - a[r]);
                     }
                 }
             }
@@ -613,7 +625,7 @@ __device__ __forceinline__ void wave_count_in_cells(const float2 (&me)[P], const
 #pragma unroll
             for (int r = 0; r < 3; r++) {
                 if (ecol[p] && n[r] && elo[p][r] >= a[r] && ehi[p][r] <= ub[r]) {
-                    cnt[p] += count_staged(stage, off[r] + elo[p][r] - a[r], off[r] + ehi[p][r] - a[r], me[p], T);
+                    v.staged(p, stage, off[r] + elo[p][r] - a[r], off[r] + ehi[p][r] - a[r]);
                     ehi[p][r] = elo[p][r];
                 }
             }
@@ -633,7 +645,7 @@ __device__ __forceinline__ void wave_count_in_cells(const float2 (&me)[P], const
                         const uint32_t k0 = max(lo[p][r], base);
                         const uint32_t k1 = min(hi[p][r], base + m);
                         if (k0 < k1) {
-                            cnt[p] += count_staged(stage, k0 - base, k1 - base, me[p], T);
+                            v.staged(p, stage, k0 - base, k1 - base);
                         }
                     }
                 }
@@ -647,7 +659,7 @@ __device__ __forceinline__ void wave_count_in_cells(const float2 (&me)[P], const
 #pragma unroll
             for (int r = 0; r < 3; r++) {
                 for (uint32_t k = elo[p][r]; k < ehi[p][r]; k++) {
-                    cnt[p] += in_range(bpos[k], me[p], T) ? 1u : 0u;
+                    v.one(p, bpos[k]);
                 }
             }
         }
@@ -680,8 +692,8 @@ __device__ __forceinline__ void collide_block(const AgentsDev& a, const GridDev&
     }
     if (w0 < a.n) {
         const uint32_t last = min(64u * P, a.n - w0) - 1u;
-        wave_count_in_cells<P>(me, valid, 0u, 0u, last >> 6, last & 63u, cx, cy, g.start, g.lw, g.wmask, g.hmask,
-                               bpos, T, stage_all + (threadIdx.x >> 6) * kStage, cnt);
+        wave_visit_cells<P>(valid, 0u, 0u, last >> 6, last & 63u, cx, cy, g.start, g.lw, g.wmask, g.hmask, bpos,
+                            stage_all + (threadIdx.x >> 6) * kStage, CountVisitor<P>{cnt, me, T});
     }
     uint32_t tot = 0;
 #pragma unroll

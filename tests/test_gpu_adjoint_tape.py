@@ -1,0 +1,73 @@
+"""The segment tape the forward run leaves for the backward pass, the lists of
+slots with neighbours, and the per-agent theta sums: gradients from the tape as
+recorded, from a replay of every segment, and from runs that keep their
+schedule agree; small, ragged and crowded agent sets, with and without
+avoidance, against the binary64 host adjoint's tolerance."""
+import numpy as np
+import pytest
+import torch
+
+import msim
+from msim import scenarios as S
+from msim.adjoint import DiffRun
+
+pytestmark = pytest.mark.gpu
+
+
+def _scenarios(sizes, nodes=64, seed=21):
+    out = []
+    for k, n in enumerate(sizes):
+        sc = S.adjoint_config(1, agents=max(n, 1), nodes=nodes, seed=seed + k)[0]
+        sc.entities, sc.speed = sc.entities[:n], sc.speed[:n]
+        out.append(sc)
+    return out
+
+
+def _gradients(run, theta, alpha, g, times=1, between=None):
+    t = theta.clone().requires_grad_(True)
+    a = alpha.clone().requires_grad_(True)
+    pos = run(t, a)
+    if between is not None:
+        between(run, theta)
+    out = []
+    for k in range(times):
+        gt, ga = torch.autograd.grad(pos, (t, a), g, retain_graph=k + 1 < times)
+        out.append((gt.double().cpu().numpy(), float(ga)))
+    return pos.detach().cpu().numpy(), out
+
+
+# sums of the same binary64 terms in another order, rounded to binary32
+def _close(x, y):
+    scale = np.abs(x[0]).max()
+    np.testing.assert_allclose(x[0], y[0], rtol=0, atol=2.0 ** -22 * scale)
+    assert abs(x[1] - y[1]) <= 2.0 ** -22 * max(abs(x[1]), abs(y[1])) + 1e-12 * scale
+
+
+@pytest.mark.parametrize("sizes", [(1,), (63, 0, 65), (256, 129), (1500, 900)])
+@pytest.mark.parametrize("ticks,every", [(7, 7), (7, 50), (23, 10), (20, 10), (9, 1)])
+@pytest.mark.parametrize("alpha", [0.0, 0.03])
+@pytest.mark.parametrize("arrivals", ["frozen", "carry"])
+def test_taped_and_replayed_gradients_agree(sizes, ticks, every, alpha, arrivals):
+    scs = _scenarios(sizes)
+    rng = torch.Generator().manual_seed(3)
+    n_roads = sum(sc.roads.shape[0] for sc in scs)
+    theta = torch.exp(0.2 * torch.randn(n_roads, generator=rng)).cuda()
+    al = torch.tensor(alpha).cuda()
+    n = sum(sizes)
+    g = torch.randn(n, 2, generator=rng).cuda()
+    b = msim.Batch(scs)
+    run = DiffRun(b, ticks, checkpoint_every=every, arrival_gradient=arrivals)
+    pos, (taped, replayed) = _gradients(run, theta, al, g, times=2)
+    b2 = msim.Batch(scs)
+    kept = DiffRun(b2, ticks, checkpoint_every=every, keep_schedule=True, arrival_gradient=arrivals)
+    # a replay between the runs leaves the working state elsewhere
+    pos2, (schedule,) = _gradients(kept, theta, al, g, between=lambda r, th: r.replay(th * 1.01, alpha))
+    np.testing.assert_array_equal(pos.view(np.uint32), pos2.view(np.uint32))
+    _close(taped, replayed)
+    _close(taped, schedule)
+    assert np.isfinite(taped[0]).all() and np.abs(taped[0]).max() > 0.0
+    pos3, (again,) = _gradients(run, theta, al, g)
+    np.testing.assert_array_equal(pos.view(np.uint32), pos3.view(np.uint32))
+    _close(taped, again)
+    b.close()
+    b2.close()
