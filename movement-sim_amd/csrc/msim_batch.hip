@@ -25,9 +25,11 @@ namespace {
 
 template <bool U, bool W>
 void badvance(msim_batch* b) {
-    const dim3 nb(std::max(1u, (b->n + kAdv * kBlock - 1) / (kAdv * kBlock)));
-    hipLaunchKernelGGL((k_advance4<U, W>), nb, dim3(kBlock), 0, b->stream, b->agents(b->cur), b->inv_cell,
-                       b->part_stats, b->roads, b->conns);
+    const uint32_t extra = b->finish_pending ? bfinish_blocks(b, kBlock) : 0u;
+    b->finish_pending = false;
+    const dim3 nb(std::max(1u, (b->n + kAdv * kBlock - 1) / (kAdv * kBlock)) + extra);
+    hipLaunchKernelGGL((k_advance4<U, W, BatchFinish>), nb, dim3(kBlock), 0, b->stream, b->agents(b->cur),
+                       b->inv_cell, b->part_stats, b->roads, b->conns, extra, bfinish_args(b));
 }
 
 constexpr uint32_t kBSortedThreads = 512;
@@ -51,8 +53,7 @@ void blaunch_sorted(msim_batch* b, const SortedMove& mv, const BatchBin& bb, boo
                            b->seg_cnt[b->cur], b->seg_group[b->cur], b->seg_start, b->n_seg, b->n, b->faults);
         bprobe_post(b);
     }
-    constexpr uint32_t waves = kBSortedThreads / 64;
-    const uint32_t extra = finish ? ((b->n_scen + waves - 1) / waves + kXcds - 1) / kXcds * kXcds : 0u;
+    const uint32_t extra = finish ? bfinish_blocks(b, kBSortedThreads) : 0u;
     bprobe_pre(b);
     hipLaunchKernelGGL((k_bmove_sorted<U, kBSortedThreads, UN, W>), dim3(b->n_seg + extra), dim3(kBSortedThreads),
                        bsorted_lds_bytes(b->max_seg_log), b->stream, mv, bb, bfinish_args(b));
@@ -193,7 +194,7 @@ int btick(msim_batch* b, bool last, bool allow_fused = true) {
         rc = benqueue_tick_sorted(b, last, allow_fused && !last && b->collide_mode == 0);
     } else {
         rc = benqueue_move(b, last);
-        if (rc == MSIM_OK) rc = benqueue_collide(b);
+        if (rc == MSIM_OK) rc = benqueue_collide(b, last || !allow_fused);
     }
     b->tick += 2;
     b->since_reorder++;

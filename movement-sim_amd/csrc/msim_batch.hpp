@@ -113,32 +113,37 @@ static __global__ __launch_bounds__(T, 8) void k_bbin_fused(const float2* __rest
     }
 }
 
-// One wave: fold scenario sidx's slots into its pair totals.
+// Pair totals of a collision dispatch, a wave per scenario.
 struct BatchFinish {
     unsigned long long* part;    // [n_scen][kScenSlots * kScenSlotStride]
     unsigned long long* totals;  // [n_scen]
     uint32_t* last;              // [n_scen]
     uint32_t n_scen;
-};
-
-__device__ __forceinline__ void bfinish_scenario(const BatchFinish& f, uint32_t sidx) {
-    unsigned long long v = 0;
-    const uint32_t lane = __lane_id();
-    if (lane < kScenSlots) {
-        unsigned long long* p = &f.part[(static_cast<size_t>(sidx) * kScenSlots + lane) * kScenSlotStride];
-        v = *p;
-        *p = 0ull;
-    }
+    // One wave: fold scenario sidx's slots into its totals.
+    __device__ __forceinline__ void scenario(uint32_t sidx) const {
+        unsigned long long v = 0;
+        const uint32_t lane = __lane_id();
+        if (lane < kScenSlots) {
+            unsigned long long* p = &part[(static_cast<size_t>(sidx) * kScenSlots + lane) * kScenSlotStride];
+            v = *p;
+            *p = 0ull;
+        }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        v += __shfl_xor(v, o, 64);
+        for (int o = 32; o > 0; o >>= 1) {
+            v += __shfl_xor(v, o, 64);
+        }
+        if (lane == 0) {
+            const unsigned long long pairs = v / 2;
+            totals[sidx] += pairs;
+            last[sidx] = static_cast<uint32_t>(pairs);
+        }
     }
-    if (lane == 0) {
-        const unsigned long long pairs = v / 2;
-        f.totals[sidx] += pairs;
-        f.last[sidx] = static_cast<uint32_t>(pairs);
+    // Extra workgroup e of a move launch (as TickFinish).
+    __device__ __forceinline__ void run(uint32_t e) const {
+        const uint32_t sidx = e * (blockDim.x >> 6) + (threadIdx.x >> 6);
+        if (sidx < n_scen) scenario(sidx);
     }
-}
+};
 
 // Sorted move of every scenario's table (see msim_sorted.hpp; the segments of
 // all scenarios are numbered in order, so a scenario's first segment starts at
@@ -152,9 +157,8 @@ static __global__ __launch_bounds__(T) void k_bmove_sorted(SortedMove mv, BatchB
     __shared__ uint32_t nh[2 * kNextReach + 1];
     __shared__ uint32_t sh[1 + T / 64];
     const uint32_t extra = gridDim.x - b.n_seg;
-    if (blockIdx.x < extra) {  // the previous tick's pair totals, beside the move: a wave per scenario
-        const uint32_t sidx = blockIdx.x * (T / 64) + (threadIdx.x >> 6);
-        if (sidx < fin.n_scen) bfinish_scenario(fin, sidx);
+    if (blockIdx.x < extra) {  // the previous tick's pair totals, beside the move
+        fin.run(blockIdx.x);
         return;
     }
     const uint32_t g = seg_order(blockIdx.x - extra, b.n_seg);
@@ -381,7 +385,7 @@ static __global__ __launch_bounds__(kBlock, 6) void k_broute_collide(SortedMove 
 }
 
 // One wave per scenario: fold the slots into the scenario's pair totals.
-static __global__ __launch_bounds__(64) void k_bfinish(BatchFinish f) { bfinish_scenario(f, blockIdx.x); }
+static __global__ __launch_bounds__(64) void k_bfinish(BatchFinish f) { f.scenario(blockIdx.x); }
 
 }  // namespace msim
 
@@ -632,7 +636,14 @@ inline BatchCollide bcollide_args(const msim_batch* b) {
     return c;
 }
 
-inline int benqueue_collide(msim_batch* b) {
+// Extra workgroups of `threads` that BatchFinish takes in front of a move.
+inline uint32_t bfinish_blocks(const msim_batch* b, uint32_t threads) {
+    const uint32_t waves = threads / 64u;
+    return ((b->n_scen + waves - 1) / waves + kXcds - 1) / kXcds * kXcds;
+}
+
+// finish = false: the pair totals are left to the next move.
+inline int benqueue_collide(msim_batch* b, bool finish = true) {
     const BatchCollide c = bcollide_args(b);
     bprobe_pre(b);
     if (b->collide_mode == 1) {
@@ -645,6 +656,8 @@ inline int benqueue_collide(msim_batch* b) {
                            b->stream, c);
     }
     bprobe_post(b);
+    b->finish_pending = !finish;
+    if (!finish) return bcheck(b, "batched collision dispatch");
     bprobe_pre(b);
     hipLaunchKernelGGL(k_bfinish, dim3(b->n_scen), dim3(64), 0, b->stream, bfinish_args(b));
     bprobe_post(b);

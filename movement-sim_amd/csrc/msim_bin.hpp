@@ -46,12 +46,17 @@ template <bool UNIFORM, bool WRITE_DIR, bool ATOMIC_BIN, bool ROUTE_INLINE>
 static __global__ __launch_bounds__(kBlock) void k_advance(AgentsDev a, GridDev g, QueueDev q,
                                                     unsigned long long* __restrict__ part_stats,
                                                     const msim_road* __restrict__ roads,
-                                                    const uint32_t* __restrict__ conns) {
+                                                    const uint32_t* __restrict__ conns, uint32_t n_extra,
+                                                    TickFinish fin) {
     __shared__ uint32_t lds[2 * (kBlock / 64)];
     __shared__ uint32_t sh_base;
-    const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+    if (blockIdx.x < n_extra) {  // the previous tick's statistics
+        fin.run(blockIdx.x);
+        return;
+    }
+    const uint32_t blk = xcd_block(blockIdx.x - n_extra, gridDim.x - n_extra);
     const uint32_t i = blk * kBlock + threadIdx.x;
-    if (blockIdx.x == 0 && threadIdx.x < kQueues) {
+    if (blockIdx.x == n_extra && threadIdx.x < kQueues) {
         q.count_next[threadIdx.x * kQueueStride] = 0u;
     }
     int inserted = 0;
@@ -141,15 +146,21 @@ static __global__ __launch_bounds__(kBlock) void k_advance(AgentsDev a, GridDev 
 // computed on but never routed, counted or read back.
 constexpr uint32_t kAdv = 4;
 
-template <bool UNIFORM, bool WRITE_DIR>
+// The first n_extra workgroups run fin (the previous tick's statistics).
+template <bool UNIFORM, bool WRITE_DIR, class FINISH>
 static __global__ __launch_bounds__(kBlock) void k_advance4(AgentsDev a, float inv_cell,
                                                      unsigned long long* __restrict__ part_stats,
                                                      const msim_road* __restrict__ roads,
-                                                     const uint32_t* __restrict__ conns) {
+                                                     const uint32_t* __restrict__ conns, uint32_t n_extra,
+                                                     FINISH fin) {
     __shared__ uint32_t arr_id[kBlock / 64][64 * kAdv];
     __shared__ float2 arr_dir[WRITE_DIR ? kBlock / 64 : 1][WRITE_DIR ? 64 * kAdv : 1];
     __shared__ uint32_t lds[2 * (kBlock / 64)];
-    const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+    if (blockIdx.x < n_extra) {
+        fin.run(blockIdx.x);
+        return;
+    }
+    const uint32_t blk = xcd_block(blockIdx.x - n_extra, gridDim.x - n_extra);
     const uint32_t t = blk * kBlock + threadIdx.x;
     const uint32_t w = threadIdx.x >> 6;
     const uint32_t i0 = t * kAdv;

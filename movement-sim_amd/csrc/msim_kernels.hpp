@@ -355,6 +355,46 @@ static __global__ __launch_bounds__(kBlock) void k_scan_down(uint32_t* __restric
     }
 }
 
+// The three scan launches' work for a table of at most kScanOne buckets: one
+// workgroup, each thread a run of m / T buckets (m a multiple of 4 T).  Each
+// launch of the chain takes 2 to 3 us however small the table; one CU scans
+// 2^14 buckets in less than two of them.
+constexpr uint32_t kScanOne = 1u << 15;
+template <uint32_t T>
+static __global__ __launch_bounds__(T) void k_scan_one(uint32_t* __restrict__ cnt, uint32_t* __restrict__ start,
+                                                       uint32_t m) {
+    constexpr uint32_t kMax = kScanOne / (4u * T);
+    __shared__ uint32_t lds[T / 64];
+    const uint32_t per = m / (4u * T);  // 16-byte words per thread
+    uint4* c4 = reinterpret_cast<uint4*>(cnt) + static_cast<size_t>(threadIdx.x) * per;
+    uint4 v[kMax];
+    uint32_t sum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kMax; k++) {
+        v[k] = k < per ? c4[k] : make_uint4(0u, 0u, 0u, 0u);
+        sum += v[k].x + v[k].y + v[k].z + v[k].w;
+    }
+    uint32_t total = 0;
+    uint32_t off = block_excl_scan<T>(sum, lds, total);
+    uint4* s4 = reinterpret_cast<uint4*>(start) + static_cast<size_t>(threadIdx.x) * per;
+#pragma unroll
+    for (uint32_t k = 0; k < kMax; k++) {
+        uint4 o;
+        o.x = off;
+        o.y = o.x + v[k].x;
+        o.z = o.y + v[k].y;
+        o.w = o.z + v[k].z;
+        off = o.w + v[k].w;
+        if (k < per) {
+            s4[k] = o;
+            c4[k] = make_uint4(0u, 0u, 0u, 0u);
+        }
+    }
+    if (threadIdx.x == 0) {
+        start[m] = total;
+    }
+}
+
 static __global__ __launch_bounds__(kBlock) void k_scatter(AgentsDev a, GridDev g) {
     const uint32_t i = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
     if (i >= a.n) {
@@ -863,6 +903,24 @@ static __global__ __launch_bounds__(64) void k_collide_finish(unsigned long long
                                                        uint32_t fold_stats) {
     finish_dispatch<SLOW>(part_pairs, ctr, hist, hist_mask, part_stats, fold_stats);
 }
+
+// Statistics of the previous tick's collision dispatch (k_collide_finish's
+// work), done inside a run by extra workgroups in front of the next move's:
+// a launch of its own for one wave took 4 to 4.5 us of ticks of 24 (10k
+// agents) to 45 us (1M).
+struct TickFinish {
+    unsigned long long* part_pairs;
+    Counters* ctr;
+    uint32_t* hist;
+    uint32_t hist_mask;
+    unsigned long long* part_stats;  // the finished tick's half
+    // Extra workgroup e (each has at least 64 threads).
+    __device__ __forceinline__ void run(uint32_t e) const {
+        if (e == 0u && threadIdx.x < 64u) {
+            finish_dispatch<false>(part_pairs, ctr, hist, hist_mask, part_stats, 1u);
+        }
+    }
+};
 
 // ---- spatial renumbering -------------------------------------------------
 

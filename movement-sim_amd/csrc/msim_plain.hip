@@ -248,18 +248,18 @@ void launch_advance_mode(msim_sim* s, bool write_dir) {
     if (s->uniform) {
         if (write_dir) {
             hipLaunchKernelGGL((k_advance_bin<MODE, true, true>), g, dim3(kBlock), 0, s->stream, a,
-                               s->grid_cur(), s->roads, s->conns, s->part_stats);
+                               s->grid_cur(), s->roads, s->conns, stats_buf(s));
         } else {
             hipLaunchKernelGGL((k_advance_bin<MODE, true, false>), g, dim3(kBlock), 0, s->stream, a,
-                               s->grid_cur(), s->roads, s->conns, s->part_stats);
+                               s->grid_cur(), s->roads, s->conns, stats_buf(s));
         }
     } else {
         if (write_dir) {
             hipLaunchKernelGGL((k_advance_bin<MODE, false, true>), g, dim3(kBlock), 0, s->stream, a,
-                               s->grid_cur(), s->roads, s->conns, s->part_stats);
+                               s->grid_cur(), s->roads, s->conns, stats_buf(s));
         } else {
             hipLaunchKernelGGL((k_advance_bin<MODE, false, false>), g, dim3(kBlock), 0, s->stream, a,
-                               s->grid_cur(), s->roads, s->conns, s->part_stats);
+                               s->grid_cur(), s->roads, s->conns, stats_buf(s));
         }
     }
 }
@@ -297,30 +297,36 @@ void launch_bins(msim_sim* s, const float2* pos, const BinDev& b, size_t lds) {
 // the bucket table rebuild (segment-owned into the other binning buffer, or
 // atomic counting + scan + scatter into the current one).  ev (optional)
 // receives an event after each launch.
+// finish (nullable): the previous tick's statistics, folded beside the
+// advance by the launch's first workgroups.
 template <bool U, bool W, bool RI>
-void launch_advance_ri(msim_sim* s, const QueueDev& q) {
+void launch_advance_ri(msim_sim* s, const QueueDev& q, const TickFinish* finish) {
     const AgentsDev a = s->agents(s->cur);
     const GridDev g = s->grid_cur();
-    const dim3 nb(agent_blocks(s->n));
+    const uint32_t extra = finish ? kXcds : 0u;
+    const dim3 nb(agent_blocks(s->n) + extra);
+    const TickFinish fin = finish ? *finish : TickFinish{};
     if (s->binning == 1) {
-        hipLaunchKernelGGL((k_advance<U, W, true, RI>), nb, dim3(kBlock), 0, s->stream, a, g, q, s->part_stats,
-                           s->roads, s->conns);
+        hipLaunchKernelGGL((k_advance<U, W, true, RI>), nb, dim3(kBlock), 0, s->stream, a, g, q, stats_buf(s),
+                           s->roads, s->conns, extra, fin);
     } else {
-        hipLaunchKernelGGL((k_advance<U, W, false, RI>), nb, dim3(kBlock), 0, s->stream, a, g, q,
-                           s->part_stats, s->roads, s->conns);
+        hipLaunchKernelGGL((k_advance<U, W, false, RI>), nb, dim3(kBlock), 0, s->stream, a, g, q, stats_buf(s),
+                           s->roads, s->conns, extra, fin);
     }
 }
 
 template <bool U, bool W>
-void launch_advance_route(msim_sim* s, const QueueDev& q) {
+void launch_advance_route(msim_sim* s, const QueueDev& q, const TickFinish* finish) {
     if (s->route_inline && s->binning != 1) {
-        const dim3 nb(std::max(1u, (s->n + kAdv * kBlock - 1) / (kAdv * kBlock)));
-        hipLaunchKernelGGL((k_advance4<U, W>), nb, dim3(kBlock), 0, s->stream, s->agents(s->cur),
-                           s->grid.inv_cell, s->part_stats, s->roads, s->conns);
+        const uint32_t extra = finish ? kXcds : 0u;
+        const dim3 nb(std::max(1u, (s->n + kAdv * kBlock - 1) / (kAdv * kBlock)) + extra);
+        hipLaunchKernelGGL((k_advance4<U, W, TickFinish>), nb, dim3(kBlock), 0, s->stream, s->agents(s->cur),
+                           s->grid.inv_cell, stats_buf(s), s->roads, s->conns, extra,
+                           finish ? *finish : TickFinish{});
     } else if (s->route_inline) {
-        launch_advance_ri<U, W, true>(s, q);
+        launch_advance_ri<U, W, true>(s, q, finish);
     } else {
-        launch_advance_ri<U, W, false>(s, q);
+        launch_advance_ri<U, W, false>(s, q, finish);
     }
 }
 
@@ -330,17 +336,27 @@ void launch_route(msim_sim* s, const QueueDev& q) {
                        s->agents(s->cur), q, s->roads, s->conns);
 }
 
-int enqueue_move_fast(msim_sim* s, bool write_dir, hipEvent_t* ev) {
+TickFinish finish_args(const msim_sim* s) {
+    return TickFinish{s->part_pairs, s->ctr, s->hist, s->hist_cap - 1, stats_buf(s)};
+}
+
+// in_run: neither the first nor the last launches of a run of ticks; its
+// scans of small tables take one launch.
+int enqueue_move_fast(msim_sim* s, bool write_dir, hipEvent_t* ev, bool in_run) {
     const uint32_t qw = kQueues * kQueueStride;
     QueueDev q{s->q_items, s->q_count + s->qpar * qw, s->q_count + (1 - s->qpar) * qw, s->q_cap};
+    const TickFinish finish = finish_args(s);  // the previous tick's half of the statistics
+    const TickFinish* pf = s->finish_pending ? &finish : nullptr;
+    s->finish_pending = false;
+    s->stats_par ^= 1;  // this tick's
     s->launch_no = 0;
     probe_pre(s);
     if (s->uniform) {
-        if (write_dir) launch_advance_route<true, true>(s, q);
-        else launch_advance_route<true, false>(s, q);
+        if (write_dir) launch_advance_route<true, true>(s, q, pf);
+        else launch_advance_route<true, false>(s, q, pf);
     } else {
-        if (write_dir) launch_advance_route<false, true>(s, q);
-        else launch_advance_route<false, false>(s, q);
+        if (write_dir) launch_advance_route<false, true>(s, q, pf);
+        else launch_advance_route<false, false>(s, q, pf);
     }
     probe_post(s);
     if (!s->route_inline) {
@@ -390,16 +406,20 @@ int enqueue_move_fast(msim_sim* s, bool write_dir, hipEvent_t* ev) {
     } else {
         const GridDev g = s->grid_cur();
         const uint32_t n_part = g.m / kScanTile;
-        probe_pre(s);
-        hipLaunchKernelGGL(k_scan_reduce, dim3(n_part), dim3(kBlock), 0, s->stream, g.cnt, g.part);
-        probe_post(s);
-        probe_pre(s);
-        hipLaunchKernelGGL(k_scan_partials, dim3(1), dim3(kPartialsThreads), 0, s->stream, g.part, n_part,
-                           g.start + g.m);
-        probe_post(s);
-        probe_pre(s);
-        hipLaunchKernelGGL(k_scan_down, dim3(n_part), dim3(kBlock), 0, s->stream, g.cnt, g.part, g.start);
-        probe_post(s);
+        if (in_run && g.m <= kScanOne) {
+            hipLaunchKernelGGL(k_scan_one<1024>, dim3(1), dim3(1024), 0, s->stream, g.cnt, g.start, g.m);
+        } else {
+            probe_pre(s);
+            hipLaunchKernelGGL(k_scan_reduce, dim3(n_part), dim3(kBlock), 0, s->stream, g.cnt, g.part);
+            probe_post(s);
+            probe_pre(s);
+            hipLaunchKernelGGL(k_scan_partials, dim3(1), dim3(kPartialsThreads), 0, s->stream, g.part, n_part,
+                               g.start + g.m);
+            probe_post(s);
+            probe_pre(s);
+            hipLaunchKernelGGL(k_scan_down, dim3(n_part), dim3(kBlock), 0, s->stream, g.cnt, g.part, g.start);
+            probe_post(s);
+        }
         probe_pre(s);
         hipLaunchKernelGGL(k_scatter, dim3(agent_blocks(s->n)), dim3(kBlock), 0, s->stream, s->agents(s->cur),
                            g);
@@ -430,7 +450,7 @@ int enqueue_move(msim_sim* s, int mode, bool write_dir, hipEvent_t* ev = nullptr
         if (s->binning == 3) {
             return fail(s, MSIM_ERR_STATE, "internal: sorted-state move dispatch before the state was sorted");
         }
-        return enqueue_move_fast(s, write_dir, ev);
+        return enqueue_move_fast(s, write_dir, ev, false);
     }
     switch (mode) {
         case kMoveAll:
@@ -460,37 +480,37 @@ int enqueue_move(msim_sim* s, int mode, bool write_dir, hipEvent_t* ev = nullptr
     return check_launch(s, "move dispatch");
 }
 
-int enqueue_collide(msim_sim* s, bool slow, hipEvent_t* ev = nullptr) {
+// The neighbour pass of a collision dispatch of initialised agents.
+void launch_collide(msim_sim* s) {
     const AgentsDev a = s->agents(s->cur);
     const dim3 g(agent_blocks(s->n));
-    const uint32_t fold = s->stats_pending ? 1u : 0u;
-    s->stats_pending = false;
+    GridDev gd = s->grid_cur();
+    const float2* bpos = s->bbpos[s->bcur];
     if (s->sorted) {
         // the state itself is in slot order: positions are read in place and
         // the counts stored by slot
-        GridDev gd = s->grid_cur();
         gd.bid = nullptr;
-        const float2* bpos = s->buf[s->cur].pos;
-        probe_pre(s);
-        if (s->collide_mode == 1) {
-            hipLaunchKernelGGL((k_collide<false>), g, dim3(kBlock), 0, s->stream, a, gd, bpos, s->part_pairs);
-        } else if (s->collide_mode == 2) {
-            hipLaunchKernelGGL(k_collide_staged<1>, g, dim3(kBlock), 0, s->stream, a, gd, bpos, s->part_pairs);
-        } else {
-            const uint32_t per = kBlock * 2u;
-            hipLaunchKernelGGL(k_collide_staged<2>, dim3(std::max(1u, (s->n + per - 1) / per)), dim3(kBlock), 0,
-                               s->stream, a, gd, bpos, s->part_pairs);
-        }
-        probe_post(s);
-        probe_pre(s);
-        hipLaunchKernelGGL(k_collide_finish<false>, dim3(1), dim3(64), 0, s->stream, s->part_pairs, s->ctr,
-                           s->hist, s->hist_cap - 1, stats_buf(s), fold);
-        probe_post(s);
-        s->ncount_at = s->cur;
-        return check_launch(s, "collision dispatch");
+        bpos = s->buf[s->cur].pos;
     }
-    if (slow) {
-        probe_pre(s);
+    if (s->collide_mode == 1) {
+        hipLaunchKernelGGL((k_collide<false>), g, dim3(kBlock), 0, s->stream, a, gd, bpos, s->part_pairs);
+    } else if (s->collide_mode == 2) {
+        hipLaunchKernelGGL(k_collide_staged<1>, g, dim3(kBlock), 0, s->stream, a, gd, bpos, s->part_pairs);
+    } else {
+        const uint32_t per = kBlock * 2u;
+        hipLaunchKernelGGL(k_collide_staged<2>, dim3(std::max(1u, (s->n + per - 1) / per)), dim3(kBlock), 0,
+                           s->stream, a, gd, bpos, s->part_pairs);
+    }
+    if (s->sorted) s->ncount_at = s->cur;
+}
+
+int enqueue_collide(msim_sim* s, bool slow) {
+    const uint32_t fold = s->stats_pending ? 1u : 0u;
+    s->stats_pending = false;
+    probe_pre(s);
+    if (slow && !s->sorted) {
+        const AgentsDev a = s->agents(s->cur);
+        const dim3 g(agent_blocks(s->n));
         hipLaunchKernelGGL((k_collide<true>), g, dim3(kBlock), 0, s->stream, a, s->grid_cur(),
                            static_cast<const float2*>(s->bbpos[s->bcur]), s->part_pairs);
         probe_post(s);
@@ -499,19 +519,7 @@ int enqueue_collide(msim_sim* s, bool slow, hipEvent_t* ev = nullptr) {
                            s->hist, s->hist_cap - 1, stats_buf(s), fold);
         hipLaunchKernelGGL(k_set_init, g, dim3(kBlock), 0, s->stream, a.init, s->n);
     } else {
-        probe_pre(s);
-        if (s->collide_mode == 1) {
-            hipLaunchKernelGGL((k_collide<false>), g, dim3(kBlock), 0, s->stream, a, s->grid_cur(),
-                               static_cast<const float2*>(s->bbpos[s->bcur]), s->part_pairs);
-        } else if (s->collide_mode == 2) {
-            hipLaunchKernelGGL(k_collide_staged<1>, g, dim3(kBlock), 0, s->stream, a, s->grid_cur(),
-                               static_cast<const float2*>(s->bbpos[s->bcur]), s->part_pairs);
-        } else {
-            const uint32_t per = kBlock * 2u;
-            hipLaunchKernelGGL(k_collide_staged<2>, dim3(std::max(1u, (s->n + per - 1) / per)), dim3(kBlock), 0,
-                               s->stream, a, s->grid_cur(), static_cast<const float2*>(s->bbpos[s->bcur]),
-                               s->part_pairs);
-        }
+        launch_collide(s);
         probe_post(s);
         probe_pre(s);
         hipLaunchKernelGGL(k_collide_finish<false>, dim3(1), dim3(64), 0, s->stream, s->part_pairs, s->ctr,
@@ -607,7 +615,7 @@ constexpr uint32_t kScanThreads = 1024;
 // Otherwise the move alone (the route choice joins the neighbour pass).
 // finish: the previous tick's statistics are folded beside the move.
 template <uint32_t U, bool UN, bool W, bool L>
-void launch_sorted(msim_sim* s, const SortedMove& mv, const BinDev& b, const SortedFinish* finish) {
+void launch_sorted(msim_sim* s, const SortedMove& mv, const BinDev& b, const TickFinish* finish) {
     if (!mv.cur.seg) {
         probe_pre(s);
         hipLaunchKernelGGL(k_seg_scan<kScanThreads>, dim3(1), dim3(kScanThreads), 0, s->stream, s->seg_cnt[s->cur],
@@ -617,7 +625,7 @@ void launch_sorted(msim_sim* s, const SortedMove& mv, const BinDev& b, const Sor
     probe_pre(s);
     hipLaunchKernelGGL((k_move_sorted<U, kSortedThreads, UN, W, L>), dim3(s->n_seg + (finish ? kXcds : 0u)),
                        dim3(kSortedThreads), sorted_lds_bytes(s->seg_log), s->stream, mv, b,
-                       finish ? *finish : SortedFinish{});
+                       finish ? *finish : TickFinish{});
     probe_post(s);
     if (!mv.cur.seg) {
         probe_pre(s);
@@ -628,7 +636,7 @@ void launch_sorted(msim_sim* s, const SortedMove& mv, const BinDev& b, const Sor
 
 template <uint32_t U, bool L>
 void launch_sorted_l(msim_sim* s, const SortedMove& mv, const BinDev& b, bool write_dir,
-                     const SortedFinish* finish) {
+                     const TickFinish* finish) {
     if (s->uniform) {
         if (write_dir) launch_sorted<U, true, true, L>(s, mv, b, finish);
         else launch_sorted<U, true, false, L>(s, mv, b, finish);
@@ -640,7 +648,7 @@ void launch_sorted_l(msim_sim* s, const SortedMove& mv, const BinDev& b, bool wr
 
 template <uint32_t U>
 void launch_sorted_u(msim_sim* s, const SortedMove& mv, const BinDev& b, bool write_dir,
-                     const SortedFinish* finish) {
+                     const TickFinish* finish) {
     if (s->lists) launch_sorted_l<U, true>(s, mv, b, write_dir, finish);
     else launch_sorted_l<U, false>(s, mv, b, write_dir, finish);
 }
@@ -653,10 +661,6 @@ void launch_route_collide(msim_sim* s, const SortedMove& mv, const BinDev& b) {
     const RouteMix mix{s->n_seg, std::max(1u, (s->n + per - 1) / per)};
     hipLaunchKernelGGL((k_route_collide<UN, 2, L>), dim3(mix.blocks()), dim3(kBlock), 0, s->stream, mv, b,
                        s->agents(s->cur), gd, static_cast<const float2*>(s->buf[s->cur].pos), s->part_pairs, mix);
-}
-
-SortedFinish finish_args(const msim_sim* s) {
-    return SortedFinish{s->part_pairs, s->ctr, s->hist, s->hist_cap - 1, stats_buf(s)};
 }
 
 // Folds the statistics a fused tick left to its successor.
@@ -687,7 +691,7 @@ int enqueue_move_sorted(msim_sim* s, bool write_dir, bool fused) {
     mv.roads = s->roads;
     mv.conns = s->conns;
     mv.spd_const = s->spd_const;
-    const SortedFinish finish = finish_args(s);  // the previous tick's half of the statistics
+    const TickFinish finish = finish_args(s);  // the previous tick's half of the statistics
     const bool fin = s->finish_pending;
     s->finish_pending = false;
     s->stats_par ^= 1;  // the next tick's collision dispatch folds this half
@@ -718,7 +722,7 @@ int enqueue_move_sorted(msim_sim* s, bool write_dir, bool fused) {
     b.margin = s->margin;
     b.n = s->n;
     s->launch_no = 0;
-    const SortedFinish* pf = fin ? &finish : nullptr;
+    const TickFinish* pf = fin ? &finish : nullptr;
     if (s->bin_unroll == 2) launch_sorted_u<2>(s, mv, b, write_dir, pf);
     else if (s->bin_unroll == 8) launch_sorted_u<8>(s, mv, b, write_dir, pf);
     else launch_sorted_u<4>(s, mv, b, write_dir, pf);
@@ -740,16 +744,20 @@ int enqueue_move_sorted(msim_sim* s, bool write_dir, bool fused) {
     return check_launch(s, "sorted tick");
 }
 
-// One tick inside a run (not its last): the sorted state with the two-slot
-// staged neighbour pass takes the two-launch form.
+// One tick inside a run (not its last), its statistics left to the next
+// move: the sorted state with the two-slot staged neighbour pass takes the
+// two-launch form.
 int enqueue_run_tick(msim_sim* s) {
+    flush_stats(s);
     if (s->sorted && s->collide_mode == 0) {
-        flush_stats(s);
         return enqueue_move_sorted(s, false, true);
     }
-    int rc = enqueue_move(s, kMoveAll, false);
-    if (rc == MSIM_OK) rc = enqueue_collide(s, false);
-    return rc;
+    int rc = s->sorted ? enqueue_move_sorted(s, false, false) : enqueue_move_fast(s, false, nullptr, true);
+    if (rc != MSIM_OK) return rc;
+    launch_collide(s);
+    s->stats_pending = false;
+    s->finish_pending = true;
+    return check_launch(s, "tick");
 }
 
 // Sorted state: neighbour counts in the current slot order, in buf[cur].

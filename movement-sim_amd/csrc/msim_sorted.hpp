@@ -732,35 +732,18 @@ __device__ __forceinline__ void sorted_segment(const SortedMove& mv, const Table
 }
 
 
-// Statistics of a finished collision dispatch (k_collide_finish's work),
-// done by one extra workgroup of the next tick's move: a launch of its own
-// for one wave took 4.5 us of a 45 us tick (1M agents).
-struct SortedFinish {
-    unsigned long long* part_pairs;
-    Counters* ctr;
-    uint32_t* hist;
-    uint32_t hist_mask;
-    unsigned long long* part_stats;  // the finished tick's half
-};
-
-__device__ __forceinline__ void sorted_finish(const SortedFinish& f) {
-    if (threadIdx.x < 64u) {
-        finish_dispatch<false>(f.part_pairs, f.ctr, f.hist, f.hist_mask, f.part_stats, 1u);
-    }
-}
-
 // Sorted move of one table (grid: n_seg workgroups, after kXcds more when the
 // previous tick's statistics are pending; dynamic LDS:
 // sorted_lds_bytes(seg_log)).
 template <uint32_t U, uint32_t T, bool UNIFORM, bool WRITE_DIR, bool LISTS>
-static __global__ __launch_bounds__(T) void k_move_sorted(SortedMove mv, BinDev b, SortedFinish fin) {
+static __global__ __launch_bounds__(T) void k_move_sorted(SortedMove mv, BinDev b, TickFinish fin) {
     extern __shared__ uint32_t hist[];
     __shared__ uint32_t lds[T / 64];
     __shared__ uint32_t nh[2 * kNextReach + 1];
     __shared__ uint32_t sh[1 + T / 64];
     const uint32_t extra = gridDim.x - b.n_seg;
-    if (blockIdx.x < extra) {  // the previous tick's statistics, beside the move (see sorted_finish)
-        if (blockIdx.x == 0) sorted_finish(fin);
+    if (blockIdx.x < extra) {  // the previous tick's statistics, beside the move
+        fin.run(blockIdx.x);
         return;
     }
     const uint32_t seg = seg_order(blockIdx.x - extra, b.n_seg);

@@ -1,6 +1,7 @@
-"""Runs on the sorted state: the two-launch tick (move; route choice with the
-neighbour pass) at the sizes where its workgroup dealing and its folded
-statistics can go wrong, against the CPU oracle bit for bit."""
+"""Ticks inside runs, whose launches differ from single dispatches': the sorted
+state's two-launch tick, the one-launch scan of small tables, and statistics
+folded by the next move, at the sizes where their workgroup dealing can go
+wrong, against the CPU oracle bit for bit."""
 import numpy as np
 import pytest
 
@@ -71,3 +72,41 @@ def test_lists_of_leaving_agents_match_oracle(opts, agents):
     assert_same(g.state(), o.st, f"{opts}, dispatches")
     assert g.pairs()[0] == o.pairs_total
     g.sync()
+
+
+@pytest.mark.parametrize("agents", [1, 257, 1025, 5000])
+@pytest.mark.parametrize("opts", [dict(binning=0), dict(binning=0, route_queue=1), dict(binning=1),
+                                  dict(binning=1, route_queue=1, table_log2=15), dict(binning=1, table_log2=16),
+                                  dict(binning=2, collide_mode=1), dict(binning=3, collide_mode=2)])
+def test_run_statistics_match_oracle(agents, opts):
+    """Pair history, insertions and state after direct and captured ticks, with
+    renumberings in between, in every layout."""
+    sc = S.config(1, scale=0.5)
+    sc.entities, sc.speed = sc.entities[:agents], sc.speed[:agents]
+    g, o = pair(sc, graph_ticks=6, reorder_interval=3, **opts)
+    ref = msim.Simulation(sc.roads, sc.conns, sc.entities, sc.pc, speed=sc.speed)
+    for ticks in (1, 5, 26, 2, 13):
+        g.run_ticks(ticks)
+        o.run_ticks(ticks)
+        for _ in range(ticks):
+            ref.sim_tick()
+        assert_same(g.state(), o.st, f"{agents} agents, {opts}")
+        np.testing.assert_array_equal(g.debug_data(), ref.debug_data())
+    total, hist = g.pairs()
+    assert total == o.pairs_total
+    assert hist.tolist() == o.pair_hist
+    g.sync()
+
+
+@pytest.mark.parametrize("n_scen", [1, 31, 33])
+@pytest.mark.parametrize("binning", [0, 2])
+def test_classic_batch_run_folds_every_scenarios_pairs(n_scen, binning):
+    scs = S.batch_config(n_scen, scale=0.004, seed=12)
+    b = msim.Batch(scs, binning=binning, graph_ticks=6, reorder_interval=3)
+    b.run_ticks(29)
+    tot, last = b.pairs()
+    for s, sc in enumerate(scs):
+        o = orc.OracleSim(sc.roads, sc.conns, sc.entities, sc.pc, speed=sc.speed)
+        o.run_ticks(29)
+        assert int(tot[s]) == o.pairs_total and int(last[s]) == o.pair_hist[-1], f"scenario {s}"
+    b.sync()
