@@ -32,8 +32,6 @@ void badvance(msim_batch* b) {
                        b->inv_cell, b->part_stats, b->roads, b->conns, extra, bfinish_args(b));
 }
 
-constexpr uint32_t kBSortedThreads = 512;
-
 inline size_t bsorted_lds_bytes(uint32_t seg_log) { return sorted_lds_bytes(seg_log); }
 
 SortedBufs bsorted_bufs(const msim_batch* b, int k) {
@@ -45,7 +43,7 @@ constexpr uint32_t kBScanThreads = 1024;
 
 // mv.cur.seg null: scan, move and route choice, each in a launch of its own.
 // Otherwise the move alone (the route choice joins the neighbour pass).
-template <uint32_t U, bool UN, bool W>
+template <uint32_t U, uint32_t T, bool UN, bool W>
 void blaunch_sorted(msim_batch* b, const SortedMove& mv, const BatchBin& bb, bool finish) {
     if (!mv.cur.seg) {
         bprobe_pre(b);
@@ -53,9 +51,9 @@ void blaunch_sorted(msim_batch* b, const SortedMove& mv, const BatchBin& bb, boo
                            b->seg_cnt[b->cur], b->seg_group[b->cur], b->seg_start, b->n_seg, b->n, b->faults);
         bprobe_post(b);
     }
-    const uint32_t extra = finish ? bfinish_blocks(b, kBSortedThreads) : 0u;
+    const uint32_t extra = finish ? bfinish_blocks(b, T) : 0u;
     bprobe_pre(b);
-    hipLaunchKernelGGL((k_bmove_sorted<U, kBSortedThreads, UN, W>), dim3(b->n_seg + extra), dim3(kBSortedThreads),
+    hipLaunchKernelGGL((k_bmove_sorted<U, T, UN, W>), dim3(b->n_seg + extra), dim3(T),
                        bsorted_lds_bytes(b->max_seg_log), b->stream, mv, bb, bfinish_args(b));
     bprobe_post(b);
     if (!mv.cur.seg) {
@@ -65,14 +63,14 @@ void blaunch_sorted(msim_batch* b, const SortedMove& mv, const BatchBin& bb, boo
     }
 }
 
-template <uint32_t U>
+template <uint32_t U, uint32_t T>
 void blaunch_sorted_u(msim_batch* b, const SortedMove& mv, const BatchBin& bb, bool write_dir, bool finish) {
     if (b->uniform) {
-        if (write_dir) blaunch_sorted<U, true, true>(b, mv, bb, finish);
-        else blaunch_sorted<U, true, false>(b, mv, bb, finish);
+        if (write_dir) blaunch_sorted<U, T, true, true>(b, mv, bb, finish);
+        else blaunch_sorted<U, T, true, false>(b, mv, bb, finish);
     } else {
-        if (write_dir) blaunch_sorted<U, false, true>(b, mv, bb, finish);
-        else blaunch_sorted<U, false, false>(b, mv, bb, finish);
+        if (write_dir) blaunch_sorted<U, T, false, true>(b, mv, bb, finish);
+        else blaunch_sorted<U, T, false, false>(b, mv, bb, finish);
     }
 }
 
@@ -110,9 +108,10 @@ int benqueue_tick_sorted(msim_batch* b, bool write_dir, bool fused) {
     bb.n_seg = b->n_seg;
     const bool finish = b->finish_pending;
     b->finish_pending = false;
-    if (b->bin_unroll == 2) blaunch_sorted_u<2>(b, mv, bb, write_dir, finish);
-    else if (b->bin_unroll == 8) blaunch_sorted_u<8>(b, mv, bb, write_dir, finish);
-    else blaunch_sorted_u<4>(b, mv, bb, write_dir, finish);
+    if (one_move_per_cu(b->n_seg, b->min_seg_log)) blaunch_sorted_u<1, kSortedWide>(b, mv, bb, write_dir, finish);
+    else if (b->bin_unroll == 2) blaunch_sorted_u<2, kSortedThreads>(b, mv, bb, write_dir, finish);
+    else if (b->bin_unroll == 8) blaunch_sorted_u<8, kSortedThreads>(b, mv, bb, write_dir, finish);
+    else blaunch_sorted_u<4, kSortedThreads>(b, mv, bb, write_dir, finish);
     b->cur = nb;
     b->bcur = 1 - b->bcur;
     if (!fused) {
@@ -488,6 +487,7 @@ extern "C" int msim_batch_create(uint32_t n_scen, const uint32_t* road_off, cons
         d.n_seg = d.m >> seg_log;
         for (uint32_t k = 0; k < d.n_seg; k++) seg_scen.push_back(s);
         b->max_seg_log = std::max(b->max_seg_log, seg_log);
+        b->min_seg_log = std::min(b->min_seg_log, seg_log);
     }
     b->n_seg = static_cast<uint32_t>(seg_scen.size());
     b->bin_unroll = o.bin_unroll ? o.bin_unroll : (o.binning == 3 ? 4u : auto_bin_unroll(b->max_seg_log));

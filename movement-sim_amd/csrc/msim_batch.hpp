@@ -410,7 +410,7 @@ int bleave_sorted(msim_batch* b);  // msim_batch.hip
 
 struct msim_batch {
     hipStream_t stream = nullptr;
-    uint32_t n_scen = 0, n = 0, n_roads = 0, n_conns = 0, n_seg = 0, start_len = 0, max_seg_log = 9;
+    uint32_t n_scen = 0, n = 0, n_roads = 0, n_conns = 0, n_seg = 0, start_len = 0, max_seg_log = 9, min_seg_log = 32;
     std::vector<uint32_t> agent_off_h, road_off_h;
     msim_road* roads = nullptr;
     uint32_t* conns = nullptr;

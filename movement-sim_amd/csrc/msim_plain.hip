@@ -562,7 +562,6 @@ SortedBufs sorted_bufs(const msim_sim* s, int k) {
 
 SegCounts seg_counts(const msim_sim* s, int k) { return SegCounts{s->seg_cnt[k], s->seg_group[k]}; }
 
-constexpr uint32_t kSortedThreads = 512;
 
 
 // Enters the sorted state from the classic layout: renumbers the agents into
@@ -614,7 +613,7 @@ constexpr uint32_t kScanThreads = 1024;
 // mv.cur.seg null: scan, move and route choice, each in a launch of its own.
 // Otherwise the move alone (the route choice joins the neighbour pass).
 // finish: the previous tick's statistics are folded beside the move.
-template <uint32_t U, bool UN, bool W, bool L>
+template <uint32_t U, uint32_t T, bool UN, bool W, bool L>
 void launch_sorted(msim_sim* s, const SortedMove& mv, const BinDev& b, const TickFinish* finish) {
     if (!mv.cur.seg) {
         probe_pre(s);
@@ -623,8 +622,8 @@ void launch_sorted(msim_sim* s, const SortedMove& mv, const BinDev& b, const Tic
         probe_post(s);
     }
     probe_pre(s);
-    hipLaunchKernelGGL((k_move_sorted<U, kSortedThreads, UN, W, L>), dim3(s->n_seg + (finish ? kXcds : 0u)),
-                       dim3(kSortedThreads), sorted_lds_bytes(s->seg_log), s->stream, mv, b,
+    hipLaunchKernelGGL((k_move_sorted<U, T, UN, W, L>), dim3(s->n_seg + (finish ? kXcds : 0u)),
+                       dim3(T), sorted_lds_bytes(s->seg_log), s->stream, mv, b,
                        finish ? *finish : TickFinish{});
     probe_post(s);
     if (!mv.cur.seg) {
@@ -634,23 +633,23 @@ void launch_sorted(msim_sim* s, const SortedMove& mv, const BinDev& b, const Tic
     }
 }
 
-template <uint32_t U, bool L>
+template <uint32_t U, uint32_t T, bool L>
 void launch_sorted_l(msim_sim* s, const SortedMove& mv, const BinDev& b, bool write_dir,
                      const TickFinish* finish) {
     if (s->uniform) {
-        if (write_dir) launch_sorted<U, true, true, L>(s, mv, b, finish);
-        else launch_sorted<U, true, false, L>(s, mv, b, finish);
+        if (write_dir) launch_sorted<U, T, true, true, L>(s, mv, b, finish);
+        else launch_sorted<U, T, true, false, L>(s, mv, b, finish);
     } else {
-        if (write_dir) launch_sorted<U, false, true, L>(s, mv, b, finish);
-        else launch_sorted<U, false, false, L>(s, mv, b, finish);
+        if (write_dir) launch_sorted<U, T, false, true, L>(s, mv, b, finish);
+        else launch_sorted<U, T, false, false, L>(s, mv, b, finish);
     }
 }
 
-template <uint32_t U>
+template <uint32_t U, uint32_t T>
 void launch_sorted_u(msim_sim* s, const SortedMove& mv, const BinDev& b, bool write_dir,
                      const TickFinish* finish) {
-    if (s->lists) launch_sorted_l<U, true>(s, mv, b, write_dir, finish);
-    else launch_sorted_l<U, false>(s, mv, b, write_dir, finish);
+    if (s->lists) launch_sorted_l<U, T, true>(s, mv, b, write_dir, finish);
+    else launch_sorted_l<U, T, false>(s, mv, b, write_dir, finish);
 }
 
 template <bool UN, bool L>
@@ -723,9 +722,10 @@ int enqueue_move_sorted(msim_sim* s, bool write_dir, bool fused) {
     b.n = s->n;
     s->launch_no = 0;
     const TickFinish* pf = fin ? &finish : nullptr;
-    if (s->bin_unroll == 2) launch_sorted_u<2>(s, mv, b, write_dir, pf);
-    else if (s->bin_unroll == 8) launch_sorted_u<8>(s, mv, b, write_dir, pf);
-    else launch_sorted_u<4>(s, mv, b, write_dir, pf);
+    if (one_move_per_cu(s->n_seg, s->seg_log)) launch_sorted_u<1, kSortedWide>(s, mv, b, write_dir, pf);
+    else if (s->bin_unroll == 2) launch_sorted_u<2, kSortedThreads>(s, mv, b, write_dir, pf);
+    else if (s->bin_unroll == 8) launch_sorted_u<8, kSortedThreads>(s, mv, b, write_dir, pf);
+    else launch_sorted_u<4, kSortedThreads>(s, mv, b, write_dir, pf);
     s->cur = nb;
     s->bcur = 1 - s->bcur;
     if (!fused) {

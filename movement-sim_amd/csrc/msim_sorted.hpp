@@ -547,6 +547,17 @@ __device__ __forceinline__ uint32_t seg_order(uint32_t bid, uint32_t n_seg) {
     return xcd_deal<4>(bid, n_seg, 3u * kCus);
 }
 
+// Move workgroups have 512 threads; where each gets a CU of its own, 1,024
+// with one slot per thread and round: the phases of a lone workgroup are a
+// chain of waits, and twice the threads take half the rounds.  Ticks, us: 100k
+// agents on 64 segments of 2^11 buckets 21.1 -> 19.4; 200k skewed agents on 64
+// of 2^12 40 -> 33; 1M on 256 of 2^12 55 -> 47; but 1M on 512 of 2^11, two
+// workgroups a CU, 39 -> 42.
+constexpr uint32_t kSortedThreads = 512, kSortedWide = 1024;
+inline bool one_move_per_cu(uint32_t n_seg, uint32_t smallest_seg_log) {
+    return n_seg <= kCus && (1u << smallest_seg_log) >= kSortedWide;  // a thread scans at least one bucket
+}
+
 // LDS of the sorted move: the segment's counters (4 bytes per bucket) and,
 // for its first sorted_map_cap new slots, each agent's window index and its
 // bucket in the segment (2 + 2 bytes).  Segments of up to 2^12 buckets map 2

@@ -57,6 +57,8 @@ def test_batch_run_folds_every_scenarios_pairs(n_scen):
     (dict(table_log2=13, segment_log2=9, table_width_log2=7), 4000),    # margin wider than 3/4 of a segment
     (dict(table_log2=14, segment_log2=12, table_width_log2=10), 60000),  # more leavers than their slots fit in LDS
     (dict(table_log2=13, segment_log2=12, table_width_log2=9), 60000),  # crowded past the map and its 16-bit window
+    (dict(table_log2=18, segment_log2=10, table_width_log2=7), 20000),  # 256 segments: workgroups of 1,024 threads
+    (dict(table_log2=19, segment_log2=10, table_width_log2=7), 20000),  # 512: of 512
 ])
 def test_lists_of_leaving_agents_match_oracle(opts, agents):
     sc = S.config(1)
