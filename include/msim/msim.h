@@ -68,7 +68,7 @@ typedef struct msim_options {
                                   lane loads its own; 2: staged, 1 slot per
                                   lane                                          */
     uint32_t bin_unroll;       /* window slots each rebinning thread loads per
-                                  round: 4 or 8 (0: 8 for segments of up to
+                                  round: 4 or 8 (0: 8 for segments of 2^12 and
                                   2^13 buckets, else 4); binning 3: 2, 4 or 8
                                   (0: 4)                                        */
 } msim_options;

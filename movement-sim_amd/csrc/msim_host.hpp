@@ -81,10 +81,14 @@ inline uint32_t auto_batch_segment_log2(uint64_t buckets, uint32_t tlog, uint32_
     return l;
 }
 
-// Window slots each rebinning thread loads per round: 8 keeps more loads in
-// flight; segments of 2^14 buckets (64 KB of LDS counters, two workgroups
-// per CU) measured faster with 4.
-inline uint32_t auto_bin_unroll(uint32_t seg_log) { return seg_log <= 13 ? 8u : 4u; }
+// Window slots each rebinning thread loads per round.  Segments of up to 2^11
+// buckets have windows of at most about 4,000 slots, which 512 threads with 8
+// each load mostly past the end: ticks of 10k agents 28.0 us with 8, 26.0 with
+// 4; 123k 30.8, 28.8; 1M 53.4, 51.0; 16 scenarios 34.6, 31.4.  At 2^12 buckets
+// (8M agents) 8 keep more loads in flight: 414 us, 431 with 4.  Segments of
+// 2^14 buckets (64 KB of LDS counters, two workgroups per CU) measured faster
+// with 4.
+inline uint32_t auto_bin_unroll(uint32_t seg_log) { return seg_log == 12u || seg_log == 13u ? 8u : 4u; }
 
 // Bounding box of the roads and agents.
 struct Extent {
