@@ -695,12 +695,9 @@ extern "C" int msim_batch_run_ticks(msim_batch* b, uint32_t n_ticks) {
 
 extern "C" int msim_batch_sync(msim_batch* b) {
     if (!b) return bfail(b, MSIM_ERR_INVALID, "NULL handle");
-    hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, b->stream, b->faults, b->box, ++b->reports);
-    int rc = bcheck(b, "k_report");
+    unsigned int f = 0;
+    int rc = bwait_report(b, &f);
     if (rc != MSIM_OK) return rc;
-    if (!await_report(b->box, b->reports)) rc = bwait(b);
-    if (rc != MSIM_OK) return rc;
-    const unsigned int f = static_cast<unsigned int>(b->box->word);
     if (f) {
         return bfail(b, MSIM_ERR_STATE, "device-side check failed (fault bits 0x%x%s%s%s)", f,
                      (f & kFaultBinCount) ? ": binned agent count != agent count" : "",
@@ -716,8 +713,7 @@ extern "C" int msim_batch_read_state(msim_batch* b, uint32_t scen, float* pos, f
     // a scenario's agents stay inside its slot range through every reorder
     const uint32_t off = b->agent_off_h[scen], na = b->agent_off_h[scen + 1] - off;
     if (na == 0) return msim_batch_sync(b);
-    void* to = b->readback.small(StateOut::kWords * sizeof(uint4) * na);
-    const StateOut o = StateOut::at(to ? to : b->read_stage, na);
+    StateOut o = StateOut::at(b->read_stage, na);
     const dim3 g(bblocks(na));
     if (b->sorted) {
         hipLaunchKernelGGL(k_export_state_rec, g, dim3(kBlock), 0, b->stream, b->agents(b->cur), b->rec[b->cur],
@@ -725,6 +721,12 @@ extern "C" int msim_batch_read_state(msim_batch* b, uint32_t scen, float* pos, f
     } else {
         hipLaunchKernelGGL(k_export_state, g, dim3(kBlock), 0, b->stream, b->agents(b->cur), off, na,
                            b->road_off_h[scen], o);
+    }
+    if (void* to = b->readback.small(StateOut::kWords * sizeof(uint4) * na)) {
+        const uint32_t words = static_cast<uint32_t>(StateOut::kWords) * na;
+        hipLaunchKernelGGL(k_copy_out, dim3(bblocks(words)), dim3(kBlock), 0, b->stream, b->read_stage,
+                           static_cast<uint4*>(to), words);
+        o = StateOut::at(to, na);
     }
     int rc = bcheck(b, "k_export_state");
     if (rc != MSIM_OK) return rc;

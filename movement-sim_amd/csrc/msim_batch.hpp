@@ -595,6 +595,16 @@ inline int bwait(msim_batch* b) {
     return MSIM_OK;
 }
 
+// The fault word as of the stream's last work, which has ended on return.
+inline int bwait_report(msim_batch* b, unsigned int* f) {
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, b->stream, b->faults, b->box, ++b->reports);
+    int rc = bcheck(b, "k_report");
+    if (rc != MSIM_OK) return rc;
+    if (!await_report(b->box, b->reports)) rc = bwait(b);
+    *f = static_cast<unsigned int>(b->box->word);
+    return rc;
+}
+
 // The parts into the caller's memory, after the stream's work and the
 // device-side checks.
 inline int bread_parts(msim_batch* b, const std::vector<ReadPart>& parts) {

@@ -406,8 +406,9 @@ int enqueue_move_fast(msim_sim* s, bool write_dir, hipEvent_t* ev, bool in_run) 
     } else {
         const GridDev g = s->grid_cur();
         const uint32_t n_part = g.m / kScanTile;
-        if (in_run && g.m <= kScanOne) {
-            hipLaunchKernelGGL(k_scan_one<1024>, dim3(1), dim3(1024), 0, s->stream, g.cnt, g.start, g.m);
+        const bool direct = in_run && g.m <= kScanDirect;
+        if (direct) {
+            hipLaunchKernelGGL(k_scan_direct, dim3(n_part), dim3(kBlock), 0, s->stream, g.cnt, g.start, g.m);
         } else {
             probe_pre(s);
             hipLaunchKernelGGL(k_scan_reduce, dim3(n_part), dim3(kBlock), 0, s->stream, g.cnt, g.part);
@@ -421,8 +422,13 @@ int enqueue_move_fast(msim_sim* s, bool write_dir, hipEvent_t* ev, bool in_run) 
             probe_post(s);
         }
         probe_pre(s);
-        hipLaunchKernelGGL(k_scatter, dim3(agent_blocks(s->n)), dim3(kBlock), 0, s->stream, s->agents(s->cur),
-                           g);
+        if (direct) {
+            hipLaunchKernelGGL(k_scatter<true>, dim3(agent_blocks(s->n)), dim3(kBlock), 0, s->stream,
+                               s->agents(s->cur), g);
+        } else {
+            hipLaunchKernelGGL(k_scatter<false>, dim3(agent_blocks(s->n)), dim3(kBlock), 0, s->stream,
+                               s->agents(s->cur), g);
+        }
         probe_post(s);
     }
     s->stats_pending = true;  // folded by the next collision dispatch's finish pass
@@ -474,7 +480,7 @@ int enqueue_move(msim_sim* s, int mode, bool write_dir, hipEvent_t* ev = nullptr
     if (ev) (void)hipEventRecord(ev[2], s->stream);
     hipLaunchKernelGGL(k_scan_down, dim3(n_part), dim3(kBlock), 0, s->stream, g.cnt, g.part, g.start);
     if (ev) (void)hipEventRecord(ev[3], s->stream);
-    hipLaunchKernelGGL(k_scatter, dim3(agent_blocks(s->n)), dim3(kBlock), 0, s->stream,
+    hipLaunchKernelGGL(k_scatter<false>, dim3(agent_blocks(s->n)), dim3(kBlock), 0, s->stream,
                        s->agents(s->cur), g);
     if (ev) (void)hipEventRecord(ev[4], s->stream);
     return check_launch(s, "move dispatch");
@@ -1329,14 +1335,19 @@ extern "C" int msim_read_state(msim_sim* s, float* pos, float* target, float* di
     if (rc != MSIM_OK) return rc;
     // caller order on the device, in the entity staging buffer (64 bytes per agent)
     static_assert(StateOut::kWords * sizeof(uint4) <= sizeof(msim_entity), "state fits the staging buffer");
-    void* to = s->readback.small(StateOut::kWords * sizeof(uint4) * n);
-    const StateOut o = StateOut::at(to ? to : s->ent_stage, n);
+    StateOut o = StateOut::at(s->ent_stage, n);
     const dim3 g(agent_blocks(s->n));
     if (s->sorted) {
         hipLaunchKernelGGL(k_export_state_rec, g, dim3(kBlock), 0, s->stream, s->agents(s->cur), s->rec[s->cur],
                            s->cold, 0u, s->n, 0u, o);
     } else {
         hipLaunchKernelGGL(k_export_state, g, dim3(kBlock), 0, s->stream, s->agents(s->cur), 0u, s->n, 0u, o);
+    }
+    if (void* to = s->readback.small(StateOut::kWords * sizeof(uint4) * n)) {
+        const uint32_t words = static_cast<uint32_t>(StateOut::kWords * n);
+        hipLaunchKernelGGL(k_copy_out, dim3(agent_blocks(words)), dim3(kBlock), 0, s->stream,
+                           reinterpret_cast<const uint4*>(s->ent_stage), static_cast<uint4*>(to), words);
+        o = StateOut::at(to, n);
     }
     rc = check_launch(s, "k_export_state");
     if (rc != MSIM_OK) return rc;
