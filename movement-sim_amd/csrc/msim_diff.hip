@@ -260,14 +260,13 @@ struct PushVisitor {
 // bit-identical.  A push beyond the windows' allowance raises kFaultBinCount
 // (the run then fails instead of rebinning an agent outside its window).
 // Positions without a neighbour stay as the move left them (p + 0 differs
-// from p only for p = -0).  move = 0: only near is recorded.
+// from p only for p = -0).
 // (One slot per lane: with two, 110 registers and half the waves, 800k agents
 // took 41 us against 28; a lane walking its cells in global memory, without
 // staging, 33.)
 template <int P>
-static __global__ __launch_bounds__(kBlock, 4) void k_davoid(DiffCells c, float alpha, uint32_t move,
-                                                             float2* __restrict__ pos, DiffNear near,
-                                                             unsigned int* __restrict__ faults) {
+static __global__ __launch_bounds__(kBlock, 4) void k_davoid(DiffCells c, float alpha, float2* __restrict__ pos,
+                                                             DiffNear near, unsigned int* __restrict__ faults) {
     __shared__ float2 stage_all[kBlock / 64 * kStage];
     const uint32_t blk = collide_order(blockIdx.x, gridDim.x);
     const uint32_t wave = blk * (kBlock / 64) + (threadIdx.x >> 6);
@@ -310,23 +309,21 @@ static __global__ __launch_bounds__(kBlock, 4) void k_davoid(DiffCells c, float 
     for (int p = 0; p < P; p++) {
         const uint32_t s = w0 + 64u * p + lane;
         const bool has = valid[p] && v.cnt[p] > 1u;
-        const bool moves = move && valid[p] && (has || me[p].x == 0.0f || me[p].y == 0.0f);
+        const bool moves = valid[p] && (has || me[p].x == 0.0f || me[p].y == 0.0f);
         const unsigned long long hm = __ballot(has);
-        if (has || moves) {
+        if (moves) {
             const uint32_t i = c.bid[s];
             if (near.list && has) {
                 near.list[w0 + kNearGroup * p + static_cast<uint32_t>(__popcll(hm & ((1ull << lane) - 1ull)))] =
                     static_cast<uint8_t>(lane);
                 near.flag[i] |= kDiffNear;
             }
-            if (moves) {
-                const float px = alpha * static_cast<float>(static_cast<double>(v.ix[p]) / v.sc);
-                const float py = alpha * static_cast<float>(static_cast<double>(v.iy[p]) / v.sc);
-                if (!(fabsf(px) <= c.push_allow) || !(fabsf(py) <= c.push_allow)) {
-                    atomicOr(faults, kFaultBinCount);
-                }
-                pos[i] = make_float2(me[p].x + px, me[p].y + py);
+            const float px = alpha * static_cast<float>(static_cast<double>(v.ix[p]) / v.sc);
+            const float py = alpha * static_cast<float>(static_cast<double>(v.iy[p]) / v.sc);
+            if (!(fabsf(px) <= c.push_allow) || !(fabsf(py) <= c.push_allow)) {
+                atomicOr(faults, kFaultBinCount);
             }
+            pos[i] = make_float2(me[p].x + px, me[p].y + py);
         }
         if (near.list && lane == 0 && w0 + kNearGroup * p < c.n) {
             near.count[wave * P + p] = static_cast<uint8_t>(__popcll(hm));
@@ -341,7 +338,9 @@ constexpr uint32_t kAlphaSlots = 64, kAlphaStride = 16;
 // Avoidance adjoint over the tick's binning, in binary64 from the run's
 // binary32 positions, for the listed slots: lam_out = lam + alpha * sum J dl
 // at their agents, and the alpha derivative sum lam . A.  A workgroup takes
-// GROUPS groups.
+// GROUPS groups.  Without lists (alpha = 0: the forward run had no avoidance
+// to list them in, and lam stays as it is) only the derivative, over all
+// slots.
 template <uint32_t GROUPS>
 static __global__ __launch_bounds__(kBlock) void k_davoid_adj(DiffCells c, DiffNear near, double alpha,
                                                        const double2* __restrict__ lam,
@@ -354,7 +353,9 @@ static __global__ __launch_bounds__(kBlock) void k_davoid_adj(DiffCells c, DiffN
     uint32_t m = 0;
 #pragma unroll
     for (uint32_t k = 0; k < GROUPS; k++) {
-        m += g0 + k < n_groups ? near.count[g0 + k] : 0u;
+        if (g0 + k < n_groups) {
+            m += near.list ? near.count[g0 + k] : min(kNearGroup, c.n - (g0 + k) * kNearGroup);
+        }
         end[k] = m;
     }
     double ga = 0.0;
@@ -368,7 +369,7 @@ static __global__ __launch_bounds__(kBlock) void k_davoid_adj(DiffCells c, DiffN
             }
         }
         const uint32_t base = (g0 + k) * kNearGroup;
-        const uint32_t s = base + near.list[base + (e - first)];
+        const uint32_t s = base + (near.list ? near.list[base + (e - first)] : e - first);
         const float2 me = c.bpos[s];
         const uint32_t i = c.bid[s];
         const double2 li = lam[i];
@@ -415,7 +416,7 @@ static __global__ __launch_bounds__(kBlock) void k_davoid_adj(DiffCells c, DiffN
         for (uint32_t k = 0; k < 4u; k++) {
             if (waiting > k) add(q[k], lj[k]);
         }
-        lam_out[i] = make_double2(li.x + alpha * gx, li.y + alpha * gy);
+        if (near.list) lam_out[i] = make_double2(li.x + alpha * gx, li.y + alpha * gy);
         ga += li.x * ax + li.y * ay;
     }
     if (m == 0u) {
@@ -742,10 +743,9 @@ void dtick(msim_batch* b, DiffState& d, const float* theta, float alpha, uint32_
         }
     }
     dbins(b, d, old_start, old_bid, new_start, new_bpos, new_bid);
-    if (alpha != 0.0f || near.list) {
-        const DiffCells c = dcells(b, new_start, new_bpos, new_bid);
-        const uint32_t move = alpha != 0.0f ? 1u : 0u;
-        hipLaunchKernelGGL(k_davoid<1>, g, dim3(kBlock), 0, b->stream, c, alpha, move, a.pos, near, b->faults);
+    if (alpha != 0.0f) {
+        hipLaunchKernelGGL(k_davoid<1>, g, dim3(kBlock), 0, b->stream, dcells(b, new_start, new_bpos, new_bid),
+                           alpha, a.pos, near, b->faults);
     }
 }
 
@@ -773,9 +773,7 @@ void launch_davoid_adj(msim_batch* b, DiffState& d, const DiffCells& c, const Di
 
 int check_diff_faults(msim_batch* b) {
     unsigned int f = 0;
-    hipError_t e = hipMemcpyAsync(&f, b->faults, sizeof(f), hipMemcpyDeviceToHost, b->stream);
-    if (e != hipSuccess) return bfail(b, MSIM_ERR_HIP, "fault readback: %s", hipGetErrorString(e));
-    int rc = bwait(b);
+    int rc = bwait_report(b, &f);
     if (rc != MSIM_OK) return rc;
     if (f & kFaultBinCount) {
         return bfail(b, MSIM_ERR_STATE,
@@ -1012,7 +1010,7 @@ extern "C" int msim_batch_diff_backward(msim_batch* b, const float* grad_pos, do
             const uint32_t j = t - t0;
             const DiffCells c = dcells(b, d.tp_start + static_cast<size_t>(b->start_len) * j, d.tp_bpos + (n + 2) * j,
                                        d.tp_bid + n * j);
-            launch_davoid_adj(b, d, c, near_at(b, d, j));
+            launch_davoid_adj(b, d, c, d.alpha != 0.0f ? near_at(b, d, j) : DiffNear{});
             const AgentsDev a = b->agents(b->cur);
             // the decisions after tick t: the tape's next entry, or after the
             // segment's last tick the agent state its replay ended in
