@@ -17,7 +17,6 @@
 #include <cstddef>
 #include <cstdint>
 #include <cstring>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -183,12 +182,10 @@ public:
             }
         };
         std::vector<std::thread> helpers;
-        for (uint32_t t = 1; t < n; t++) {
-            try {
-                helpers.emplace_back(work, t);
-            } catch (const std::system_error&) {
-                break;  // the threads there are take all pieces
-            }
+        try {
+            helpers.reserve(n);
+            for (uint32_t t = 1; t < n; t++) helpers.emplace_back(work, t);
+        } catch (...) {  // no more threads: those there are take all pieces
         }
         work(0);
         for (std::thread& h : helpers) h.join();
