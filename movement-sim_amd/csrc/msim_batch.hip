@@ -8,8 +8,8 @@
 // contiguous binned slots [agent_off_s, agent_off_s + n_s), so the rebinning
 // and neighbour kernels only need the scenario's table parameters, found from
 // the segment (rebinning) or by binary search over agent_off (neighbours).
-// A tick is 5 launches for all scenarios; ticks run as captured hipGraph
-// segments.  Per-scenario results are bit-identical to plain runs.
+// A tick is 2 to 5 launches for all scenarios (2 in runs on the sorted state);
+// ticks run as captured hipGraph segments.  Per-scenario results are bit-identical to plain runs.
 #include "msim_batch.hpp"
 
 #include <cmath>
@@ -549,12 +549,18 @@ extern "C" int msim_batch_create(uint32_t n_scen, const uint32_t* road_off, cons
     uint32_t n_max = 0;
     for (const ScenDev& d : sc) n_max = std::max(n_max, d.n);
     BALLOC(b->read_stage, StateOut::kWords * static_cast<size_t>(n_max));
-    if (rc == MSIM_OK && hipHostMalloc(reinterpret_cast<void**>(&b->box), sizeof(Mailbox), hipHostMallocDefault) !=
-                             hipSuccess) {
-        b->box = nullptr;
-        rc = bfail(b, MSIM_ERR_OOM, "hipHostMalloc(%zu) failed", sizeof(Mailbox));
+    // two mailboxes, in lines of their own
+    void* boxes = nullptr;
+    if (rc == MSIM_OK && hipHostMalloc(&boxes, 2 * 128, hipHostMallocDefault) != hipSuccess) {
+        boxes = nullptr;
+        rc = bfail(b, MSIM_ERR_OOM, "hipHostMalloc(%d) failed", 2 * 128);
     }
-    if (rc == MSIM_OK) b->box->word = 0;
+    b->box = static_cast<Mailbox*>(boxes);
+    if (rc == MSIM_OK) {
+        b->verdict = reinterpret_cast<Mailbox*>(static_cast<char*>(boxes) + 128);
+        b->box->word = 0;
+        b->verdict->word = 0;
+    }
 #undef BALLOC
     if (rc != MSIM_OK) {
         std::string e = b->err;

@@ -473,6 +473,7 @@ struct msim_batch {
     msim::ReadBack readback;
     uint4* read_stage = nullptr;      // [StateOut::kWords * largest scenario] a scenario's state in caller order
     msim::Mailbox* box = nullptr;     // pinned fault report (msim_batch_sync)
+    msim::Mailbox* verdict = nullptr;  // in the same allocation: parameter checks of the differentiable tick
     unsigned int reports = 0;
     DiffState* diff = nullptr;
 

@@ -108,7 +108,7 @@ struct msim_sim {
     int qpar = 0;
     Counters* ctr = nullptr;
     unsigned long long* part_stats = nullptr;  // [2][kSlots * kSlotStride] advance statistics
-    int stats_par = 0;  // half of part_stats the last move dispatch added to (sorted state: alternates)
+    int stats_par = 0;  // half of part_stats the last move dispatch added to; alternates
     unsigned long long* part_pairs = nullptr;  // [kSlots * kSlotStride] neighbour sums
     uint32_t* hist = nullptr;
     uint32_t hist_cap = 0;

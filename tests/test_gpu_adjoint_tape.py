@@ -71,3 +71,40 @@ def test_taped_and_replayed_gradients_agree(sizes, ticks, every, alpha, arrivals
     _close(taped, again)
     b.close()
     b2.close()
+
+
+# the multipliers are checked on the device, in 2^17 threads: few of them, and
+# more than one pass; the largest (its agents cross many cells a tick, and the
+# rebinning windows have to allow for that) and a bad one at the end
+@pytest.mark.parametrize("sizes,nodes", [((40,), 64), ((3000, 500), 90_000)])
+@pytest.mark.parametrize("bad", [-1.0, float("inf"), float("nan")])
+def test_multipliers_are_checked_on_the_device(sizes, nodes, bad):
+    scs = _scenarios(sizes, nodes=nodes)
+    b = msim.Batch(scs)
+    run = DiffRun(b, 6, checkpoint_every=3)
+    theta = torch.ones(b.n_roads, device="cuda")
+    theta[b.n_roads // 2 :] = 9.0
+    theta[-1] = 20.0
+    al = torch.tensor(0.01).cuda()
+    g = torch.ones(sum(sizes), 2, device="cuda")
+    pos, (expect,) = _gradients(run, theta, al, g)
+    out = torch.empty(sum(sizes), 2, device="cuda")
+    # elsewhere in an allocation, and pinned memory of the host
+    held = torch.cat([torch.zeros(3, device="cuda"), theta])
+    host = torch.empty(b.n_roads, pin_memory=True).copy_(theta)
+    for ptr in (held[3:].data_ptr(), host.data_ptr()):
+        torch.cuda.synchronize()
+        b.diff_forward(ptr, 0.01, out.data_ptr())
+        np.testing.assert_array_equal(out.cpu().numpy().view(np.uint32), pos.view(np.uint32))
+    wrong = theta.clone()
+    wrong[-1] = bad
+    t = theta.clone().requires_grad_(True)
+    a = al.clone().requires_grad_(True)
+    p = run(t, a)
+    torch.cuda.synchronize()
+    for _ in range(2):
+        with pytest.raises(msim.MsimError, match=rf"theta\[{b.n_roads - 1}\]"):
+            b.diff_forward(wrong.data_ptr(), 0.01, out.data_ptr())
+    gt, ga = torch.autograd.grad(p, (t, a), g)  # the run before is still there
+    _close(expect, (gt.double().cpu().numpy(), float(ga)))
+    b.close()
