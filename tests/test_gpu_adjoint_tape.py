@@ -73,6 +73,33 @@ def test_taped_and_replayed_gradients_agree(sizes, ticks, every, alpha, arrivals
     b2.close()
 
 
+# one launch copies a snapshot's arrays: short arrays, word remainders, and
+# arrays longer than one pass of the copying grid (2^22 words)
+@pytest.mark.parametrize("sizes,nodes", [((1,), 64), ((3,), 64), ((5, 2), 64), ((1_048_577, 31), 20_000)])
+@pytest.mark.parametrize("uniform", [False, True])
+def test_runs_start_again_from_the_initial_state(sizes, nodes, uniform):
+    scs = _scenarios(sizes, nodes=nodes)
+    if uniform:
+        for sc in scs:
+            sc.speed = None
+    n = sum(sizes)
+    b, ref = msim.Batch(scs), msim.Batch(scs)
+    ref.run_ticks(4)
+    expect = np.concatenate([ref.state(k)["pos"] for k in range(len(scs))])
+    run = DiffRun(b, 4, checkpoint_every=2)
+    theta = torch.ones(b.n_roads, device="cuda")
+    g = torch.ones(n, 2, device="cuda")
+    grads = []
+    for _ in range(3):
+        pos, (taped, replayed) = _gradients(run, theta, torch.tensor(0.0).cuda(), g, times=2)
+        np.testing.assert_array_equal(pos.view(np.uint32), expect.view(np.uint32))
+        _close(taped, replayed)
+        grads.append(taped)
+    _close(grads[0], grads[2])
+    b.close()
+    ref.close()
+
+
 # the multipliers are checked on the device, in 2^17 threads: few of them, and
 # more than one pass; the largest (its agents cross many cells a tick, and the
 # rebinning windows have to allow for that) and a bad one at the end
