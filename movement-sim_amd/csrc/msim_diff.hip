@@ -374,19 +374,103 @@ static __global__ __launch_bounds__(kBlock, 4) void k_davoid(DiffCells c, float 
 // atomic per workgroup (on one word the workgroups' atomics queue up).
 constexpr uint32_t kAlphaSlots = 64, kAlphaStride = 16;
 
-// Avoidance adjoint over the tick's binning, in binary64 from the run's
-// binary32 positions, for the listed slots: lam_out = lam + alpha * sum J dl
-// at their agents, and the alpha derivative sum lam . A.  A workgroup takes
-// GROUPS groups.  Without lists (alpha = 0: the forward run had no avoidance
-// to list them in, and lam stays as it is) only the derivative, over all
-// slots.
-template <uint32_t GROUPS>
-static __global__ __launch_bounds__(kBlock) void k_davoid_adj(DiffCells c, DiffNear near, double alpha,
-                                                       const double2* __restrict__ lam,
-                                                       double2* __restrict__ lam_out,
-                                                       double* __restrict__ galpha) {
+struct DiffMove {
+    uint32_t n;
+    const float* spd;
+    float spd_const;
+    const float* theta;
+    DiffTapeDev tp;
+    const float2* nxt_tgt;
+    const uint32_t* nxt_road;
+    uint32_t carry;
+    double* acc;
+    double* gtheta;
+};
+
+// Move adjoint of agent k, binary64 from the run's binary32 values: l is the
+// avoidance adjoint's result, returned is the λ before the move.
+// An arrival's snap is constant under frozen decisions (λ = 0).  With carry,
+// it is differentiated as if the arrival carried its leftover time onto the
+// next road (nxt_tgt, nxt_road: the decisions after this tick),
+// p' = T + (1 - L/s) s2 u2 with L = |T - p|, u2 the next road's direction and
+// s, s2 the two roads' speeds: λ = (s2/s) u (u2·λ'), ∂/∂θ[road] += v L s2/s²
+// (u2·λ'), ∂/∂θ[next road] += v (1 - L/s)(u2·λ').
+// An agent's terms for the road it is on are summed in acc and added to
+// gtheta where, going back in time, it leaves the road (its arrival, about one
+// tick in 25; k_dflush for the first road): 800k agents, one atomic each per
+// tick, took 40 us.
+template <bool UNIFORM>
+__device__ __forceinline__ double2 dmove_adj(const DiffMove& m, uint32_t k, uint8_t flag, double2 l) {
+    if (flag & kDiffNoMove) {
+        return l;
+    }
+    const float2 p = m.tp.pos[k];
+    const float2 T = m.tp.tgt[k];
+    const uint32_t r = m.tp.road[k];
+    const float v = UNIFORM ? m.spd_const : m.spd[k];
+    const double s = static_cast<double>(v * m.theta[r]);  // the run's binary32 speed
+    const double dx = static_cast<double>(T.x) - p.x;
+    const double dy = static_cast<double>(T.y) - p.y;
+    const double len = sqrt(dx * dx + dy * dy);
+    if (flag & kDiffArrived) {
+        double2 out = make_double2(0.0, 0.0);
+        const uint32_t r2 = m.nxt_road[k];
+        double on_next = m.acc[k], on_this = 0.0;
+        if (m.carry) {
+            const float2 T2 = m.nxt_tgt[k];
+            const double ex = static_cast<double>(T2.x) - T.x;
+            const double ey = static_cast<double>(T2.y) - T.y;
+            const double E = sqrt(ex * ex + ey * ey);
+            const double s2 = static_cast<double>(v * m.theta[r2]);
+            // a zero speed (theta[r] == 0) carries nothing: the frozen snap
+            if (E > 0.0 && s > 0.0) {
+                const double ux = len > 0.0 ? dx / len : 0.0;
+                const double uy = len > 0.0 ? dy / len : 0.0;
+                const double g2 = (ex / E) * l.x + (ey / E) * l.y;
+                out = make_double2(ux * (s2 / s) * g2, uy * (s2 / s) * g2);
+                on_this = static_cast<double>(v) * (len * s2 / (s * s)) * g2;
+                on_next += static_cast<double>(v) * (1.0 - len / s) * g2;
+            }
+        }
+        m.acc[k] = on_this;
+        if (on_next != 0.0) atomicAdd(&m.gtheta[r2], on_next);
+        return out;
+    }
+    const double ux = dx / len;
+    const double uy = dy / len;
+    const double ul = ux * l.x + uy * l.y;
+    const double f = s / len;
+    m.acc[k] += static_cast<double>(v) * ul;
+    return make_double2(l.x - f * (l.x - ux * ul), l.y - f * (l.y - uy * ul));
+}
+
+// One tick of the adjoint, lam -> lam_out in agent order.
+// The first near_blocks workgroups take the avoidance over the tick's binning,
+// in binary64 from the run's binary32 positions, for the listed slots, GROUPS
+// groups each: lam + alpha * sum J dl at their agents, from there the move
+// adjoint, and the alpha derivative sum lam . A.  The other workgroups take
+// the move adjoint of the agents without neighbours.  (One launch: the second
+// part fills what the first leaves idle, and lam is read once.  A gradient of
+// 2 x 1.5k agents over 40 ticks 2.40 -> 2.35 ms, of 8 x 100k over 100 16.0 ->
+// 15.0; the second part first: 2.44 and 16.5.)
+// Without lists (alpha = 0: the forward run had no avoidance to list them in)
+// the first part sums the derivative over all slots and the second takes all
+// agents.
+template <uint32_t GROUPS, bool UNIFORM>
+static __global__ __launch_bounds__(kBlock) void k_dadjoint(DiffCells c, DiffNear near, double alpha,
+                                                     uint32_t near_blocks, DiffMove mv,
+                                                     const double2* __restrict__ lam,
+                                                     double2* __restrict__ lam_out, double* __restrict__ galpha) {
     __shared__ double red[kBlock / 64];
-    const uint32_t blk = collide_order(blockIdx.x, gridDim.x);
+    if (blockIdx.x >= near_blocks) {
+        const uint32_t k = (blockIdx.x - near_blocks) * kBlock + threadIdx.x;
+        if (k < mv.n) {
+            const uint8_t flag = mv.tp.flag[k];
+            if (!(flag & kDiffNear)) lam_out[k] = dmove_adj<UNIFORM>(mv, k, flag, lam[k]);
+        }
+        return;
+    }
+    const uint32_t blk = collide_order(blockIdx.x, near_blocks);
     const uint32_t n_groups = (c.n + kNearGroup - 1u) / kNearGroup, g0 = blk * GROUPS;
     uint32_t end[GROUPS];
     uint32_t m = 0;
@@ -455,7 +539,10 @@ static __global__ __launch_bounds__(kBlock) void k_davoid_adj(DiffCells c, DiffN
         for (uint32_t k = 0; k < 4u; k++) {
             if (waiting > k) add(q[k], lj[k]);
         }
-        if (near.list) lam_out[i] = make_double2(li.x + alpha * gx, li.y + alpha * gy);
+        if (near.list) {
+            lam_out[i] = dmove_adj<UNIFORM>(mv, i, mv.tp.flag[i],
+                                            make_double2(li.x + alpha * gx, li.y + alpha * gy));
+        }
         ga += li.x * ax + li.y * ay;
     }
     if (m == 0u) {
@@ -473,76 +560,6 @@ static __global__ __launch_bounds__(kBlock) void k_davoid_adj(DiffCells c, DiffN
         for (uint32_t k = 0; k < kBlock / 64; k++) t += red[k];
         if (t != 0.0) atomicAdd(&galpha[(blk % kAlphaSlots) * kAlphaStride], t);
     }
-}
-
-// Move adjoint in agent order, binary64 from the run's binary32 values.
-// lam2 holds the avoidance adjoint's result for the agents flagged kDiffNear.
-// An arrival's snap is constant under frozen decisions (λ = 0).  With carry,
-// it is differentiated as if the arrival carried its leftover time onto the
-// next road (nxt_tgt, nxt_road: the decisions after this tick),
-// p' = T + (1 - L/s) s2 u2 with L = |T - p|, u2 the next road's direction and
-// s, s2 the two roads' speeds: λ = (s2/s) u (u2·λ'), ∂/∂θ[road] += v L s2/s²
-// (u2·λ'), ∂/∂θ[next road] += v (1 - L/s)(u2·λ').
-// An agent's terms for the road it is on are summed in acc and added to
-// gtheta where, going back in time, it leaves the road (its arrival, about one
-// tick in 25; k_dflush for the first road): 800k agents, one atomic each per
-// tick, took 40 us.
-template <bool UNIFORM>
-static __global__ __launch_bounds__(kBlock) void k_dmove_adj(uint32_t n, const float* __restrict__ spd,
-                                                      float spd_const, const float* __restrict__ theta,
-                                                      DiffTapeDev tp, const float2* __restrict__ nxt_tgt,
-                                                      const uint32_t* __restrict__ nxt_road, uint32_t carry,
-                                                      double2* __restrict__ lam, const double2* __restrict__ lam2,
-                                                      double* __restrict__ acc, double* __restrict__ gtheta) {
-    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= n) {
-        return;
-    }
-    const uint8_t flag = tp.flag[k];
-    const double2 l = (flag & kDiffNear) ? lam2[k] : lam[k];
-    if (flag & kDiffNoMove) {
-        if (flag & kDiffNear) lam[k] = l;
-        return;
-    }
-    const float2 p = tp.pos[k];
-    const float2 T = tp.tgt[k];
-    const uint32_t r = tp.road[k];
-    const float v = UNIFORM ? spd_const : spd[k];
-    const double s = static_cast<double>(v * theta[r]);  // the run's binary32 speed
-    const double dx = static_cast<double>(T.x) - p.x;
-    const double dy = static_cast<double>(T.y) - p.y;
-    const double len = sqrt(dx * dx + dy * dy);
-    if (flag & kDiffArrived) {
-        double2 out = make_double2(0.0, 0.0);
-        const uint32_t r2 = nxt_road[k];
-        double on_next = acc[k], on_this = 0.0;
-        if (carry) {
-            const float2 T2 = nxt_tgt[k];
-            const double ex = static_cast<double>(T2.x) - T.x;
-            const double ey = static_cast<double>(T2.y) - T.y;
-            const double E = sqrt(ex * ex + ey * ey);
-            const double s2 = static_cast<double>(v * theta[r2]);
-            // a zero speed (theta[r] == 0) carries nothing: the frozen snap
-            if (E > 0.0 && s > 0.0) {
-                const double ux = len > 0.0 ? dx / len : 0.0;
-                const double uy = len > 0.0 ? dy / len : 0.0;
-                const double g2 = (ex / E) * l.x + (ey / E) * l.y;
-                out = make_double2(ux * (s2 / s) * g2, uy * (s2 / s) * g2);
-                on_this = static_cast<double>(v) * (len * s2 / (s * s)) * g2;
-                on_next += static_cast<double>(v) * (1.0 - len / s) * g2;
-            }
-        }
-        lam[k] = out;
-        acc[k] = on_this;
-        if (on_next != 0.0) atomicAdd(&gtheta[r2], on_next);
-        return;
-    }
-    const double ux = dx / len;
-    const double uy = dy / len;
-    const double ul = ux * l.x + uy * l.y;
-    const double f = s / len;
-    lam[k] = make_double2(l.x - f * (l.x - ux * ul), l.y - f * (l.y - uy * ul));
-    acc[k] += static_cast<double>(v) * ul;
 }
 
 // The sums of the roads the agents start on, and the alpha derivative.
@@ -887,17 +904,29 @@ void dtick_taped(msim_batch* b, DiffState& d, uint32_t t, uint32_t j, const uint
           near_at(b, d, j));
 }
 
-// 512 slots a workgroup, so that the listed fifth of them fills its lanes
-// better (800k agents: 36 us at 256 slots, 30 at 512); small runs need the
-// workgroups (3k agents: 8.6 us at 256, 9.3 at 512).
-void launch_davoid_adj(msim_batch* b, DiffState& d, const DiffCells& c, const DiffNear& near) {
-    const double alpha = static_cast<double>(d.alpha);
-    if (b->n <= (1u << 17)) {
-        hipLaunchKernelGGL(k_davoid_adj<4>, dim3(bblocks(b->n)), dim3(kBlock), 0, b->stream, c, near, alpha, d.lam,
-                           d.lam2, d.alpha_slots);
+template <uint32_t GROUPS, bool UNIFORM>
+void launch_dadjoint_g(msim_batch* b, const DiffState& d, const DiffCells& c, const DiffNear& near,
+                       const DiffMove& mv) {
+    constexpr uint32_t kSlotsPer = GROUPS * kNearGroup;
+    const uint32_t nb = std::max(1u, (b->n + kSlotsPer - 1u) / kSlotsPer);
+    hipLaunchKernelGGL((k_dadjoint<GROUPS, UNIFORM>), dim3(nb + bblocks(b->n)), dim3(kBlock), 0, b->stream, c, near,
+                       static_cast<double>(d.alpha), nb, mv, d.lam, d.lam2, d.alpha_slots);
+}
+
+// The workgroups with the listed slots are the long ones: all of them start at
+// once (five a CU) up to 640k agents, by taking more groups each.  Gradients
+// over 30 ticks with 4, 8, 16 and 32 groups, us: 300k agents 2,127, 2,142,
+// 2,208, 2,477; 600k 3,361, 3,071, 3,093, 3,467; 1.6M 7,142, 6,435, 6,220,
+// 6,330; 3.2M 13,365, 11,862, 11,327, 11,292.
+template <bool UNIFORM>
+void launch_dadjoint(msim_batch* b, const DiffState& d, const DiffCells& c, const DiffNear& near, const DiffMove& mv) {
+    constexpr uint32_t kAtOnce = 5u * kCus;
+    if (b->n <= kAtOnce * 4u * kNearGroup) {
+        launch_dadjoint_g<4, UNIFORM>(b, d, c, near, mv);
+    } else if (b->n <= kAtOnce * 8u * kNearGroup) {
+        launch_dadjoint_g<8, UNIFORM>(b, d, c, near, mv);
     } else {
-        hipLaunchKernelGGL(k_davoid_adj<8>, dim3((bblocks(b->n) + 1u) / 2u), dim3(kBlock), 0, b->stream, c, near,
-                           alpha, d.lam, d.lam2, d.alpha_slots);
+        launch_dadjoint_g<16, UNIFORM>(b, d, c, near, mv);
     }
 }
 
@@ -1187,20 +1216,20 @@ extern "C" int msim_batch_diff_backward(msim_batch* b, const float* grad_pos, do
             const uint32_t j = t - t0;
             const DiffCells c = dcells(b, d.tp_start + static_cast<size_t>(b->start_len) * j, d.tp_bpos + (n + 2) * j,
                                        d.tp_bid + n * j);
-            launch_davoid_adj(b, d, c, d.alpha != 0.0f ? near_at(b, d, j) : DiffNear{});
             const AgentsDev a = b->agents(b->cur);
             // the decisions after tick t: the tape's next entry, or after the
             // segment's last tick the agent state its replay ended in
             const float2* nt = t + 1 < t1 ? tape_at(d.tape, n, j + 1).tgt : a.tgt;
             const uint32_t* nr = t + 1 < t1 ? tape_at(d.tape, n, j + 1).road : a.road;
-            const uint32_t carry = d.carry ? 1u : 0u;
+            const DiffMove mv{b->n, a.spd, a.spd_const, d.theta, tape_at(d.tape, n, j), nt, nr, d.carry ? 1u : 0u,
+                              d.acc, d.gtheta};
+            const DiffNear near = d.alpha != 0.0f ? near_at(b, d, j) : DiffNear{};
             if (b->uniform) {
-                hipLaunchKernelGGL(k_dmove_adj<true>, g, dim3(kBlock), 0, b->stream, b->n, a.spd, a.spd_const,
-                                   d.theta, tape_at(d.tape, n, j), nt, nr, carry, d.lam, d.lam2, d.acc, d.gtheta);
+                launch_dadjoint<true>(b, d, c, near, mv);
             } else {
-                hipLaunchKernelGGL(k_dmove_adj<false>, g, dim3(kBlock), 0, b->stream, b->n, a.spd, a.spd_const,
-                                   d.theta, tape_at(d.tape, n, j), nt, nr, carry, d.lam, d.lam2, d.acc, d.gtheta);
+                launch_dadjoint<false>(b, d, c, near, mv);
             }
+            std::swap(d.lam, d.lam2);
             rc = bcheck(b, "adjoint tick");
         }
     }

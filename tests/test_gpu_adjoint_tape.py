@@ -135,3 +135,23 @@ def test_multipliers_are_checked_on_the_device(sizes, nodes, bad):
     gt, ga = torch.autograd.grad(p, (t, a), g)  # the run before is still there
     _close(expect, (gt.double().cpu().numpy(), float(ga)))
     b.close()
+
+
+# a tick of the adjoint takes 4, 8 or 16 groups of 64 slots a workgroup
+@pytest.mark.parametrize("agents", [326_980, 326_981, 654_660, 654_661])
+def test_group_counts_of_the_adjoint_agree(agents):
+    scs = _scenarios((agents, 700), nodes=40_000)
+    alone = _scenarios((1, 700), nodes=40_000)[1:]
+    # the second scenario alone runs with the smallest count
+    grads = []
+    for maps in (scs, alone):
+        b = msim.Batch(maps)
+        n, first = sum(sc.entities.shape[0] for sc in maps), b.n_roads - maps[-1].roads.shape[0]
+        g = torch.zeros(n, 2, device="cuda")
+        g[-700:] = torch.randn(700, 2, generator=torch.Generator().manual_seed(9)).cuda()
+        theta = torch.ones(b.n_roads, device="cuda")
+        _, (got,) = _gradients(DiffRun(b, 8, checkpoint_every=4), theta, torch.tensor(0.03).cuda(), g)
+        assert not got[0][:first].any()
+        grads.append((got[0][first:], got[1]))
+        b.close()
+    _close(grads[1], grads[0])
