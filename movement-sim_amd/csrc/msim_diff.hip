@@ -302,9 +302,10 @@ struct PushVisitor {
 // from p only for p = -0).
 // (One slot per lane: with two, 110 registers and half the waves, 800k agents
 // took 41 us against 28; a lane walking its cells in global memory, without
-// staging, 33.)
+// staging, 33.  Seven waves a SIMD instead of six, 69 registers: a gradient of
+// 800k agents over 100 ticks 15.07 -> 14.87 ms; eight spill.)
 template <int P>
-static __global__ __launch_bounds__(kBlock, 4) void k_davoid(DiffCells c, float alpha, float2* __restrict__ pos,
+static __global__ __launch_bounds__(kBlock, 7) void k_davoid(DiffCells c, float alpha, float2* __restrict__ pos,
                                                              DiffNear near, unsigned int* __restrict__ faults) {
     __shared__ float2 stage_all[kBlock / 64 * kStage];
     const uint32_t blk = collide_order(blockIdx.x, gridDim.x);
@@ -917,7 +918,8 @@ void launch_dadjoint_g(msim_batch* b, const DiffState& d, const DiffCells& c, co
 // once (five a CU) up to 640k agents, by taking more groups each.  Gradients
 // over 30 ticks with 4, 8, 16 and 32 groups, us: 300k agents 2,127, 2,142,
 // 2,208, 2,477; 600k 3,361, 3,071, 3,093, 3,467; 1.6M 7,142, 6,435, 6,220,
-// 6,330; 3.2M 13,365, 11,862, 11,327, 11,292.
+// 6,330; 3.2M 13,365, 11,862, 11,327, 11,292.  (Six workgroups a CU, by
+// spilling: 800k agents over 100 ticks 14.9 -> 15.2 ms.)
 template <bool UNIFORM>
 void launch_dadjoint(msim_batch* b, const DiffState& d, const DiffCells& c, const DiffNear& near, const DiffMove& mv) {
     constexpr uint32_t kAtOnce = 5u * kCus;
