@@ -48,7 +48,8 @@ void blaunch_sorted(msim_batch* b, const SortedMove& mv, const BatchBin& bb, boo
     if (!mv.cur.seg) {
         bprobe_pre(b);
         hipLaunchKernelGGL(k_seg_scan<kBScanThreads>, dim3(1), dim3(kBScanThreads), 0, b->stream,
-                           b->seg_cnt[b->cur], b->seg_group[b->cur], b->seg_start, b->n_seg, b->n, b->faults);
+                           b->seg_cnt[b->cur], b->seg_group[b->cur], seg_group_words(b->n_seg), b->seg_start,
+                           b->n_seg, b->n, b->faults);
         bprobe_post(b);
     }
     const uint32_t extra = finish ? bfinish_blocks(b, T) : 0u;
@@ -216,7 +217,8 @@ int benter_sorted(msim_batch* b) {
     const dim3 gs((b->n_seg + kBlock - 1) / kBlock);
     for (int k = 0; k < 2; k++) {
         hipLaunchKernelGGL(k_fill_u32, gs, dim3(kBlock), 0, b->stream, b->seg_cnt[k], 0u, b->n_seg);
-        hipLaunchKernelGGL(k_fill_u32, gs, dim3(kBlock), 0, b->stream, b->seg_group[k], 0u, seg_groups(b->n_seg));
+        const uint32_t words = seg_group_words(b->n_seg);
+        hipLaunchKernelGGL(k_fill_u32, dim3(bblocks(words)), dim3(kBlock), 0, b->stream, b->seg_group[k], 0u, words);
     }
     if (b->uniform) {
         hipLaunchKernelGGL(k_bsorted_next<true>, g, dim3(kBlock), 0, b->stream, bsorted_bufs(b, b->cur), b->blk_scen,
@@ -536,8 +538,8 @@ extern "C" int msim_batch_create(uint32_t n_scen, const uint32_t* road_off, cons
         BALLOC(b->seg_start, b->n_seg + 1);
         BALLOC(b->seg_cnt[0], b->n_seg);
         BALLOC(b->seg_cnt[1], b->n_seg);
-        BALLOC(b->seg_group[0], seg_groups(b->n_seg));
-        BALLOC(b->seg_group[1], seg_groups(b->n_seg));
+        BALLOC(b->seg_group[0], seg_group_words(b->n_seg));
+        BALLOC(b->seg_group[1], seg_group_words(b->n_seg));
         BALLOC(b->seg_arr, b->n_seg);
     }
     BALLOC(b->part, static_cast<size_t>(n_scen) * kScenSlots * kScenSlotStride);

@@ -450,7 +450,7 @@ struct msim_batch {
     float* arr_spd = nullptr;               // [n] their speeds (per-agent speeds only)
     uint32_t* seg_start = nullptr;          // [n_seg + 1] first slot of each segment (k_seg_scan)
     uint32_t* seg_cnt[2] = {nullptr, nullptr};  // per buffer: agents per segment for the move leaving it
-    uint32_t* seg_group[2] = {nullptr, nullptr};  // and per kGroupSegs segments
+    uint32_t* seg_group[2] = {nullptr, nullptr};  // and per group of segments
     bool finish_pending = false;  // run_ticks: the last tick's pair totals are folded by the next move
     uint32_t* seg_arr = nullptr;            // [n_seg] arrivals of each segment
     uint32_t bin_unroll = 4;  // window slots per rebinning thread and load round
@@ -626,7 +626,9 @@ inline GridDev bgrid(const msim_batch* b) {
     return g;
 }
 
-inline SegCounts bseg_counts(const msim_batch* b, int k) { return SegCounts{b->seg_cnt[k], b->seg_group[k]}; }
+inline SegCounts bseg_counts(const msim_batch* b, int k) {
+    return SegCounts{b->seg_cnt[k], b->seg_group[k], seg_group_log2(b->n_seg)};
+}
 
 inline BatchFinish bfinish_args(const msim_batch* b) { return BatchFinish{b->part, b->totals, b->last, b->n_scen}; }
 

@@ -90,6 +90,23 @@ inline uint32_t auto_batch_segment_log2(uint64_t buckets, uint32_t tlog, uint32_
 // with 4.
 inline uint32_t auto_bin_unroll(uint32_t seg_log) { return seg_log == 12u || seg_log == 13u ? 8u : 4u; }
 
+// Sums of the sorted state's per-segment counts, over groups of 2^l
+// consecutive segments: every move workgroup adds up the groups before its own
+// segment's and the segments before it in its group, so l is about half of
+// log2(n_seg) (at least 4) and neither has more than about sqrt(n_seg) words
+// (2^17 segments: 512 + 255; groups of 16 would be 8,192).
+constexpr uint32_t seg_group_log2(uint32_t n_seg) {
+    uint32_t l = 0;
+    while (l < 31u && (1u << l) < n_seg) l++;
+    return l > 8u ? l / 2u : 4u;
+}
+// Words from one group's sum to the next.  Side by side, 32 sums share a cache
+// line, to which every workgroup then adds: see SegCounts.
+constexpr uint32_t kGroupStride = 8;
+constexpr uint32_t seg_group_words(uint32_t n_seg) {
+    return ((n_seg + (1u << seg_group_log2(n_seg)) - 1u) >> seg_group_log2(n_seg)) * kGroupStride;
+}
+
 // Bounding box of the roads and agents.
 struct Extent {
     float x0 = 0.0f, x1 = 0.0f, y0 = 0.0f, y1 = 0.0f;

@@ -80,7 +80,7 @@ struct msim_sim {
     float* arr_spd = nullptr;               // [n] their speeds (per-agent speeds only)
     uint32_t* seg_start = nullptr;          // [n_seg + 1] first slot of each segment (k_seg_scan)
     uint32_t* seg_cnt[2] = {nullptr, nullptr};  // per buffer: agents per segment for the move leaving it
-    uint32_t* seg_group[2] = {nullptr, nullptr};  // and per kGroupSegs segments
+    uint32_t* seg_group[2] = {nullptr, nullptr};  // and per group of segments
     bool lists = false;  // agents that will leave their segment are listed (SegLists)
     SegLists leave[2] = {};  // per buffer, for the move leaving it
     bool finish_pending = false;  // run_ticks: the last tick's statistics are folded by the next move
@@ -566,8 +566,9 @@ SortedBufs sorted_bufs(const msim_sim* s, int k) {
     return SortedBufs{b.pos, s->rec[k], s->nxt[k], b.dir};
 }
 
-SegCounts seg_counts(const msim_sim* s, int k) { return SegCounts{s->seg_cnt[k], s->seg_group[k]}; }
-
+SegCounts seg_counts(const msim_sim* s, int k) {
+    return SegCounts{s->seg_cnt[k], s->seg_group[k], seg_group_log2(s->n_seg)};
+}
 
 
 // Enters the sorted state from the classic layout: renumbers the agents into
@@ -587,7 +588,9 @@ int enter_sorted(msim_sim* s) {
     const dim3 gs((s->n_seg + kBlock - 1) / kBlock);
     for (int k = 0; k < 2; k++) {
         hipLaunchKernelGGL(k_fill_u32, gs, dim3(kBlock), 0, s->stream, s->seg_cnt[k], 0u, s->n_seg);
-        hipLaunchKernelGGL(k_fill_u32, gs, dim3(kBlock), 0, s->stream, s->seg_group[k], 0u, seg_groups(s->n_seg));
+        const uint32_t words = seg_group_words(s->n_seg);
+        hipLaunchKernelGGL(k_fill_u32, dim3(agent_blocks(words)), dim3(kBlock), 0, s->stream, s->seg_group[k], 0u,
+                           words);
     }
     if (s->lists) {
         hipLaunchKernelGGL(k_seg_records, gs, dim3(kBlock), 0, s->stream, s->leave[s->cur], s->bstart[s->bcur],
@@ -624,7 +627,8 @@ void launch_sorted(msim_sim* s, const SortedMove& mv, const BinDev& b, const Tic
     if (!mv.cur.seg) {
         probe_pre(s);
         hipLaunchKernelGGL(k_seg_scan<kScanThreads>, dim3(1), dim3(kScanThreads), 0, s->stream, s->seg_cnt[s->cur],
-                           s->seg_group[s->cur], s->seg_start, s->n_seg, s->n, &s->ctr->faults);
+                           s->seg_group[s->cur], seg_group_words(s->n_seg), s->seg_start, s->n_seg, s->n,
+                           &s->ctr->faults);
         probe_post(s);
     }
     probe_pre(s);
@@ -1101,8 +1105,8 @@ extern "C" int msim_create(const msim_road* roads, uint32_t n_roads, const uint3
         ALLOC(s->seg_start, s->n_seg + 1);
         ALLOC(s->seg_cnt[0], s->n_seg);
         ALLOC(s->seg_cnt[1], s->n_seg);
-        ALLOC(s->seg_group[0], seg_groups(s->n_seg));
-        ALLOC(s->seg_group[1], seg_groups(s->n_seg));
+        ALLOC(s->seg_group[0], seg_group_words(s->n_seg));
+        ALLOC(s->seg_group[1], seg_group_words(s->n_seg));
         // Lists reach the two neighbouring segments only.  They replace the
         // margins on both sides of a window, so they pay where the margins
         // add a quarter or more to it: move of 8M agents (margin 0.38 of a

@@ -20,7 +20,7 @@
 //     previous slot order, the segment and the margin on both sides;
 //   * the segment's first slot follows from counts made before the launch:
 //     the previous move and route choice counted, per segment and per group
-//     of kGroupSegs segments, the agents whose next bucket lies in it, so no
+//     of segments (SegCounts), the agents whose next bucket lies in it, so no
 //     segment waits for another.  Inside run_ticks every workgroup sums the
 //     counts before its segment itself; a single dispatch runs k_seg_scan
 //     first;
@@ -45,6 +45,7 @@
 #pragma once
 
 #include "msim_bin.hpp"
+#include "msim_host.hpp"
 
 namespace msim {
 
@@ -101,23 +102,39 @@ __device__ __forceinline__ uint4 hot_record(float2 tgt, float spd, uint32_t call
 __device__ __forceinline__ uint4 cold_word(uint32_t road, uint2 c) { return make_uint4(road, c.x, c.y, 0u); }
 
 // Agents whose next bucket lies in each segment, and the sums of those
-// counts over groups of kGroupSegs consecutive segments: a segment's first
-// slot is then the sum of the groups before its own and of at most
-// kGroupSegs - 1 segments, which the workgroup of the segment adds up while
-// its window is in flight (12,000 segments: 750 + 15 words).  Larger groups
-// would put more of the workgroups' atomics on one word.
-constexpr uint32_t kGroupLog = 4, kGroupSegs = 1u << kGroupLog;
-__host__ __device__ constexpr uint32_t seg_groups(uint32_t n_seg) { return (n_seg + kGroupSegs - 1u) >> kGroupLog; }
+// counts over groups of 2^log consecutive segments (seg_group_log2): a
+// segment's first slot is then the sum of the groups before its own and of the
+// segments before it in its group, which the workgroup of the segment adds up
+// while its window is in flight.
+// The groups' words are bound by the atomics that meet in one cache line, some
+// 6 ns each: a workgroup adds to its segment and its neighbours, which are
+// mostly of one group, so it adds their sum at once (leave_flush, next_flush),
+// and the words lie kGroupStride apart.  Ticks of 1M agents, us, each count
+// added to its group by itself and the words side by side -> as here: 512
+// segments 48 -> 41, 1,024 66 -> 48, 2,048 84 -> 64; 100k agents on 256
+// segments 39 -> 22; without the sums over groups at all 40, 47, 63, 21.
 struct SegCounts {
     uint32_t* seg;    // [n_seg]
-    uint32_t* group;  // [seg_groups(n_seg)]
+    uint32_t* group;  // [seg_group_words(n_seg)]
+    uint32_t log;
+    __device__ void add_seg(uint32_t g, uint32_t v) const { atomicAdd(&seg[g], v); }
+    __device__ void add_group(uint32_t gg, uint32_t v) const { atomicAdd(&group[gg * kGroupStride], v); }
     __device__ void add(uint32_t g, uint32_t v) const {
-        atomicAdd(&seg[g], v);
-        atomicAdd(&group[g >> kGroupLog], v);
+        add_seg(g, v);
+        add_group(g >> log, v);
     }
     __device__ void clear(uint32_t g) const {
         seg[g] = 0u;
-        if ((g & (kGroupSegs - 1u)) == 0u) group[g >> kGroupLog] = 0u;
+        if ((g & ((1u << log) - 1u)) == 0u) group[(g >> log) * kGroupStride] = 0u;
+    }
+    // Thread tid's part of the counts before segment g (summed over the
+    // workgroup's threads).
+    __device__ uint32_t before(uint32_t g, uint32_t tid, uint32_t threads) const {
+        const uint32_t gg = g >> log;
+        uint32_t v = 0;
+        for (uint32_t k = tid; k < gg; k += threads) v += group[k * kGroupStride];
+        for (uint32_t k = (gg << log) + tid; k < g; k += threads) v += seg[k];
+        return v;
     }
 };
 
@@ -194,11 +211,25 @@ __device__ __forceinline__ void next_add(const NextCount& nc, uint32_t bucket, b
 // Workgroup-level, after a barrier: nh into the global counts.
 __device__ __forceinline__ void next_flush(const NextCount& nc) {
     const int k = static_cast<int>(threadIdx.x);
-    if (k < 2 * kNextReach + 1 && nc.nh[k]) {
-        const int nl = static_cast<int>(nc.n_local);
-        const int l = ((static_cast<int>(nc.g_local) + k - kNextReach) % nl + nl) % nl;
-        nc.next.add(nc.seg_first + static_cast<uint32_t>(l), nc.nh[k]);
+    if (k >= 2 * kNextReach + 1) {
+        return;
     }
+    const int nl = static_cast<int>(nc.n_local);
+    auto segment = [&](int j) {
+        const int l = ((static_cast<int>(nc.g_local) + j - kNextReach) % nl + nl) % nl;
+        return nc.seg_first + static_cast<uint32_t>(l);
+    };
+    const uint32_t g = segment(k), gg = g >> nc.next.log;
+    if (nc.nh[k]) nc.next.add_seg(g, nc.nh[k]);
+    uint32_t sum = 0;  // of the counts in g's group, added by the first of them
+    bool first = true;
+    for (int j = 0; j < 2 * kNextReach + 1; j++) {
+        if (segment(j) >> nc.next.log == gg) {
+            sum += nc.nh[j];
+            first = first && j >= k;
+        }
+    }
+    if (first && sum) nc.next.add_group(gg, sum);
 }
 
 // The agents that may land in a segment, numbered from 0: old slots [a0, a1),
@@ -311,10 +342,22 @@ __device__ __forceinline__ void leave_round(const Leavers& lv, const uint32_t (&
 // and n1 (down); the rest stay.
 __device__ __forceinline__ void leave_flush(const Leavers& lv, const SegCounts& next, uint32_t seg_first,
                                             uint32_t placed, uint32_t n0, uint32_t n1) {
-    const uint32_t up = lv.n[0] - n0, down = lv.n[1] - n1;
-    if (threadIdx.x == 0u && placed != up + down) next.add(seg_first + lv.g, placed - up - down);
-    if (threadIdx.x == 1u && up) next.add(seg_first + lv.above, up);
-    if (threadIdx.x == 2u && down) next.add(seg_first + lv.below, down);
+    const uint32_t up = lv.n[0] - n0, down = lv.n[1] - n1, stay = placed - up - down;
+    const uint32_t own = (seg_first + lv.g) >> next.log, above = (seg_first + lv.above) >> next.log,
+                   below = (seg_first + lv.below) >> next.log;
+    if (threadIdx.x == 0u) {  // its group's sum takes the neighbours of the same group along
+        const uint32_t sum = stay + (above == own ? up : 0u) + (below == own ? down : 0u);
+        if (stay) next.add_seg(seg_first + lv.g, stay);
+        if (sum) next.add_group(own, sum);
+    }
+    if (threadIdx.x == 1u && up) {
+        next.add_seg(seg_first + lv.above, up);
+        if (above != own) next.add_group(above, up);
+    }
+    if (threadIdx.x == 2u && down) {
+        next.add_seg(seg_first + lv.below, down);
+        if (below != own) next.add_group(below, down);
+    }
 }
 
 __device__ __forceinline__ Leavers leavers_of(const SortedMove& mv, const NextCount& nc, uint32_t base, uint32_t end) {
@@ -585,9 +628,7 @@ __device__ __forceinline__ void sorted_segment(const SortedMove& mv, const Table
     // the counts before the segment, or its scanned slots: loaded while the window is counted
     uint32_t before = 0, st0 = 0, st1 = 0;
     if (mv.cur.seg) {
-        const uint32_t gg = g >> kGroupLog, in = (gg << kGroupLog) + tid;
-        for (uint32_t k = tid; k < gg; k += T) before += mv.cur.group[k];
-        if (in < g) before += mv.cur.seg[in];  // in < g leaves tid < kGroupSegs
+        before = mv.cur.before(g, tid, T);
         st1 = mv.cur.seg[g];
     } else {
         st0 = mv.seg_start[g];
@@ -778,8 +819,8 @@ static __global__ __launch_bounds__(T) void k_move_sorted(SortedMove mv, BinDev 
 // per lane) and kept in registers for both the chunk sum and the offsets.
 template <uint32_t T>
 static __global__ __launch_bounds__(T) void k_seg_scan(uint32_t* __restrict__ cnt, uint32_t* __restrict__ group,
-                                                       uint32_t* __restrict__ seg_start, uint32_t n_seg, uint32_t n,
-                                                       unsigned int* faults) {
+                                                       uint32_t group_words, uint32_t* __restrict__ seg_start,
+                                                       uint32_t n_seg, uint32_t n, unsigned int* faults) {
     constexpr uint32_t W = T / 64, K = 16;
     __shared__ uint32_t wsum[W];
     const uint32_t lane = __lane_id(), w = threadIdx.x >> 6;
@@ -826,7 +867,7 @@ static __global__ __launch_bounds__(T) void k_seg_scan(uint32_t* __restrict__ cn
             run += static_cast<uint32_t>(__shfl(static_cast<int>(inc), 63, 64));
         }
     }
-    for (uint32_t k = threadIdx.x; k < seg_groups(n_seg); k += T) {
+    for (uint32_t k = threadIdx.x; k < group_words; k += T) {
         group[k] = 0u;
     }
     if (threadIdx.x == 0) {
