@@ -453,7 +453,7 @@ extern "C" int msim_batch_create(uint32_t n_scen, const uint32_t* road_off, cons
         smax = 0.0f;
         for (uint32_t i = 0; i < n; i++) smax = std::max(smax, speed[i]);
     }
-    const uint32_t D = static_cast<uint32_t>(std::floor(smax * (1.0f + 1.0f / 1048576.0f) / cell)) + 1u;
+    const uint32_t reach = cell_reach(smax, cell);
     uint64_t buckets = 0;
     for (uint32_t s = 0; s < n_scen; s++) {
         ScenDev& d = sc[s];
@@ -470,7 +470,7 @@ extern "C" int msim_batch_create(uint32_t n_scen, const uint32_t* road_off, cons
         d.m = 1u << tlog;
         d.wmask = (1u << d.lw) - 1u;
         d.hmask = (1u << (tlog - d.lw)) - 1u;
-        d.margin = (D + 1u) * (d.wmask + 1u) + D;
+        d.margin = (reach + 1u) * (d.wmask + 1u) + reach;
         buckets += d.m;
     }
     for (uint32_t s = 0; s < n_scen; s++) {

@@ -50,20 +50,50 @@ inline uint32_t auto_width_log2(uint32_t tlog, uint32_t rows_log) {
     return l;
 }
 
-// Segment owned by one rebinning workgroup: about 128 segments of 2^9 to
-// 2^11 buckets (2^12 in tables of 2^22 and more), or two table rows where
-// those are longer (a window adds one to three rows on both sides), up to
-// 2^14 buckets (64 KB of LDS counters).  Ticks of the classic layout, us: 1M
-// agents on 2^20 buckets in rows of 2^10: 61.5 at 2^12, 62.5 at 2^11, 74 at
-// 2^10, 71 at 2^13; in rows of 2^11, 88 at 2^14 (64 segments, most CUs idle)
-// against 73; in rows of 2^7, 56 at 2^11, 58 at 2^12; 123k agents on 2^17: 33
-// at 2^9 and 2^10, 34 at 2^11, 39 at 2^12.
-inline uint32_t auto_segment_log2(uint32_t tlog, uint32_t lw) {
-    uint32_t l = tlog > 21u ? 12u : (tlog > 18u ? 11u : (tlog > 16u ? tlog - 7u : 9u));
+// Segment sizes: two table rows at least (a window adds reach + 1 rows on
+// both sides), up to 2^14 buckets (64 KB of LDS counters).
+inline uint32_t segment_in_bounds(uint32_t l, uint32_t tlog, uint32_t lw) {
     if (l < lw + 1u) l = lw + 1u;
     if (l > 14) l = 14;
-    if (l > tlog) l = tlog;
-    return l;
+    return l > tlog ? tlog : l;
+}
+
+// Segment owned by one rebinning workgroup of the classic layouts (reach:
+// cells an agent moves at most in a tick, plus one; look_back: binning 2):
+// 16 table rows, against which the rows a window adds are few, but of small
+// tables about 128 segments, so that the CUs have work; where a window adds
+// two rows a side (reach 1) fewer rows do.  Ticks, us:
+//   two passes, reach 1: 2^22 buckets in rows of 2^11, 2.2M agents, 116 at
+//     2^14, 127 at 2^13, 133 at 2^12; 2^21, rows of 2^10, 1.1M agents, 79, 71,
+//     66 and 70 at 2^11; 2^20, rows of 2^10, 1M agents, 115, 104, 85, 81;
+//   reach 2: 2^23, rows of 2^10, 4.3M agents, 233, 248, 263; 2^21, rows of
+//     2^9, 2M agents, 120, 105, 109, 132; 2^20, rows of 2^9, 1M agents, 88,
+//     69, 61, 72; 2^20, rows of 2^5, 94 at 2^12, 73 at 2^11, 63 at 2^9;
+//     123k agents on 2^17, 39 at 2^12, 34 at 2^11, 33 at 2^10 and 2^9;
+//   look-back: 2^23, rows of 2^10, 216 at 2^14, 235 at 2^12; 2^20, rows of
+//     2^9, reach 1, 61 at 2^12, 64 at 2^11; 2^19, rows of 2^6, 300k agents, 38
+//     at 2^11, 44 at 2^10.
+inline uint32_t auto_segment_log2(uint32_t tlog, uint32_t lw, uint32_t reach, bool look_back) {
+    uint32_t most = 9;
+    if (tlog >= 22u) most = 14;
+    else if (tlog == 21u) most = reach < 2u ? 12u : 14u;
+    else if (tlog == 20u) most = reach < 2u && !look_back ? 11u : 12u;
+    else if (tlog > 16u) most = tlog > 18u ? 11u : tlog - 7u;
+    // a look-back chain of many small segments is slow
+    const uint32_t least = tlog > 20u ? 10u : (look_back ? (most < 11u ? most : 11u) : 9u);
+    uint32_t l = lw + 4u;
+    if (l > most) l = most;
+    if (l < least) l = least;
+    return segment_in_bounds(l, tlog, lw);
+}
+
+// The same for the sorted state: about 128 segments of 2^9 to 2^11 buckets
+// (2^12 in tables of 2^22 and more).  Ticks of 1.6M agents on 2^21 buckets in
+// rows of 2^8, us: 89 at 2^14, 62 at 2^13, 61 at 2^12 and 2^11, 72 at 2^10; 9M
+// on 2^24 in rows of 2^11: 433, 341, 348, 432, 1,199; 300k on 2^19 in rows of
+// 2^8: 66, 40, 28, 24, 28.
+inline uint32_t auto_sorted_segment_log2(uint32_t tlog, uint32_t lw) {
+    return segment_in_bounds(tlog > 21u ? 12u : (tlog > 18u ? 11u : (tlog > 16u ? tlog - 7u : 9u)), tlog, lw);
 }
 
 // The same for one of many tables in a launch, of `buckets` in all, whose
@@ -75,10 +105,13 @@ inline uint32_t auto_segment_log2(uint32_t tlog, uint32_t lw) {
 inline uint32_t auto_batch_segment_log2(uint64_t buckets, uint32_t tlog, uint32_t lw) {
     uint32_t l = 11;
     while (l > 9 && (buckets >> l) < 384u) l--;
-    if (l < lw + 1u) l = lw + 1u;
-    if (l > 14) l = 14;
-    if (l > tlog) l = tlog;
-    return l;
+    return segment_in_bounds(l, tlog, lw);
+}
+
+// Cells an agent of at most this speed moves per axis and tick at most, plus
+// one (the heading has |dir| = speed up to rounding).
+inline uint32_t cell_reach(float max_speed, float cell) {
+    return static_cast<uint32_t>(std::floor(max_speed * (1.0f + 1.0f / 1048576.0f) / cell)) + 1u;
 }
 
 // Window slots each rebinning thread loads per round.  Segments of up to 2^11

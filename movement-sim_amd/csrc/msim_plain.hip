@@ -977,7 +977,15 @@ extern "C" int msim_create(const msim_road* roads, uint32_t n_roads, const uint3
     if (lw < 2 || lw + 2 > tlog) {
         return fail(nullptr, MSIM_ERR_INVALID, "table_width_log2 must be in [2, table_log2 - 2]");
     }
-    const uint32_t seg_log = o.segment_log2 ? o.segment_log2 : auto_segment_log2(tlog, lw);
+    float smax = kShaderSpeed;
+    if (speed) {
+        smax = 0.0f;
+        for (uint32_t i = 0; i < n_entities; i++) smax = std::max(smax, speed[i]);
+    }
+    const uint32_t reach = cell_reach(smax, cell);
+    const uint32_t auto_seg =
+        o.binning == 3 ? auto_sorted_segment_log2(tlog, lw) : auto_segment_log2(tlog, lw, reach, o.binning == 2);
+    const uint32_t seg_log = o.segment_log2 ? o.segment_log2 : auto_seg;
     if (seg_log < 9 || seg_log > 14 || seg_log > tlog) {
         return fail(nullptr, MSIM_ERR_INVALID, "segment_log2 must be in [9, 14] and <= table_log2");
     }
@@ -1055,16 +1063,9 @@ extern "C" int msim_create(const msim_road* roads, uint32_t n_roads, const uint3
     s->seg_log = seg_use;
     s->n_seg = g.m >> seg_use;
     s->bin_unroll = o.binning == 3 ? sorted_unroll : (o.bin_unroll ? o.bin_unroll : auto_bin_unroll(seg_use));
-    // An agent moves at most max_speed per axis per tick (the heading has
-    // |dir| = speed up to rounding), i.e. at most D cells; in linear bucket
-    // order that is at most (D + 1) rows plus D columns.
-    float smax = kShaderSpeed;
-    if (speed) {
-        smax = 0.0f;
-        for (uint32_t i = 0; i < n_entities; i++) smax = std::max(smax, speed[i]);
-    }
-    const uint32_t D = static_cast<uint32_t>(std::floor(smax * (1.0f + 1.0f / 1048576.0f) / cell)) + 1u;
-    s->margin = (D + 1u) * (g.wmask + 1u) + D;
+    // An agent moves at most `reach` cells per axis and tick; in linear bucket
+    // order that is at most reach + 1 rows plus reach columns.
+    s->margin = (reach + 1u) * (g.wmask + 1u) + reach;
 
     const size_t n_adv = (static_cast<size_t>(n) + kAdv - 1) / kAdv * kAdv;
 #define ALLOC(p, cnt)                                   \
