@@ -441,6 +441,7 @@ extern "C" int msim_batch_create(uint32_t n_scen, const uint32_t* road_off, cons
         return bfail(nullptr, MSIM_ERR_HIP, "hipStreamCreate failed");
     }
     (void)hipGetDevice(&b->device);
+    b->readback.on(b->device, b->stream);
     int lds_max = 65536;
     (void)hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, b->device);
 

@@ -1033,6 +1033,8 @@ extern "C" int msim_create(const msim_road* roads, uint32_t n_roads, const uint3
         return fail(nullptr, MSIM_ERR_HIP, "hipStreamCreate failed");
     }
 
+    s->readback.on(s->device, s->stream);
+
     // LDS per workgroup bounds the segment size (4 bytes per bucket counter).
     int lds_max = 65536;
     (void)hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, s->device);
@@ -1299,7 +1301,7 @@ namespace {
 template <class Ready>
 int read_parts(msim_sim* s, const std::vector<ReadPart>& parts, Ready&& ready) {
     hipError_t e = hipSuccess;
-    const int rc = s->readback.read(s->device, s->stream, parts, s->watchdog_ms, &e, ready);
+    const int rc = s->readback.read(parts, s->watchdog_ms, &e, ready);
     if (rc >= 0) return rc;
     if (e == hipErrorNotReady) {
         return fail(s, MSIM_ERR_TIMEOUT, "readback did not finish within %u ms", s->watchdog_ms);

@@ -81,8 +81,34 @@ hipError_t bounded_wait(uint32_t watchdog_ms, Busy&& busy) {
     }
 }
 
+// Makes a device the calling thread's current one, for as long as it lives.
+// Events, pinned memory and the null stream belong to the device that is
+// current, which need not be the handle's.
+class DeviceScope {
+public:
+    explicit DeviceScope(int device) {
+        if (hipGetDevice(&before_) != hipSuccess) before_ = device;
+        if (before_ != device) (void)hipSetDevice(device);
+        device_ = device;
+    }
+    ~DeviceScope() {
+        if (before_ != device_) (void)hipSetDevice(before_);
+    }
+    DeviceScope(const DeviceScope&) = delete;
+    DeviceScope& operator=(const DeviceScope&) = delete;
+
+private:
+    int before_ = 0, device_ = 0;
+};
+
 class ReadBack {
 public:
+    // The handle's device and stream.
+    void on(int device, hipStream_t stream) {
+        device_ = device;
+        stream_ = stream;
+    }
+
     // 64 MB of entities, two slots a thread, ms: slots of 0.5 MB 3.2 (every
     // transfer has a fixed cost), 1 MB 2.3, 2 MB 1.9, 4 MB 2.0; 4 threads 1.97,
     // 6 1.91, 8 1.94.
@@ -90,7 +116,10 @@ public:
 
     // Pinned memory that kernels may write `bytes` of results to directly
     // (null past one slot): no transfer follows the kernel.
-    void* small(size_t bytes) { return bytes <= kSlot && reserve(1) ? slots_ : nullptr; }
+    void* small(size_t bytes) {
+        const DeviceScope scope(device_);
+        return bytes <= kSlot && reserve(1) ? slots_ : nullptr;
+    }
     static constexpr uint32_t kThreads = 6;
 
     ReadBack() = default;
@@ -108,8 +137,8 @@ public:
     // returns 0, or a code that is passed on.  Otherwise returns 0, or -1 with
     // *err set (hipErrorNotReady: the watchdog expired).
     template <class Ready>
-    int read(int device, hipStream_t stream, const std::vector<ReadPart>& parts, uint32_t watchdog_ms, hipError_t* err,
-             Ready&& ready) {
+    int read(const std::vector<ReadPart>& parts, uint32_t watchdog_ms, hipError_t* err, Ready&& ready) {
+        const DeviceScope scope(device_);
         size_t total = 0;
         bool there = !parts.empty();
         for (const ReadPart& p : parts) {
@@ -125,11 +154,11 @@ public:
             return rc;
         }
         if (total <= kSlot) {  // everything through one slot, one wait
-            if (!reserve(1)) return direct(stream, parts, err, ready);
+            if (!reserve(1)) return direct(parts, err, ready);
             size_t at = 0;
             for (const ReadPart& p : parts) {
                 if (!p.bytes) continue;
-                *err = hipMemcpyAsync(slots_ + at, p.src, p.bytes, hipMemcpyDeviceToHost, stream);
+                *err = hipMemcpyAsync(slots_ + at, p.src, p.bytes, hipMemcpyDeviceToHost, stream_);
                 if (*err != hipSuccess) return -1;
                 at += (p.bytes + 255) / 256 * 256;
             }
@@ -145,7 +174,7 @@ public:
         }
         // one thread per slot's worth, two slots each
         const uint32_t n = static_cast<uint32_t>(std::min<size_t>(kThreads, std::max<size_t>(1, total / kSlot)));
-        if (!reserve(2 * n)) return direct(stream, parts, err, ready);
+        if (!reserve(2 * n)) return direct(parts, err, ready);
         const int rc = ready();
         if (rc) return rc;
         std::vector<Piece> pieces;
@@ -158,7 +187,7 @@ public:
         std::atomic<size_t> next{0};
         std::atomic<int> fault{static_cast<int>(hipSuccess)};
         auto work = [&](uint32_t t) {
-            if (t) (void)hipSetDevice(device);  // a new thread starts on device 0
+            if (t) (void)hipSetDevice(device_);  // a new thread starts on device 0
             Piece held[2] = {};
             int in = 0;
             for (;;) {
@@ -168,8 +197,8 @@ public:
                 hipError_t e = hipSuccess;
                 if (k < pieces.size() && fault.load() == hipSuccess) {
                     mine = pieces[k];
-                    e = hipMemcpyAsync(slot(2 * t + in), mine.src, mine.bytes, hipMemcpyDeviceToHost, stream);
-                    if (e == hipSuccess) e = hipEventRecord(events_[2 * t + in], stream);
+                    e = hipMemcpyAsync(slot(2 * t + in), mine.src, mine.bytes, hipMemcpyDeviceToHost, stream_);
+                    if (e == hipSuccess) e = hipEventRecord(events_[2 * t + in], stream_);
                 }
                 in ^= 1;
                 const Piece& old = held[in];  // copied out while the new one is on its way
@@ -191,7 +220,7 @@ public:
         for (std::thread& h : helpers) h.join();
         *err = static_cast<hipError_t>(fault.load());
         if (*err != hipSuccess) {
-            (void)hipStreamSynchronize(stream);  // no copy into the slots is left behind
+            (void)hipStreamSynchronize(stream_);  // no copy into the slots is left behind
             return -1;
         }
         return 0;
@@ -230,16 +259,18 @@ private:
 
     // Without pinned memory: the runtime's own staging.
     template <class Ready>
-    int direct(hipStream_t stream, const std::vector<ReadPart>& parts, hipError_t* err, Ready&& ready) {
+    int direct(const std::vector<ReadPart>& parts, hipError_t* err, Ready&& ready) {
         int rc = ready();
         for (const ReadPart& p : parts) {
             if (rc || !p.bytes) continue;
-            *err = hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, stream);
+            *err = hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, stream_);
             if (*err != hipSuccess) return -1;
         }
         return rc ? rc : ready();
     }
 
+    int device_ = 0;
+    hipStream_t stream_ = nullptr;
     char* slots_ = nullptr;
     uint32_t n_slots_ = 0;
     std::vector<hipEvent_t> events_;

@@ -1,0 +1,46 @@
+"""Readbacks on the host side (csrc/msim_read.hpp over a stand-in for the HIP
+runtime): what cannot be brought about on one GPU, or only by breaking it."""
+import os
+
+import pytest
+
+import cxx
+
+FAKE = os.path.join(cxx.ROOT, "tests", "fake_hip")
+PRELUDE = r"""
+#include <cassert>
+#include "msim_read.hpp"
+using namespace msim;
+constexpr size_t MB = size_t{1} << 20;
+static std::vector<char> pattern(size_t bytes) {
+    std::vector<char> v(bytes);
+    for (size_t k = 0; k < bytes; k++) v[k] = static_cast<char>(k * 31 + k / 4093);
+    return v;
+}
+#define CHECK(c) do { if (!(c)) { std::printf("line %d: %s\n", __LINE__, #c); std::exit(1); } } while (0)
+"""
+
+
+def check(tmp_path, body):
+    assert cxx.run(tmp_path, PRELUDE + body, includes=[FAKE]) == "ok\n"
+
+
+@pytest.mark.parametrize("megabytes", [1, 5, 40])
+def test_another_device_is_current(tmp_path, megabytes):
+    """The handle's device need not be the calling thread's, and the calling
+    thread's stays what it was."""
+    check(tmp_path, r"""
+int main() {
+    FakeStream stream;
+    stream.device = 1;
+    ReadBack rb;
+    rb.on(1, &stream);
+    const std::vector<char> src = pattern(%d * MB);
+    std::vector<char> dst(src.size());
+    hipError_t e = hipSuccess;
+    CHECK(rb.read({{dst.data(), src.data(), src.size()}}, 1000, &e, [] { return 0; }) == 0);
+    CHECK(e == hipSuccess && dst == src);
+    CHECK(fake_device == 0);
+    std::printf("ok\n");
+}
+""" % megabytes)
