@@ -118,7 +118,9 @@ public:
     // (null past one slot): no transfer follows the kernel.
     void* small(size_t bytes) {
         const DeviceScope scope(device_);
-        return bytes <= kSlot && reserve(1) ? slots_ : nullptr;
+        if (bytes > kSlot || !idle() || !reserve(1)) return nullptr;
+        writing_ = true;
+        return slots_;
     }
     static constexpr uint32_t kThreads = 6;
 
@@ -135,10 +137,23 @@ public:
     // Reads the parts in stream order.  ready() waits for the stream (and
     // whatever else must hold before the caller's memory is written) and
     // returns 0, or a code that is passed on.  Otherwise returns 0, or -1 with
-    // *err set (hipErrorNotReady: the watchdog expired).
+    // *err set (hipErrorNotReady: the watchdog expired).  After a failure the
+    // slots are left alone until the stream has drained (idle).
     template <class Ready>
     int read(const std::vector<ReadPart>& parts, uint32_t watchdog_ms, hipError_t* err, Ready&& ready) {
         const DeviceScope scope(device_);
+        const int rc = read_parts(parts, watchdog_ms, err, ready);
+        if (rc == 0) {
+            writing_ = false;
+        } else if (rc == -1 && *err != hipErrorNotReady) {
+            (void)bounded_wait(watchdog_ms, [&] { return hipStreamQuery(stream_); });
+        }
+        return rc;
+    }
+
+private:
+    template <class Ready>
+    int read_parts(const std::vector<ReadPart>& parts, uint32_t watchdog_ms, hipError_t* err, Ready&& ready) {
         size_t total = 0;
         bool there = !parts.empty();
         for (const ReadPart& p : parts) {
@@ -154,7 +169,8 @@ public:
             return rc;
         }
         if (total <= kSlot) {  // everything through one slot, one wait
-            if (!reserve(1)) return direct(parts, err, ready);
+            if (!idle() || !reserve(1)) return direct(parts, err, ready);
+            writing_ = true;
             size_t at = 0;
             for (const ReadPart& p : parts) {
                 if (!p.bytes) continue;
@@ -174,9 +190,10 @@ public:
         }
         // one thread per slot's worth, two slots each
         const uint32_t n = static_cast<uint32_t>(std::min<size_t>(kThreads, std::max<size_t>(1, total / kSlot)));
-        if (!reserve(2 * n)) return direct(parts, err, ready);
+        if (!idle() || !reserve(2 * n)) return direct(parts, err, ready);
         const int rc = ready();
         if (rc) return rc;
+        writing_ = true;
         std::vector<Piece> pieces;
         for (const ReadPart& p : parts) {
             for (size_t o = 0; o < p.bytes; o += kSlot) {
@@ -219,14 +236,9 @@ public:
         work(0);
         for (std::thread& h : helpers) h.join();
         *err = static_cast<hipError_t>(fault.load());
-        if (*err != hipSuccess) {
-            (void)hipStreamSynchronize(stream_);  // no copy into the slots is left behind
-            return -1;
-        }
-        return 0;
+        return *err == hipSuccess ? 0 : -1;
     }
 
-private:
     struct Piece {
         char* dst = nullptr;
         const char* src = nullptr;
@@ -234,6 +246,12 @@ private:
     };
 
     char* slot(uint32_t k) const { return slots_ + k * kSlot; }
+
+    // False while a call that failed may have left work that writes the slots.
+    bool idle() {
+        if (writing_ && hipStreamQuery(stream_) != hipErrorNotReady) writing_ = false;
+        return !writing_;
+    }
 
     bool reserve(uint32_t n) {
         if (n > n_slots_) {
@@ -271,6 +289,7 @@ private:
 
     int device_ = 0;
     hipStream_t stream_ = nullptr;
+    bool writing_ = false;
     char* slots_ = nullptr;
     uint32_t n_slots_ = 0;
     std::vector<hipEvent_t> events_;

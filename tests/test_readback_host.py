@@ -44,3 +44,39 @@ int main() {
     std::printf("ok\n");
 }
 """ % megabytes)
+
+
+@pytest.mark.parametrize("megabytes", [1, 40])
+def test_transfer_that_does_not_finish(tmp_path, megabytes):
+    """A transfer past the watchdog is reported after the watchdog; the slots it
+    may still write are neither used nor freed until the stream has drained."""
+    check(tmp_path, r"""
+int main() {
+    FakeStream stream;
+    ReadBack rb;
+    rb.on(0, &stream);
+    const std::vector<char> src = pattern(%d * MB);
+    std::vector<char> dst(src.size());
+    hipError_t e = hipSuccess;
+    auto read = [&] {
+        return rb.read({{dst.data(), src.data(), src.size()}}, 60, &e, [&] {
+            return src.size() <= 2 * MB && stream.stuck ? 5 : 0;  // small ones: what waits is ready()
+        });
+    };
+    CHECK(read() == 0 && dst == src);
+    stream.stuck = true;
+    const auto t0 = std::chrono::steady_clock::now();
+    const int rc = read();
+    CHECK(rc == 5 || (rc == -1 && e == hipErrorNotReady));
+    CHECK(std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(1000));
+    CHECK(fake().unbounded_waits == 0);
+    const int frees = fake().frees;
+    CHECK(rb.small(100) == nullptr);
+    CHECK(fake().frees == frees);
+    stream.stuck = false;
+    dst.assign(dst.size(), 0);
+    CHECK(rb.small(100) != nullptr);
+    CHECK(read() == 0 && dst == src);
+    std::printf("ok\n");
+}
+""" % megabytes)
