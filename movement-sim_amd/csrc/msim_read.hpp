@@ -142,7 +142,12 @@ public:
     template <class Ready>
     int read(const std::vector<ReadPart>& parts, uint32_t watchdog_ms, hipError_t* err, Ready&& ready) {
         const DeviceScope scope(device_);
-        const int rc = read_parts(parts, watchdog_ms, err, ready);
+        size_t total = 0;
+        for (const ReadPart& p : parts) total += p.bytes;
+        std::vector<ReadPart> known, rest;
+        for (const ReadPart& p : parts) (by_runtime(p, total) ? known : rest).push_back(p);
+        int rc = rest.empty() && !known.empty() ? ready() : read_parts(rest, watchdog_ms, err, ready);
+        if (rc == 0 && !known.empty()) rc = read_known(known, watchdog_ms, err);
         if (rc == 0) {
             writing_ = false;
         } else if (rc == -1 && *err != hipErrorNotReady) {
@@ -152,6 +157,37 @@ public:
     }
 
 private:
+    // Where the runtime copies by itself: device memory (of any size), and
+    // memory that the caller has pinned when the results do not fit one slot:
+    // 64 MB of entities at 54 GB/s, 37 through the slots; 640 KB take 43 us
+    // against 39.
+    bool by_runtime(const ReadPart& p, size_t total) const {
+        if (!p.bytes) return false;
+        const hipMemoryType first = memory_type(p.dst);
+        if (first == hipMemoryTypeUnregistered) return false;
+        return first == memory_type(static_cast<const char*>(p.dst) + p.bytes - 1) &&
+               (first == hipMemoryTypeDevice || total > kSlot);
+    }
+
+    static hipMemoryType memory_type(const void* p) {
+        hipPointerAttribute_t a{};
+        if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+            (void)hipGetLastError();
+            return hipMemoryTypeUnregistered;
+        }
+        return a.type;
+    }
+
+    int read_known(const std::vector<ReadPart>& parts, uint32_t watchdog_ms, hipError_t* err) {
+        writing_ = true;  // src may lie in a slot
+        for (const ReadPart& p : parts) {
+            *err = hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDefault, stream_);
+            if (*err != hipSuccess) return -1;
+        }
+        *err = bounded_wait(watchdog_ms, [&] { return hipStreamQuery(stream_); });
+        return *err == hipSuccess ? 0 : -1;
+    }
+
     template <class Ready>
     int read_parts(const std::vector<ReadPart>& parts, uint32_t watchdog_ms, hipError_t* err, Ready&& ready) {
         size_t total = 0;

@@ -1,7 +1,7 @@
 // The part of the HIP runtime that the readback header calls, on the host:
 // several devices, streams that may never drain, pinned memory counted.
-// Copies are done when they are enqueued; on a stuck stream they are only
-// noted.  Test infrastructure.
+// Copies are done when they are enqueued; on a stuck stream, or to a device,
+// they are only noted.  Test infrastructure.
 #pragma once
 
 #include <atomic>
@@ -25,7 +25,7 @@ struct FakeDim {
 static FakeDim threadIdx;
 
 enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2, hipErrorInvalidHandle = 400, hipErrorNotReady = 600 };
-enum hipMemcpyKind { hipMemcpyDeviceToHost = 2 };
+enum hipMemcpyKind { hipMemcpyDeviceToHost = 2, hipMemcpyDefault = 4 };
 enum hipMemoryType { hipMemoryTypeUnregistered = 0, hipMemoryTypeHost = 1, hipMemoryTypeDevice = 2, hipMemoryTypeManaged = 3 };
 constexpr unsigned int hipEventDisableTiming = 2, hipHostMallocDefault = 0;
 
@@ -51,7 +51,8 @@ struct FakeRuntime {
     std::map<char*, size_t> pinned;  // by hipHostMalloc, and what a test adds as its own
     std::map<char*, size_t> on_device;
     size_t pinned_bytes = 0;
-    std::atomic<int> pins{0}, frees{0}, copies{0}, copies_to_pinned{0}, unbounded_waits{0};
+    std::atomic<int> pins{0}, frees{0}, copies{0}, unbounded_waits{0};
+    std::map<void*, size_t> copied_to;  // destinations of copies
     std::atomic<bool> no_pinning{false};
     std::atomic<int> null_stream_device{-1};  // device of the last wait on the null stream
 };
@@ -127,10 +128,10 @@ inline hipError_t hipStreamSynchronize(hipStream_t s) {
 }
 inline hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKind, hipStream_t s) {
     fake().copies++;
-    {
-        std::lock_guard<std::mutex> lk(fake().m);
-        if (fake_find(fake().pinned, dst)) fake().copies_to_pinned++;
-    }
-    if (!s->stuck) std::memcpy(dst, src, bytes);
+    std::unique_lock<std::mutex> lk(fake().m);
+    fake().copied_to[dst] = bytes;
+    const bool device = fake_find(fake().on_device, dst);
+    lk.unlock();
+    if (!s->stuck && !device) std::memcpy(dst, src, bytes);
     return hipSuccess;
 }

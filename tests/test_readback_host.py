@@ -80,3 +80,40 @@ int main() {
     std::printf("ok\n");
 }
 """ % megabytes)
+
+
+@pytest.mark.parametrize("kilobytes", [3, 1000, 5000, 40000])
+def test_destinations_the_runtime_knows(tmp_path, kilobytes):
+    """Device memory is never written by the host; pinned memory takes one copy
+    where the results do not fit a slot; both beside ordinary memory."""
+    check(tmp_path, r"""
+#include <sys/mman.h>
+int main() {
+    FakeStream stream;
+    ReadBack rb;
+    rb.on(0, &stream);
+    const size_t bytes = size_t{1000} * %d;
+    const std::vector<char> src = pattern(3 * bytes);
+    std::vector<char> pageable(bytes), own(bytes);
+    char* device = static_cast<char*>(mmap(nullptr, bytes, PROT_NONE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0));
+    fake().on_device[device] = bytes;
+    fake().pinned[own.data()] = own.size();
+    hipError_t e = hipSuccess;
+    auto is = [&](const std::vector<char>& v, size_t from) { return std::memcmp(v.data(), src.data() + from, bytes) == 0; };
+    CHECK(rb.read({{device, src.data(), bytes}, {pageable.data(), src.data() + bytes, bytes},
+                   {own.data(), src.data() + 2 * bytes, bytes}}, 1000, &e, [] { return 0; }) == 0);
+    CHECK(fake().copied_to[device] == bytes);
+    CHECK(is(pageable, bytes) && is(own, 2 * bytes));
+    const bool direct = 3 * bytes > 2 * MB;
+    CHECK(fake().copied_to.count(own.data()) == (direct ? 1u : 0u));
+    if (direct) CHECK(fake().copied_to[own.data()] == bytes);
+    // what a kernel has written to a slot
+    if (void* slot = rb.small(1000)) {
+        std::memcpy(slot, src.data(), 1000);
+        fake().copied_to.clear();
+        CHECK(rb.read({{device, slot, 1000}}, 1000, &e, [] { return 0; }) == 0);
+        CHECK(fake().copied_to[device] == 1000);
+    }
+    std::printf("ok\n");
+}
+""" % kilobytes)
