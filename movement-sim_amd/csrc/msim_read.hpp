@@ -1,12 +1,12 @@
-// msim_read.hpp — device-to-host readback through a handle's own pinned
-// buffers, and the bounded wait the entry points share.
+// msim_read.hpp — device-to-host readback through pinned slots that the
+// handles of a device share, and the bounded wait the entry points share.
 //
 // A copy into the caller's (pageable) memory goes through the runtime's
 // staging buffer, copied out by one thread which also takes
 // the page faults of a fresh array: 64 MB of entities took 6.1 ms, 10 GB/s,
-// where the link moves 56 GB/s.  Here several threads each bring pieces into
-// pinned slots of their own and copy them out, so link, copies and page faults
-// overlap.
+// where the link moves 56 GB/s (17 into pages that are there).  Here several
+// threads each bring pieces into pinned slots of their own and copy them out,
+// so link, copies and page faults overlap.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -17,6 +17,8 @@
 #include <cstddef>
 #include <cstdint>
 #include <cstring>
+#include <memory>
+#include <mutex>
 #include <thread>
 #include <vector>
 
@@ -101,44 +103,139 @@ private:
     int before_ = 0, device_ = 0;
 };
 
+// The pinned slots of one device, lent to one readback at a time each and
+// shared by the device's handles: 24 MB at most however many handles there
+// are, given back to the system with the last of them.  Pinning costs about
+// 70 us a MB, more than a readback of less than 30 MB gains by it, so the first
+// one of those takes the runtime's path and only the second pins.  (Pinned by
+// every handle in its first readback, a handle of 200k agents read once beside
+// another took 2.3 ms where the runtime's path takes 1.0.)
+class SlotPool {
+public:
+    // 64 MB of entities, two slots a thread, ms: slots of 0.5 MB 3.2 (every
+    // transfer has a fixed cost), 1 MB 2.3, 2 MB 1.9, 4 MB 2.0; 4 threads 1.97,
+    // 6 1.91, 8 1.94.
+    static constexpr size_t kBytes = size_t{2} << 20;
+    static constexpr uint32_t kMost = 12;
+    static constexpr size_t kPinAtOnce = size_t{32} << 20;
+    struct Slot {
+        char* mem = nullptr;
+        hipEvent_t done = nullptr;
+    };
+    struct Lease {
+        Slot slot[kMost];
+        uint32_t n = 0;
+    };
+
+    // The device's pool, for as long as someone holds it; null without memory
+    // for it.
+    static std::shared_ptr<SlotPool> of(int device) noexcept {
+        static std::mutex m;
+        static std::vector<std::weak_ptr<SlotPool>> pools;  // by device
+        try {
+            std::lock_guard<std::mutex> lk(m);
+            const size_t d = static_cast<size_t>(std::max(device, 0));
+            if (pools.size() <= d) pools.resize(d + 1);
+            std::shared_ptr<SlotPool> p = pools[d].lock();
+            if (!p) pools[d] = p = std::make_shared<SlotPool>(device);
+            return p;
+        } catch (...) {
+            return nullptr;
+        }
+    }
+
+    explicit SlotPool(int device) : device_(device) {}
+    SlotPool(const SlotPool&) = delete;
+    SlotPool& operator=(const SlotPool&) = delete;
+    ~SlotPool() {  // nothing is lent: borrowers hold the pool
+        const DeviceScope scope(device_);
+        for (uint32_t k = 0; k < idle_.n; k++) (void)hipEventDestroy(idle_.slot[k].done);
+        for (uint32_t k = 0; k < blocks_; k++) (void)hipHostFree(block_[k]);
+    }
+
+    // `least` to `want` slots for a readback of `bytes`, or none.
+    void lend(Lease& to, uint32_t least, uint32_t want, size_t bytes) {
+        std::lock_guard<std::mutex> lk(m_);
+        const bool pin = used_ || bytes >= kPinAtOnce;
+        used_ = true;
+        const DeviceScope scope(device_);
+        if (pin && idle_.n < want) grow(std::min(want - idle_.n, kMost - made_));
+        to.n = 0;
+        if (idle_.n < least) return;
+        while (to.n < want && idle_.n > 0) to.slot[to.n++] = idle_.slot[--idle_.n];
+    }
+
+    void give_back(Lease& from) {
+        std::lock_guard<std::mutex> lk(m_);
+        while (from.n > 0) idle_.slot[idle_.n++] = from.slot[--from.n];
+    }
+
+private:
+    // n more slots, in one allocation (12 of 2 MB each take 4 ms to free, one of
+    // 24 MB 0.8); as many as there is memory and events for.
+    void grow(uint32_t n) {
+        void* p = nullptr;
+        if (n == 0) return;
+        if (hipHostMalloc(&p, n * kBytes, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            return;
+        }
+        block_[blocks_++] = p;
+        made_ += n;
+        for (uint32_t k = 0; k < n; k++) {
+            Slot s{static_cast<char*>(p) + k * kBytes, nullptr};
+            if (hipEventCreateWithFlags(&s.done, hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                return;
+            }
+            idle_.slot[idle_.n++] = s;
+        }
+    }
+
+    const int device_;
+    std::mutex m_;
+    Lease idle_;
+    void* block_[kMost] = {};
+    uint32_t blocks_ = 0, made_ = 0;  // made_: slots in the blocks
+    bool used_ = false;
+};
+
 class ReadBack {
 public:
     // The handle's device and stream.
     void on(int device, hipStream_t stream) {
         device_ = device;
         stream_ = stream;
+        pool_ = SlotPool::of(device);
     }
 
-    // 64 MB of entities, two slots a thread, ms: slots of 0.5 MB 3.2 (every
-    // transfer has a fixed cost), 1 MB 2.3, 2 MB 1.9, 4 MB 2.0; 4 threads 1.97,
-    // 6 1.91, 8 1.94.
-    static constexpr size_t kSlot = size_t{2} << 20;
+    static constexpr size_t kSlot = SlotPool::kBytes;
 
-    // Pinned memory that kernels may write `bytes` of results to directly
-    // (null past one slot): no transfer follows the kernel.
+    // Pinned memory that kernels may write `bytes` of results to directly, for
+    // the next read(); null past one slot, or when there is none to be had.  No
+    // transfer follows the kernel.
     void* small(size_t bytes) {
-        const DeviceScope scope(device_);
-        if (bytes > kSlot || !idle() || !reserve(1)) return nullptr;
+        if (bytes > kSlot) return nullptr;
+        refused_ = !borrow(1, 1, bytes);
+        if (refused_) return nullptr;
         writing_ = true;
-        return slots_;
+        return lease_.slot[0].mem;
     }
-    static constexpr uint32_t kThreads = 6;
+    static constexpr uint32_t kThreads = SlotPool::kMost / 2;
 
     ReadBack() = default;
     ReadBack(const ReadBack&) = delete;
     ReadBack& operator=(const ReadBack&) = delete;
+    // The handle's stream has drained by now.
     ~ReadBack() {
-        for (hipEvent_t e : events_) {
-            (void)hipEventDestroy(e);
-        }
-        if (slots_) (void)hipHostFree(slots_);
+        if (pool_) pool_->give_back(lease_);
     }
 
     // Reads the parts in stream order.  ready() waits for the stream (and
     // whatever else must hold before the caller's memory is written) and
     // returns 0, or a code that is passed on.  Otherwise returns 0, or -1 with
     // *err set (hipErrorNotReady: the watchdog expired).  After a failure the
-    // slots are left alone until the stream has drained (idle).
+    // slots stay with this handle, unused, until its stream has drained (idle).
     template <class Ready>
     int read(const std::vector<ReadPart>& parts, uint32_t watchdog_ms, hipError_t* err, Ready&& ready) {
         const DeviceScope scope(device_);
@@ -153,6 +250,7 @@ public:
         } else if (rc == -1 && *err != hipErrorNotReady) {
             (void)bounded_wait(watchdog_ms, [&] { return hipStreamQuery(stream_); });
         }
+        if (idle() && pool_) pool_->give_back(lease_);
         return rc;
     }
 
@@ -194,7 +292,7 @@ private:
         bool there = !parts.empty();
         for (const ReadPart& p : parts) {
             total += (p.bytes + 255) / 256 * 256;
-            there = there && slots_ && p.src >= slots_ && p.src < slots_ + kSlot;
+            there = there && lease_.n && p.src >= lease_.slot[0].mem && p.src < lease_.slot[0].mem + kSlot;
         }
         *err = hipSuccess;
         if (there) {  // written to small() by a kernel
@@ -205,12 +303,16 @@ private:
             return rc;
         }
         if (total <= kSlot) {  // everything through one slot, one wait
-            if (!idle() || !reserve(1)) return direct(parts, err, ready);
+            if (refused_ || !borrow(1, 1, total)) {
+                refused_ = false;
+                return direct(parts, err, ready);
+            }
             writing_ = true;
+            char* const slot = lease_.slot[0].mem;
             size_t at = 0;
             for (const ReadPart& p : parts) {
                 if (!p.bytes) continue;
-                *err = hipMemcpyAsync(slots_ + at, p.src, p.bytes, hipMemcpyDeviceToHost, stream_);
+                *err = hipMemcpyAsync(slot + at, p.src, p.bytes, hipMemcpyDeviceToHost, stream_);
                 if (*err != hipSuccess) return -1;
                 at += (p.bytes + 255) / 256 * 256;
             }
@@ -219,14 +321,15 @@ private:
             at = 0;
             for (const ReadPart& p : parts) {
                 if (!p.bytes) continue;
-                std::memcpy(p.dst, slots_ + at, p.bytes);
+                std::memcpy(p.dst, slot + at, p.bytes);
                 at += (p.bytes + 255) / 256 * 256;
             }
             return 0;
         }
         // one thread per slot's worth, two slots each
-        const uint32_t n = static_cast<uint32_t>(std::min<size_t>(kThreads, std::max<size_t>(1, total / kSlot)));
-        if (!idle() || !reserve(2 * n)) return direct(parts, err, ready);
+        const uint32_t most = static_cast<uint32_t>(std::min<size_t>(kThreads, std::max<size_t>(1, total / kSlot)));
+        if (!borrow(2, 2 * most, total)) return direct(parts, err, ready);
+        const uint32_t n = lease_.n / 2;
         const int rc = ready();
         if (rc) return rc;
         writing_ = true;
@@ -250,14 +353,16 @@ private:
                 hipError_t e = hipSuccess;
                 if (k < pieces.size() && fault.load() == hipSuccess) {
                     mine = pieces[k];
-                    e = hipMemcpyAsync(slot(2 * t + in), mine.src, mine.bytes, hipMemcpyDeviceToHost, stream_);
-                    if (e == hipSuccess) e = hipEventRecord(events_[2 * t + in], stream_);
+                    const SlotPool::Slot& s = lease_.slot[2 * t + in];
+                    e = hipMemcpyAsync(s.mem, mine.src, mine.bytes, hipMemcpyDeviceToHost, stream_);
+                    if (e == hipSuccess) e = hipEventRecord(s.done, stream_);
                 }
                 in ^= 1;
                 const Piece& old = held[in];  // copied out while the new one is on its way
                 if (e == hipSuccess && old.bytes) {
-                    e = bounded_wait(watchdog_ms, [&] { return hipEventQuery(events_[2 * t + in]); });
-                    if (e == hipSuccess) std::memcpy(old.dst, slot(2 * t + in), old.bytes);
+                    const SlotPool::Slot& s = lease_.slot[2 * t + in];
+                    e = bounded_wait(watchdog_ms, [&] { return hipEventQuery(s.done); });
+                    if (e == hipSuccess) std::memcpy(old.dst, s.mem, old.bytes);
                 }
                 if (e != hipSuccess) fault.store(static_cast<int>(e));
                 if (!mine.bytes) return;
@@ -281,34 +386,18 @@ private:
         size_t bytes = 0;
     };
 
-    char* slot(uint32_t k) const { return slots_ + k * kSlot; }
-
     // False while a call that failed may have left work that writes the slots.
     bool idle() {
         if (writing_ && hipStreamQuery(stream_) != hipErrorNotReady) writing_ = false;
         return !writing_;
     }
 
-    bool reserve(uint32_t n) {
-        if (n > n_slots_) {
-            void* p = nullptr;
-            if (hipHostMalloc(&p, n * kSlot, hipHostMallocDefault) != hipSuccess) {
-                (void)hipGetLastError();
-                return false;
-            }
-            if (slots_) (void)hipHostFree(slots_);
-            slots_ = static_cast<char*>(p);
-            n_slots_ = n;
-        }
-        while (events_.size() < n) {
-            hipEvent_t e = nullptr;
-            if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-                (void)hipGetLastError();
-                return false;
-            }
-            events_.push_back(e);
-        }
-        return true;
+    // `least` to `want` slots in lease_.
+    bool borrow(uint32_t least, uint32_t want, size_t bytes) {
+        if (!pool_ || !idle()) return false;
+        pool_->give_back(lease_);  // of a call that ended before its read()
+        pool_->lend(lease_, least, want, bytes);
+        return lease_.n != 0;
     }
 
     // Without pinned memory: the runtime's own staging.
@@ -326,9 +415,9 @@ private:
     int device_ = 0;
     hipStream_t stream_ = nullptr;
     bool writing_ = false;
-    char* slots_ = nullptr;
-    uint32_t n_slots_ = 0;
-    std::vector<hipEvent_t> events_;
+    bool refused_ = false;  // small() had no slot for the readback under way
+    std::shared_ptr<SlotPool> pool_;
+    SlotPool::Lease lease_;
 };
 
 }  // namespace msim
