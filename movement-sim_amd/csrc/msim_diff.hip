@@ -962,6 +962,7 @@ extern "C" int msim_batch_diff_setup(msim_batch* b, uint32_t n_ticks, uint32_t c
     if (rc != MSIM_OK) return rc;
     DiffState* d = new DiffState();
     b->diff = d;
+    const DeviceScope scope(b->device);  // copies below run on its null stream
     d->T = n_ticks;
     d->C = std::min(checkpoint_every, n_ticks);
     d->n_ck = (n_ticks + d->C - 1) / d->C;
@@ -1006,7 +1007,7 @@ extern "C" int msim_batch_diff_setup(msim_batch* b, uint32_t n_ticks, uint32_t c
             e = hipMemcpy(scen_h.data(), b->scen, sizeof(ScenDev) * b->n_scen, hipMemcpyDeviceToHost);
         }
         if (e == hipSuccess) e = hipMemcpy(d->scen, b->scen, sizeof(ScenDev) * b->n_scen, hipMemcpyDeviceToDevice);
-        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // the handle's stream does not wait for it
+        if (e == hipSuccess) e = wait_null_stream(b->device);
         if (e != hipSuccess) rc = bfail(b, MSIM_ERR_HIP, "scenario table copy: %s", hipGetErrorString(e));
     }
     if (rc == MSIM_OK && b->start_len) {
@@ -1093,8 +1094,8 @@ int set_params(msim_batch* b, DiffState& d, const float* theta, float alpha, flo
         hipError_t e = hipMemcpy(dst, th.data(), sizeof(float) * n, hipMemcpyHostToDevice);
         if (e != hipSuccess) return bfail(b, MSIM_ERR_HIP, "theta upload: %s", hipGetErrorString(e));
     }
-    // theta may come from work on the null stream, which the handle's does not wait for
-    if (hipStreamSynchronize(nullptr) != hipSuccess) return bfail(b, MSIM_ERR_HIP, "parameter upload failed");
+    // theta may come from work on the null stream of its device
+    if (wait_null_stream(b->device) != hipSuccess) return bfail(b, MSIM_ERR_HIP, "parameter upload failed");
     const float* src = direct ? theta : dst;
     const unsigned int report = ++d.checks;
     ParamWords* const words = d.words + report % 2u;

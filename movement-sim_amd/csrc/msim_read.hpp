@@ -103,6 +103,13 @@ private:
     int before_ = 0, device_ = 0;
 };
 
+// Waits for the work on a device's null stream, which a handle's non-blocking
+// stream does not wait for.
+inline hipError_t wait_null_stream(int device) {
+    const DeviceScope scope(device);
+    return hipStreamSynchronize(nullptr);
+}
+
 // The pinned slots of one device, lent to one readback at a time each and
 // shared by the device's handles: 24 MB at most however many handles there
 // are, given back to the system with the last of them.  Pinning costs about

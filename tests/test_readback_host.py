@@ -256,3 +256,18 @@ int main() {
     std::printf("ok\n");
 }
 """)
+
+
+def test_null_stream_of_the_handles_device(tmp_path):
+    """A handle's parameters may come from the null stream of its device, which
+    need not be the current one."""
+    check(tmp_path, r"""
+int main() {
+    for (int current = 0; current < 2; current++) {
+        hipSetDevice(current);
+        CHECK(wait_null_stream(1) == hipSuccess);
+        CHECK(fake().null_stream_device == 1 && fake_device == current);
+    }
+    std::printf("ok\n");
+}
+""")
