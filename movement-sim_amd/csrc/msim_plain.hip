@@ -1137,7 +1137,11 @@ extern "C" int msim_create(const msim_road* roads, uint32_t n_roads, const uint3
         s->lists = s->margin <= (1u << s->seg_log) && 8u * s->margin >= (1u << s->seg_log);
         for (int k = 0; k < 2 && s->lists; k++) {
             ALLOC(s->leave[k].rec, s->n_seg);
-            ALLOC(s->leave[k].leave, n);
+            // an entry per agent, in the binned positions, which the sorted
+            // state does not use (arrays of their own made creating and
+            // destroying a handle of 100k agents 1.3 -> 1.7 ms)
+            static_assert(sizeof(uint2) == sizeof(float2), "an entry in a position's place");
+            s->leave[k].leave = reinterpret_cast<uint2*>(s->bbpos[k]);
         }
         ALLOC(s->seg_arr, s->n_seg);
     }
