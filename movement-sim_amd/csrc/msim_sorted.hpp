@@ -601,6 +601,11 @@ inline bool one_move_per_cu(uint32_t n_seg, uint32_t smallest_seg_log) {
     return n_seg <= kCus && (1u << smallest_seg_log) >= kSortedWide;  // a thread scans at least one bucket
 }
 
+// Waves a SIMD has to have room for: two workgroups a CU with eight slots per
+// thread (the lists' two more registers, 130, had left one: 1M agents on 512
+// segments 58 -> 64 us).
+constexpr uint32_t sorted_waves(uint32_t unroll) { return unroll == 8u ? 4u : 1u; }
+
 // LDS of the sorted move: the segment's counters (4 bytes per bucket) and,
 // for its first sorted_map_cap new slots, each agent's window index and its
 // bucket in the segment (2 + 2 bytes).  Segments of up to 2^12 buckets map 2
@@ -788,7 +793,7 @@ __device__ __forceinline__ void sorted_segment(const SortedMove& mv, const Table
 // previous tick's statistics are pending; dynamic LDS:
 // sorted_lds_bytes(seg_log)).
 template <uint32_t U, uint32_t T, bool UNIFORM, bool WRITE_DIR, bool LISTS>
-static __global__ __launch_bounds__(T) void k_move_sorted(SortedMove mv, BinDev b, TickFinish fin) {
+static __global__ __launch_bounds__(T, sorted_waves(U)) void k_move_sorted(SortedMove mv, BinDev b, TickFinish fin) {
     extern __shared__ uint32_t hist[];
     __shared__ uint32_t lds[T / 64];
     __shared__ uint32_t nh[2 * kNextReach + 1];
