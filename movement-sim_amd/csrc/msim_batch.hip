@@ -746,7 +746,7 @@ extern "C" int msim_batch_read_state(msim_batch* b, uint32_t scen, float* pos, f
     if (road_index) parts.push_back({road_index, o.road, sizeof(uint32_t) * na});
     if (rand_state) parts.push_back({rand_state, o.rng, sizeof(uint4) * na});
     if (neighbour_count) parts.push_back({neighbour_count, o.ncount, sizeof(uint32_t) * na});
-    return bread_parts(b, parts);
+    return bread_parts(b, parts, true);
 }
 
 extern "C" int msim_batch_read_pairs(msim_batch* b, uint64_t* totals, uint32_t* last) {

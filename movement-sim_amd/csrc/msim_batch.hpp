@@ -608,9 +608,9 @@ inline int bwait_report(msim_batch* b, unsigned int* f) {
 
 // The parts into the caller's memory, after the stream's work and the
 // device-side checks.
-inline int bread_parts(msim_batch* b, const std::vector<ReadPart>& parts) {
+inline int bread_parts(msim_batch* b, const std::vector<ReadPart>& parts, bool host = false) {
     hipError_t e = hipSuccess;
-    const int rc = b->readback.read(parts, b->watchdog_ms, &e, [&] { return msim_batch_sync(b); });
+    const int rc = b->readback.read(parts, b->watchdog_ms, &e, [&] { return msim_batch_sync(b); }, host);
     if (rc >= 0) return rc;
     if (e == hipErrorNotReady) {
         return bfail(b, MSIM_ERR_TIMEOUT, "readback did not finish within %u ms", b->watchdog_ms);

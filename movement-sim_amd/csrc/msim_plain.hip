@@ -1327,9 +1327,9 @@ namespace {
 // The parts into the caller's memory, after the stream's work and the
 // device-side checks.
 template <class Ready>
-int read_parts(msim_sim* s, const std::vector<ReadPart>& parts, Ready&& ready) {
+int read_parts(msim_sim* s, const std::vector<ReadPart>& parts, Ready&& ready, bool host = false) {
     hipError_t e = hipSuccess;
-    const int rc = s->readback.read(parts, s->watchdog_ms, &e, ready);
+    const int rc = s->readback.read(parts, s->watchdog_ms, &e, ready, host);
     if (rc >= 0) return rc;
     if (e == hipErrorNotReady) {
         return fail(s, MSIM_ERR_TIMEOUT, "readback did not finish within %u ms", s->watchdog_ms);
@@ -1337,8 +1337,8 @@ int read_parts(msim_sim* s, const std::vector<ReadPart>& parts, Ready&& ready) {
     return fail(s, MSIM_ERR_HIP, "readback failed: %s", hipGetErrorString(e));
 }
 
-int read_parts(msim_sim* s, const std::vector<ReadPart>& parts) {
-    return read_parts(s, parts, [&] { return check_faults(s); });
+int read_parts(msim_sim* s, const std::vector<ReadPart>& parts, bool host = false) {
+    return read_parts(s, parts, [&] { return check_faults(s); }, host);
 }
 
 }  // namespace
@@ -1393,7 +1393,7 @@ extern "C" int msim_read_state(msim_sim* s, float* pos, float* target, float* di
     if (road_index) parts.push_back({road_index, o.road, sizeof(uint32_t) * n});
     if (rand_state) parts.push_back({rand_state, o.rng, sizeof(uint4) * n});
     if (neighbour_count) parts.push_back({neighbour_count, o.ncount, sizeof(uint32_t) * n});
-    return read_parts(s, parts);
+    return read_parts(s, parts, true);
 }
 
 extern "C" int msim_read_debug(msim_sim* s, uint32_t out[10]) {
@@ -1427,7 +1427,7 @@ extern "C" int msim_read_pairs(msim_sim* s, uint64_t* total, uint32_t* per_tick,
                            reinterpret_cast<const uint4*>(s->hist), static_cast<uint4*>(to), words);
         from = to;
     }
-    int rc = hist.empty() ? counters() : read_parts(s, {{hist.data(), from, bytes}}, counters);
+    int rc = hist.empty() ? counters() : read_parts(s, {{hist.data(), from, bytes}}, counters, true);
     if (rc != MSIM_OK) return rc;
     const Counters c = *s->ctr_host;
     if (total) *total = c.pairs_total;

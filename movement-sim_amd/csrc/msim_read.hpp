@@ -243,13 +243,20 @@ public:
     // returns 0, or a code that is passed on.  Otherwise returns 0, or -1 with
     // *err set (hipErrorNotReady: the watchdog expired).  After a failure the
     // slots stay with this handle, unused, until its stream has drained (idle).
+    // host: the destinations are host memory, so nothing needs to be asked about
+    // them for results of up to a slot (0.4 us each; a small state has six).
     template <class Ready>
-    int read(const std::vector<ReadPart>& parts, uint32_t watchdog_ms, hipError_t* err, Ready&& ready) {
+    int read(const std::vector<ReadPart>& parts, uint32_t watchdog_ms, hipError_t* err, Ready&& ready,
+             bool host = false) {
         const DeviceScope scope(device_);
         size_t total = 0;
         for (const ReadPart& p : parts) total += p.bytes;
         std::vector<ReadPart> known, rest;
-        for (const ReadPart& p : parts) (by_runtime(p, total) ? known : rest).push_back(p);
+        if (host && total <= kSlot) {
+            rest = parts;
+        } else {
+            for (const ReadPart& p : parts) (by_runtime(p, total) ? known : rest).push_back(p);
+        }
         int rc = rest.empty() && !known.empty() ? ready() : read_parts(rest, watchdog_ms, err, ready);
         if (rc == 0 && !known.empty()) rc = read_known(known, watchdog_ms, err);
         if (rc == 0) {
