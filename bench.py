@@ -133,7 +133,8 @@ def plain_line(args, sc):
     print(f"# timed {args.steps} ticks in {el:.3f} s", file=sys.stderr, flush=True)
 
     # per-kernel durations: HIP events right before and after one launch per
-    # tick, on the handle's stream, each kernel probed in turn
+    # tick, on the handle's stream, each kernel probed in turn and launched by
+    # itself (the timed ticks join some of them: their sum is more than a tick)
     _, kms = sim.time_ticks(args.profile_ticks, kernels=True)
     per_launch_ms = {k: v / args.profile_ticks for k, v in kms.items()}
     roof = roofline(per_launch_ms, n, bool(info["uniform_speed"]), args.config)

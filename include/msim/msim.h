@@ -70,7 +70,9 @@ typedef struct msim_options {
     uint32_t bin_unroll;       /* window slots each rebinning thread loads per
                                   round: 4 or 8 (0: 8 for segments of 2^12 and
                                   2^13 buckets, else 4); binning 3: 2, 4 or 8
-                                  (0: 4)                                        */
+                                  (0: 4), but 1 slot for 1,024 threads, whatever
+                                  is given, with at most 256 segments, of at
+                                  least 2^10 buckets each                       */
 } msim_options;
 
 typedef struct msim_info {
@@ -86,7 +88,9 @@ typedef struct msim_info {
     uint32_t uniform_speed;    /* 1 when no per-agent speed array was given   */
     uint32_t n_uninitialized;  /* agents whose Entity.initialized is still 0  */
     uint64_t device_bytes;     /* device memory held by the handle            */
-    uint32_t kernels_per_tick; /* launches of one fused tick (msim_time_ticks) */
+    uint32_t kernels_per_tick; /* launches of a tick made as two single dispatches
+                                  (msim_time_ticks' per-kernel pass); inside
+                                  msim_run_ticks a tick has fewer             */
     uint32_t binning;          /* msim_options.binning in effect              */
 } msim_info;
 
@@ -133,7 +137,8 @@ int msim_sync(msim_sim* sim);
  * 64-byte layout.  color is (0,0,1,1) for an agent that was in at least one
  * pair in the last collision dispatch and (0,1,0,1) otherwise
  * (random_move.comp:545-548,876), or the uploaded colour before any
- * collision dispatch.  Synchronous. */
+ * collision dispatch.  out may be any host memory (pinned memory receives the
+ * transfer itself) or memory of a device.  Synchronous. */
 int msim_read_entities(msim_sim* sim, msim_entity* out, uint32_t first, uint32_t count);
 
 /* Replaces the debugData readback (Simulator.cpp:199,273).  out[0] counts
@@ -158,7 +163,8 @@ int msim_read_pairs(msim_sim* sim, uint64_t* total, uint32_t* per_tick, uint32_t
 /* Spatial-index export, the uniform-grid counterpart of get_quad_tree_nodes
  * (Simulator.cpp:149-153; node layout GpuQuadTree.hpp:14-41).  cell_xy gets
  * the integer cell (floor(x/cell), floor(y/cell)) of every agent as binned by
- * the last move dispatch (2 ints per agent).  Synchronous. */
+ * the last move dispatch (2 ints per agent), in host or device memory as
+ * msim_read_entities' records.  Synchronous. */
 int msim_read_cells(msim_sim* sim, int32_t* cell_xy);
 
 /* Grid occupancy for the UI overlay, the counterpart of the quadtree nodes
@@ -185,16 +191,19 @@ int msim_read_cells_noalloc(msim_sim* sim, int32_t* cell_xy);
 int msim_get_info(msim_sim* sim, msim_info* out);
 
 /* Time n_ticks fused ticks on the handle's stream with HIP events.
- * ms_total receives the elapsed time; kernel_ms (may be NULL) receives the
- * summed duration of each kernel of the tick, measured by bracketing every
- * launch with events in a second, separate pass of n_ticks ticks, in launch
- * order (see msim_kernel_name; n_kernel_ms entries at most).  Both passes
- * advance the simulation. */
+ * ms_total receives the elapsed time of msim_run_ticks(n_ticks); kernel_ms (may
+ * be NULL) receives the summed duration of each kernel of the tick, measured by
+ * bracketing every launch with events in a second, separate pass of n_ticks
+ * ticks, in launch order (see msim_kernel_name; n_kernel_ms entries at most).
+ * That pass makes a tick's two dispatches singly, a launch per kernel; a run
+ * joins some of them and leaves a tick's statistics to the next tick, so the
+ * kernels' times add up to more than a tick of the run.  Both passes advance
+ * the simulation. */
 int msim_time_ticks(msim_sim* sim, uint32_t n_ticks, float* ms_total,
                     float* kernel_ms, uint32_t n_kernel_ms);
 
-/* Name of the k-th kernel of a fused tick in msim_time_ticks' order, or NULL
- * for k >= msim_info.kernels_per_tick. */
+/* Name of the k-th kernel of msim_time_ticks' per-kernel pass, in its order, or
+ * NULL for k >= msim_info.kernels_per_tick. */
 const char* msim_kernel_name(const msim_sim* sim, uint32_t k);
 
 /* Stream the handle enqueues on (a hipStream_t), for callers that order
@@ -241,13 +250,15 @@ int msim_batch_read_state(msim_batch* b, uint32_t scen, float* pos, float* targe
                           uint32_t* road_index, uint32_t* rand_state, uint32_t* neighbour_count);
 
 /* Cumulative pair totals (n_scen entries) and the pairs of each scenario's
- * last collision dispatch (n_scen entries); either may be NULL. */
+ * last collision dispatch (n_scen entries), in host or device memory; either
+ * may be NULL. */
 int msim_batch_read_pairs(msim_batch* b, uint64_t* totals, uint32_t* last);
 
 /* Elapsed milliseconds of n_ticks batched ticks (HIP events).  kernel_ms (may
  * be NULL) receives each kernel's summed duration over a second, separate
- * pass of n_ticks ticks in which every launch is bracketed by events, in
- * msim_batch_kernel_name order.  Both passes advance the simulation. */
+ * pass of n_ticks ticks, each kernel a launch of its own bracketed by events
+ * (as in msim_time_ticks), in msim_batch_kernel_name order.  Both passes
+ * advance the simulation. */
 int msim_batch_time_ticks(msim_batch* b, uint32_t n_ticks, float* ms_total, float* kernel_ms,
                           uint32_t n_kernel_ms);
 

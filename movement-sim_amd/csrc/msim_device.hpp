@@ -198,12 +198,12 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t bid, uint32_t nblocks) {
 // map, rows the world folds onto twice).  With more workgroups than the GPU
 // holds at once (resident), the XCDs take chunks of CHUNK consecutive indices
 // in turn: contiguous slices gave whole XCDs half the work of others.  Up to
-// that many, every workgroup runs at once anyway, and slices keep what an
-// XCD wrote in one kernel in its L2 for the next.  Move of 8M agents on 2,048
+// that many, every workgroup runs at once anyway, and a slice's data may stay
+// in its XCD's L2 from one kernel to the next.  Move of 8M agents on 2,048
 // segments (1,000 to 12,600 agents each): 264 us in slices, 164 in chunks; of
-// 5.8M agents in 64 scenarios 120 -> 112; of 1M agents on 512 segments 25 in
-// slices, 27 in chunks.  Chunks of 1, 4 and 16 are within 2% of each other, 32
-// is 4% slower.
+// 5.8M agents in 64 scenarios 120 -> 112; of 1M agents on 512 segments 22.8
+// either way.  Chunks of 1, 4 and 16 are within 2% of each other, 32 is 4%
+// slower.
 template <uint32_t CHUNK>
 __device__ __forceinline__ uint32_t xcd_deal(uint32_t bid, uint32_t nblocks, uint32_t resident) {
     if (nblocks <= resident) {

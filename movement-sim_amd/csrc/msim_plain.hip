@@ -1132,7 +1132,7 @@ extern "C" int msim_create(const msim_road* roads, uint32_t n_roads, const uint3
         // Lists reach the two neighbouring segments only.  They replace the
         // margins on both sides of a window, so they pay where the margins
         // add a quarter or more to it: move of 8M agents (margin 0.38 of a
-        // segment) 164 -> 152 us, of 1M (0.38) 24.7 -> 23.7; with narrow
+        // segment) 157 -> 154 us, of 1M (0.38) 25.8 -> 22.8; with narrow
         // tables (margin 0.02) they measured 1% slower than windows.
         s->lists = s->margin <= (1u << s->seg_log) && 8u * s->margin >= (1u << s->seg_log);
         for (int k = 0; k < 2 && s->lists; k++) {

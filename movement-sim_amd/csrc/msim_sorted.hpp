@@ -596,9 +596,8 @@ __device__ __forceinline__ uint32_t seg_order(uint32_t bid, uint32_t n_seg) {
 // Move workgroups have 512 threads; where each gets a CU of its own, 1,024
 // with one slot per thread and round: the phases of a lone workgroup are a
 // chain of waits, and twice the threads take half the rounds.  Ticks, us: 100k
-// agents on 64 segments of 2^11 buckets 21.1 -> 19.4; 200k skewed agents on 64
-// of 2^12 40 -> 33; 1M on 256 of 2^12 55 -> 47; but 1M on 512 of 2^11, two
-// workgroups a CU, 39 -> 42.
+// agents on 64 segments of 2^11 buckets 22.7 -> 19.5; 1M on 256 of 2^12 43.6 ->
+// 39.2; but 1M on 512 of 2^11, two workgroups a CU, 37.8 -> 41.9.
 constexpr uint32_t kSortedThreads = 512, kSortedWide = 1024;
 inline bool one_move_per_cu(uint32_t n_seg, uint32_t smallest_seg_log) {
     return n_seg <= kCus && (1u << smallest_seg_log) >= kSortedWide;  // a thread scans at least one bucket
